@@ -312,16 +312,16 @@ def work(case):
 # --------------------------------------------------------------- tolerance
 def tolerance(case):
     """About four times the distance of the path from exact(): rel 2.1e-3 to 2.5e-3 for attention and its gradients
-    in bf16, 2.6e-4 to 3.1e-4 in fp16, 2e-7 to 4e-7 (forward) in fp32, twice that where some scores are eight times
-    as large; 5.2e-3 for the MLP block in bf16. The whole model's logits and cached rows are 1.7e-2 to 2.0e-2 away
+    in bf16, 2.6e-4 to 3.1e-4 in fp16, 2.4e-7 to 9.2e-7 in fp32, two to three times that in the gradients where some
+    scores are eight times as large; 5.2e-3 for the MLP block in bf16. The whole model's logits and cached rows are 1.7e-2 to 2.0e-2 away
     in bf16 after four layers: there 3e-2, the most that still tells a wrong answer from rounding."""
-    rel = {"fp32": 2e-6, "fp16": 1.25e-3, "bf16": 1e-2}[case["dtype"]]
+    rel = {"fp32": 4e-6, "fp16": 1.25e-3, "bf16": 1e-2}[case["dtype"]]
     if case["kind"] == "mlp":
         rel *= 2
     elif case["kind"] in ("step", "prompt"):
         rel = {"fp16": 8e-3, "bf16": 3e-2}[case["dtype"]]
-    elif case["kind"] == "train":
-        rel *= (2 if case["outliers"] else 1) * (2 if case["dtype"] == "fp32" else 1)  # a chain of four fp32 sums
+    elif case["kind"] == "train" and case["outliers"]:
+        rel *= 3 if case["dtype"] == "fp16" else 2
     return {"rel": rel}
 
 
