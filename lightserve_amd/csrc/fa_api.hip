@@ -596,8 +596,7 @@ struct GemvSplit {
 
 // The MFMA kernel (fa_gemv_mfma.hip) serves 3..32 rows when every matrix's
 // width is a multiple of 128 and the input is x or x with a SwiGLU gate (not a
-// fused norm): K-ranges of at most 256 rows (four 64-row tiles per
-// workgroup), 128-column blocks.
+// fused norm).
 bool gemv_uses_mfma(const lsfa_gemv_group_args* a) {
   if (a->m < 3 || a->m > 32 || a->norm_weight || a->k % 8 != 0 || a->x_stride % 8 != 0 || !aligned16(a->x))
     return false;
@@ -610,14 +609,23 @@ bool gemv_uses_mfma(const lsfa_gemv_group_args* a) {
   return n / 128 <= LSFA_GEMV_COUNTER_BYTES / 64;
 }
 
+// Its split: as many K-ranges of at least 256 rows as keep the grid within
+// one workgroup per CU (column blocks x splits <= 256), ranges multiples of the
+// 32-row step. Measured at 8 rows over 1..16 splits: 48 blocks 28.0 us at 1,
+// 13.5 at 5, 16.6 at 6; 32 blocks of K = 14336 88 at 1, 23.1 at 8, 30.4 at 10;
+// 224 blocks 42.3 at 1, 44.0 at 2, 47.6 at 8: a second workgroup on some CUs
+// only adds partials. The workspace has room for 512 workgroups' partials.
 GemvSplit gemv_split_mfma(long long M, long long K, long long N) {
   GemvSplit g;
   M = std::max(M, 0LL); K = std::max(K, 0LL); N = std::max(N, 0LL);
-  g.kc = (int)std::min(256LL, std::max(64LL, (K + 63) / 64 * 64));
+  const long long blocks = std::max(1LL, N / 128);
+  const long long most = std::max(1LL, (K + 255) / 256);
+  const long long want = std::max(1LL, std::min(256 / blocks, most));
+  g.kc = (int)std::max(32LL, ((K + want - 1) / want + 31) / 32 * 32);
   g.splits = (int)std::max(1LL, (K + g.kc - 1) / g.kc);
   if (g.splits > 1) {
     g.counter_bytes = LSFA_GEMV_COUNTER_BYTES;
-    g.bytes = g.counter_bytes + align256((uint64_t)g.splits * M * N * 4);
+    g.bytes = g.counter_bytes + align256((uint64_t)std::min(512 / blocks, most) * M * N * 4);
   }
   return g;
 }

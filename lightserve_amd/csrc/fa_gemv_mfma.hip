@@ -3,46 +3,67 @@
 // for the decode steps of a batch, where the VALU kernel (fa_gemv.hip) spends
 // more time on its products than on the weight bytes.
 //
-// The product is computed transposed, y^T = W^T x^T, on v_mfma_f32_32x32x16:
-// the A operand W^T [32 columns x 16 rows of K] comes from LDS through the
-// transposing read (ds_read_b64_tr_b16) of W tiles stored row-major, exactly as
-// the attention kernels read V^T; the B operand x^T [16 x 32 rows of x] (rows
-// past M are zero) stays in registers for the whole K-range.
-//   Grid (N / 128 column blocks, splits): a 4-wave workgroup owns 128 columns
-//   (one 32-column block per wave) and a K-range of at most 256 rows, i.e. four
-//   64 x 128 tiles (16 KB each) that go global -> LDS by direct loads
-//   (buffer_load ... lds) into four separate buffers, all issued up front: the
-//   workgroup keeps 64 KB in flight and no buffer is reused, so the loop needs
-//   no barrier beyond one per tile for the other waves' parts. Tiles past the
-//   K-range are issued with empty descriptors (they load zeros and cost no HBM
-//   traffic), which keeps each wave's count of outstanding loads fixed.
-//   With one split a wave rounds its 32 x M sums into y; otherwise the partial
-//   sums, two-level arrival counters and last-workgroup reduction work as in
-//   fa_gemv.hip (device-scope atomic stores and loads, no cache maintenance),
-//   with the partials stored column-major, [split][column][row], so that the
-//   32 lanes of each accumulator register (32 rows of one column) store
-//   consecutive words and the last workgroup reads them back contiguously.
+// The product is a pass over W (2 M FLOP per 2-byte weight, M <= 32), so it is
+// bound by HBM as long as W streams without gaps. W therefore goes from memory
+// straight into registers, two steps deep, with no LDS, barrier or reuse
+// between a wave's load and its use:
+//   A wave owns 128 columns and walks K in steps of 32 rows. Lane (c, kg) =
+//   (l % 16, l / 16) loads 16 bytes (columns 8c .. 8c+7) of the eight rows
+//   8 kg .. 8 kg + 7 of a step, so a load instruction covers four 256-byte row
+//   segments and a step is eight instructions, 8 KB. The lane then holds an
+//   8 x 8 block with K across its registers; 32 v_perm_b32 turn it into eight
+//   operands of eight K values, one per column, and operand j of the wave is
+//   the W^T tile {8 c + j} x {32 rows} of v_mfma_f32_16x16x32 (an operand's
+//   rows may be any 16 columns, so the stride of 8 costs nothing; the permutes
+//   take 128 issue cycles per 8 KB, and a CU's share of HBM delivers 8 KB in
+//   about 750).
+//   x^T is the B operand: lane (row l % 16, kg) loads 16 bytes of its row.
+//   The four waves of a workgroup take the steps of its K-range in turn and
+//   add their sums through LDS.
+//   Grid (N / 128 column blocks, splits). With one split a workgroup rounds its
+//   sums into y; otherwise partial sums, arrival counters and the last
+//   workgroup's reduction work as in fa_gemv.hip (device-scope atomic stores
+//   and loads, no cache maintenance).
+// Measured at 8 rows, bf16, graph replays over weights that no cache holds, in
+// us, against W through LDS in one-shot workgroups of 256 rows x 128 columns:
+//   4096 -> 4096+1024+1024 (50 MB): 21.4 -> 13.5    4096 -> 4096 (34 MB): 16.9 -> 10.9
+//   4096 -> 2 x 14336 (235 MB): 68.3 -> 42.3 (5.6 TB/s)    14336 -> 4096: 44.4 -> 23.1
+//   4096 -> 128256 (1.05 GB): 286 -> 165 (6.4 TB/s)
+// and at 32 rows 37.1 -> 16.4, 31.3 -> 13.7, 99.4 -> 46.2, 85.5 -> 27.2, 406 -> 177.
+// Three or four steps in flight, or eight waves, change nothing (+-3%): what is
+// left on the small products is the launch's own latency and the reduction.
 #include "fa_common.hpp"
 
 namespace lsfa {
 
-constexpr int kMfmaCols = 128;     // columns per workgroup (LDS tile width)
-constexpr int kMfmaTileRows = 64;  // rows per LDS tile
-constexpr int kMfmaTiles = 4;      // tiles per workgroup: K-range <= 256 rows
-constexpr int kMfmaTileElems = kMfmaTileRows * kMfmaCols;
+constexpr int kMfmaCols = 128;   // columns per workgroup
+constexpr int kMfmaWaves = 4;    // waves per workgroup
+constexpr int kMfmaStep = 32;    // rows of W per step
+constexpr int kMfmaDepth = 2;    // steps of a wave in flight
+constexpr int kMfmaLd = kMfmaCols + 4;  // row stride of the wave sums in LDS (floats)
 constexpr int kMfmaCounterSlots = 16;
 
-template <typename T>
-__global__ __launch_bounds__(256) void fa_gemv_mfma_kernel(const GemvParams p) {
+__device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4 mfma16(f16x8 a, f16x8 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+// 16-byte read-once load (non-temporal); lanes whose offset is out of range read zero.
+__device__ __forceinline__ u32x4 load16_nt(__amdgpu_buffer_rsrc_t rs, int voff, int soff) {
+  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, voff, soff, 2));
+}
+
+// MT: blocks of 16 rows (M <= 16 MT). GATE: x stands for silu(xg) * x.
+template <typename T, int MT, bool GATE>
+__global__ __launch_bounds__(64 * kMfmaWaves, 2) void fa_gemv_mfma_kernel(const GemvParams p) {
+  constexpr int NW = kMfmaWaves, DEPTH = kMfmaDepth;
   using X8 = typename VecT<T>::x8;
-  using X4 = typename VecT<T>::x4;
-  constexpr int DP = kMfmaCols;
-  extern __shared__ __attribute__((aligned(16))) char mfma_raw[];  // kMfmaTiles tiles
-  T* mfma_smem = (T*)mfma_raw;
+  extern __shared__ __attribute__((aligned(16))) float wave_sums[];  // [NW / 2][16 MT][kMfmaLd]
   __shared__ int last_arrival;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l32 = lane & 31, hh = lane >> 5;
+  const int c = lane & 15, kg = lane >> 4;
   const int split = blockIdx.y;
   const int k_begin = split * p.kc;
   const int k_len = max(0, min(p.K, k_begin + p.kc) - k_begin);
@@ -57,124 +78,159 @@ __global__ __launch_bounds__(256) void fa_gemv_mfma_kernel(const GemvParams p) {
   const int64_t sy = g == 0 ? p.sy[0] : (g == 1 ? p.sy[1] : (g == 2 ? p.sy[2] : p.sy[3]));
   const int n_local = n_blk - col_off;
 
-  // x^T as the B operand for every 16-row step of the K-range. The
-  // transposed read below gives the A operand its 16 rows in the order
-  // 4hh + (0..3), 8 + 4hh + (0..3) (slot s <-> row 8(s/4) + 4hh + s%4), so B
-  // takes the same order: lane holds x[l32][16 step + 4hh .. + 3] and
-  // x[l32][16 step + 8 + 4hh .. + 3]. Rows past M and columns past the range
-  // are zero (the loads are clamped in bounds, then masked).
-  // With a gate the operand is bf16(bf16(silu(gate)) * x), the two roundings
-  // of F.silu(gate) * up.
-  X8 xop[kMfmaTiles * 4];
-  {
-    const int m = min(l32, p.M - 1);
-    const T* xr = (const T*)p.x + (int64_t)m * p.sx + k_begin;
-    const T* gr = p.xg != nullptr ? (const T*)p.xg + (int64_t)m * p.sxg + k_begin : nullptr;
-    auto load4 = [&](int k) -> u32x2 {
-      u32x2 v = *(const u32x2*)(xr + k);
-      if (gr != nullptr) {
-        const X4 up = __builtin_bit_cast(X4, v);
-        const X4 gt = __builtin_bit_cast(X4, *(const u32x2*)(gr + k));
-        X4 o;
+  // Rows of x past M repeat the last one: their sums are never stored.
+  const T* xr[MT];
+  const T* gr[MT];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
+  for (int t = 0; t < MT; ++t) {
+    const int m = min(16 * t + c, p.M - 1);
+    xr[t] = (const T*)p.x + (int64_t)m * p.sx + k_begin;
+    gr[t] = GATE ? (const T*)p.xg + (int64_t)m * p.sxg + k_begin : nullptr;
+  }
+  const T* wk = w + (int64_t)k_begin * sw + n_local;
+  const int row_bytes = (int)(sw * 2);
+  const int lane_off = 8 * kg * row_bytes + 16 * c;
+
+  struct Step {
+    u32x4 w[8];
+    u32x4 x[MT];
+    u32x4 g[GATE ? MT : 1];
+  };
+  // The loads of one step, always the same number of them, so that the wait
+  // before a step's use counts the next step's loads as still in flight. K is
+  // a multiple of 8, so a lane's eight rows are inside the K-range or past it
+  // together; past it W reads as zero (offset out of range: no memory access)
+  // and x, read at its row's start, is masked on use.
+  auto load = [&](int step, Step& s) {
+    const int k = step * kMfmaStep;
+    const bool in = k + 8 * kg < k_len;
+    const __amdgpu_buffer_rsrc_t rs = tile_rsrc(wk + (int64_t)min(k, k_len) * sw, 0x7fffffff);
+    const int voff = in ? lane_off : (int)0x80000000;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) s.w[r] = load16_nt(rs, voff, r * row_bytes);
+    const int kx = in ? k + 8 * kg : 0;
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      s.x[t] = ldg16(xr[t] + kx);
+      if (GATE) s.g[t] = ldg16(gr[t] + kx);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  f32x4 acc[MT][8];
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto use = [&](int step, const Step& s) {
+    const bool in = step * kMfmaStep + 8 * kg < k_len;
+    X8 xb[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      u32x4 raw = s.x[t];
+      if (GATE) {
+        // silu(gate) rounded to T, times x rounded to T: the two roundings of
+        // F.silu(gate) * up.
+        const X8 up = __builtin_bit_cast(X8, raw), gt = __builtin_bit_cast(X8, s.g[t]);
+        X8 o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
           const float gv = (float)gt[e];
           const float act = (float)(T)(gv / (1.0f + expf(-gv)));
           o[e] = (T)(act * (float)up[e]);
         }
-        v = __builtin_bit_cast(u32x2, o);
+        raw = __builtin_bit_cast(u32x4, o);
       }
-      return v;
-    };
 #pragma unroll
-    for (int st = 0; st < kMfmaTiles * 4; ++st) {
-      const int k0 = 16 * st + 4 * hh, k1 = k0 + 8;
-      // An empty K-range (k = 0, or a split past the end) loads nothing: the
-      // clamped index would fall before the row (uniform branch).
-      u32x2 lo = u32x2{0u, 0u}, hi = u32x2{0u, 0u};
-      if (k_len > 0) {
-        lo = load4(min(k0, k_len - 4));
-        hi = load4(min(k1, k_len - 4));
-      }
-      if (l32 >= p.M || k0 >= k_len) lo = u32x2{0u, 0u};
-      if (l32 >= p.M || k1 >= k_len) hi = u32x2{0u, 0u};
-      const u32x4 raw = {lo[0], lo[1], hi[0], hi[1]};
-      xop[st] = __builtin_bit_cast(X8, raw);
+      for (int e = 0; e < 4; ++e) raw[e] = in ? raw[e] : 0u;
+      xb[t] = __builtin_bit_cast(X8, raw);
     }
-  }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {  // columns 2q and 2q + 1 of the lane's eight
+      u32x4 lo, hi;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        lo[e] = __builtin_amdgcn_perm(s.w[2 * e + 1][q], s.w[2 * e][q], 0x05040100u);
+        hi[e] = __builtin_amdgcn_perm(s.w[2 * e + 1][q], s.w[2 * e][q], 0x07060302u);
+      }
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        acc[t][2 * q] = mfma16(__builtin_bit_cast(X8, lo), xb[t], acc[t][2 * q]);
+        acc[t][2 * q + 1] = mfma16(__builtin_bit_cast(X8, hi), xb[t], acc[t][2 * q + 1]);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
 
-  // Direct tile loads: wave w moves rows 16w .. 16w + 15 of each tile (four
-  // 1 KB chunks); lane t of chunk c lands at tile byte (4w + c) * 1024 + 16t
-  // = (row, swizzled 16-byte segment). Descriptors are clipped to the rows of
-  // the K-range, so rows past it read as zero.
-  int vo[4];
+  if (k_len > 0) {  // uniform: an empty K-range reads neither x nor W
+    const int steps = (k_len + kMfmaStep - 1) / kMfmaStep;
+    Step s[DEPTH];
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const int byte = (wave * 4 + c) * 1024 + lane * 16;
-    const int row = byte / (DP * 2);
-    const int seg = ((byte % (DP * 2)) / 16) ^ seg_swz<DP>(row);
-    vo[c] = (int)(row * sw * 2) + seg * 16;
-  }
+    for (int d = 0; d < DEPTH; ++d) load(wave + d * NW, s[d]);
+    for (int st = wave; st < steps; st += DEPTH * NW) {
 #pragma unroll
-  for (int t = 0; t < kMfmaTiles; ++t) {
-    const int rows = min(k_len - t * kMfmaTileRows, kMfmaTileRows);
-    const T* base = w + (int64_t)(k_begin + t * kMfmaTileRows) * sw + n_local;
-    const __amdgpu_buffer_rsrc_t rs = tile_rsrc(rows > 0 ? base : w, rows > 0 ? (int)(rows * sw * 2) : 0);
-    LDS_AS char* dst = (LDS_AS char*)(mfma_smem + t * kMfmaTileElems);
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (LDS_AS void*)(dst + (wave * 4 + c) * 1024), 16, vo[c], 0, 0, 0);
-  }
-
-  // Transposed-read offsets of this wave's 32 columns (as the attention
-  // kernels' V^T reads).
-  const int tr_row = 4 * hh + ((lane & 15) >> 2);
-  const int tr_col = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-  const int voff0 = swz_off<DP>(tr_row, 32 * wave + tr_col) * 2;
-  const int voff1 = swz_off<DP>(tr_row + 8, 32 * wave + tr_col) * 2;
-
-  f32x16 acc = f32x16{};
-  const int ntiles = (k_len + kMfmaTileRows - 1) / kMfmaTileRows;
-#pragma unroll
-  for (int t = 0; t < kMfmaTiles; ++t) {
-    // Each wave issued 4 loads per tile; tile t has landed once at most
-    // 4 * (tiles after t) of them are outstanding.
-    if (t == 0) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
-    if (t == 1) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-    if (t == 2) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-    if (t == 3) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();  // the other waves' rows of tile t have landed too
-    if (t < ntiles) {
-      const LDS_AS char* tile = (const LDS_AS char*)(mfma_smem + t * kMfmaTileElems);
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        const LDS_AS char* b = tile + ks * 16 * DP * 2;
-        const X8 a = cat4<X8, X4>(lds_read_tr((const LDS_AS T*)(b + voff0)), lds_read_tr((const LDS_AS T*)(b + voff1)));
-        acc = mfma32(a, xop[4 * t + ks], acc);
+      for (int d = 0; d < DEPTH; ++d) {
+        use(st + d * NW, s[d]);
+        load(st + (DEPTH + d) * NW, s[d]);
       }
     }
   }
 
-  // acc: lane l, register i holds y^T[column 32w + 8(i/4) + 4hh + i%4][row l32].
-  const int m = l32;
-  if (p.splits == 1) {
-    if (m < p.M) {
+  // acc[t][j] register i holds row 16 t + l % 16 of column 32 kg + 8 i + j. The
+  // upper half of the waves hands its sums to the lower half, which adds them
+  // to its own, so that LDS holds NW / 2 blocks.
+  constexpr int HW = NW / 2;
+  auto slot = [&](int t) { return wave_sums + ((wave % HW) * 16 * MT + 16 * t + c) * kMfmaLd + 32 * kg; };
+  if (wave >= HW) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int n = 32 * wave + 8 * (i >> 2) + 4 * hh + (i & 3);
-        y[(int64_t)m * sy + n_local + n] = (T)acc[i];
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        *(f32x4*)(slot(t) + 8 * i) = f32x4{acc[t][0][i], acc[t][1][i], acc[t][2][i], acc[t][3][i]};
+        *(f32x4*)(slot(t) + 8 * i + 4) = f32x4{acc[t][4][i], acc[t][5][i], acc[t][6][i], acc[t][7][i]};
       }
-    }
-    return;
   }
-  if (m < p.M) {
-    float* dst = p.partial + ((int64_t)split * p.N + n_blk) * p.M + m;
+  __syncthreads();
+  if (wave < HW) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int n = 32 * wave + 8 * (i >> 2) + 4 * hh + (i & 3);
-      __hip_atomic_store(dst + (int64_t)n * p.M, acc[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        *(f32x4*)(slot(t) + 8 * i) += f32x4{acc[t][0][i], acc[t][1][i], acc[t][2][i], acc[t][3][i]};
+        *(f32x4*)(slot(t) + 8 * i + 4) += f32x4{acc[t][4][i], acc[t][5][i], acc[t][6][i], acc[t][7][i]};
+      }
+  }
+  __syncthreads();
+  // The block's sums in pairs of columns, row by row: thread tid takes pairs
+  // tid, tid + 64 NW, ...
+  constexpr int IT = 16 * MT * (kMfmaCols / 2) / (64 * NW);
+  const int pairs = p.M * (kMfmaCols / 2);
+  const int64_t sstride = (int64_t)p.N * p.M / 2;
+  uint64_t* base = (uint64_t*)(p.partial + (int64_t)n_blk * p.M);
+  auto put = [&](int pair, float s0, float s1) {
+    T* dst = y + (int64_t)(pair / (kMfmaCols / 2)) * sy + n_local + 2 * (pair % (kMfmaCols / 2));
+    dst[0] = (T)s0;
+    dst[1] = (T)s1;
+  };
+#pragma unroll
+  for (int it = 0; it < IT; ++it) {
+    const int pair = tid + it * 64 * NW;
+    if (pair < pairs) {
+      const float* src = wave_sums + (pair / (kMfmaCols / 2)) * kMfmaLd + 2 * (pair % (kMfmaCols / 2));
+      float s0 = src[0], s1 = src[1];
+#pragma unroll
+      for (int wv = 1; wv < HW; ++wv) {
+        s0 += src[wv * 16 * MT * kMfmaLd];
+        s1 += src[wv * 16 * MT * kMfmaLd + 1];
+      }
+      if (p.splits == 1)
+        put(pair, s0, s1);
+      else
+        __hip_atomic_store(base + split * sstride + pair,
+                           (uint64_t)__float_as_uint(s0) | (uint64_t)__float_as_uint(s1) << 32, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
     }
   }
+  if (p.splits == 1) return;
   // Handoff to the workgroup that arrives last, built on gfx950's device
   // coherence rather than on release/acquire fences: the partials are
   // agent-scope atomic stores (write-through to the device-coherent level,
@@ -191,45 +247,71 @@ __global__ __launch_bounds__(256) void fa_gemv_mfma_kernel(const GemvParams p) {
   __syncthreads();
   if (tid == 0) {
     int* ctr = p.counters + blockIdx.x * kMfmaCounterSlots;
-    const int group = split & 7;
-    const int group_size = (p.splits - group + 7) >> 3;
-    const int groups = min(p.splits, 8);
-    bool last = false;
-    if (__hip_atomic_fetch_add(ctr + group, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == group_size - 1) {
-      __hip_atomic_store(ctr + group, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      last = __hip_atomic_fetch_add(ctr + 8, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == groups - 1;
+    // One counter for up to eight splits (the arrivals are spread over more
+    // than the 175 ns that each takes), two levels above.
+    bool last = true;
+    if (p.splits > 8) {
+      const int group = split & 7;
+      const int group_size = (p.splits - group + 7) >> 3;
+      last = __hip_atomic_fetch_add(ctr + group, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == group_size - 1;
+      if (last) __hip_atomic_store(ctr + group, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (last) {
+      last = __hip_atomic_fetch_add(ctr + 8, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == min(p.splits, 8) - 1;
       if (last) __hip_atomic_store(ctr + 8, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     last_arrival = last;
   }
   __syncthreads();
   if (!last_arrival) return;
-  // The last workgroup: the block's 128 x M partials are contiguous per
-  // split; thread tid sums elements tid, tid + 256, ... (element e is column
-  // e / M, row e % M) over the splits in split order.
-  const int64_t sstride = (int64_t)p.N * p.M;
-  const float* base = p.partial + (int64_t)n_blk * p.M;
-  for (int e = tid; e < kMfmaCols * p.M; e += 256) {
-    float s = 0.f;
-#pragma unroll 8
-    for (int s2 = 0; s2 < p.splits; ++s2)
-      s += __hip_atomic_load(base + s2 * sstride + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const int c = e / p.M, mr = e - c * p.M;
-    y[(int64_t)mr * sy + n_local + c] = (T)s;
+  // The last workgroup adds the block's partials, contiguous per split, in
+  // split order, the loads of up to four splits in flight together.
+  float t0[IT], t1[IT];
+#pragma unroll
+  for (int it = 0; it < IT; ++it) t0[it] = t1[it] = 0.f;
+  constexpr int SB = IT <= 2 ? 8 : 4;
+  for (int s0 = 0; s0 < p.splits; s0 += SB) {
+    uint64_t v[SB][IT];
+#pragma unroll
+    for (int b = 0; b < SB; ++b)
+#pragma unroll
+      for (int it = 0; it < IT; ++it) {
+        const int pair = tid + it * 64 * NW;
+        v[b][it] = (s0 + b < p.splits && pair < pairs)
+                       ? __hip_atomic_load(base + (s0 + b) * sstride + pair, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                       : 0;
+      }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int b = 0; b < SB; ++b)
+#pragma unroll
+      for (int it = 0; it < IT; ++it) {
+        t0[it] += __uint_as_float((uint32_t)v[b][it]);
+        t1[it] += __uint_as_float((uint32_t)(v[b][it] >> 32));
+      }
   }
+#pragma unroll
+  for (int it = 0; it < IT; ++it)
+    if (tid + it * 64 * NW < pairs) put(tid + it * 64 * NW, t0[it], t1[it]);
+}
+
+template <typename T, int MT>
+static hipError_t launch_gemv_mfma(const GemvParams& p, hipStream_t s) {
+  const dim3 grid((unsigned)(p.N / kMfmaCols), (unsigned)p.splits);
+  const size_t lds = (size_t)(kMfmaWaves / 2) * 16 * MT * kMfmaLd * 4;
+  if (p.xg != nullptr)
+    hipLaunchKernelGGL((fa_gemv_mfma_kernel<T, MT, true>), grid, dim3(64 * kMfmaWaves), lds, s, p);
+  else
+    hipLaunchKernelGGL((fa_gemv_mfma_kernel<T, MT, false>), grid, dim3(64 * kMfmaWaves), lds, s, p);
+  return hipGetLastError();
 }
 
 // Host entry used by the C ABI layer: arguments validated, every matrix's
-// width a multiple of 128, kc a multiple of 64 of at most 256, 3 <= M <= 32.
+// width a multiple of 128, K and kc multiples of 8, 3 <= M <= 32.
 hipError_t gemv_mfma(const GemvParams& p, bool is_bf16, hipStream_t s) {
   if (p.M == 0 || p.N == 0) return hipSuccess;
-  const dim3 grid((unsigned)(p.N / kMfmaCols), (unsigned)p.splits);
-  const size_t lds = (size_t)kMfmaTiles * kMfmaTileElems * 2;
-  if (is_bf16)
-    hipLaunchKernelGGL(fa_gemv_mfma_kernel<__bf16>, grid, dim3(256), lds, s, p);
-  else
-    hipLaunchKernelGGL(fa_gemv_mfma_kernel<_Float16>, grid, dim3(256), lds, s, p);
-  return hipGetLastError();
+  if (p.M <= 16) return is_bf16 ? launch_gemv_mfma<__bf16, 1>(p, s) : launch_gemv_mfma<_Float16, 1>(p, s);
+  return is_bf16 ? launch_gemv_mfma<__bf16, 2>(p, s) : launch_gemv_mfma<_Float16, 2>(p, s);
 }
 
 }  // namespace lsfa

@@ -13,17 +13,16 @@ single pass over B's bytes, so bf16/fp16 products with M <= 2 go to the
 library's skinny kernel (lsfa_gemv: one launch, a K-split pass over B at HBM
 rate whose last workgroup per column block sums the fp32 partials and rounds
 once), which hipBLASLt's general tiles reach at a fraction of the bandwidth.
-From 3 to 32 rows, plain products whose widths are multiples of 128 run on
-a second kernel that computes them on MFMA (W tiles through LDS, transposed
-reads); measured on MI355X over the LLaMA-3-8B decode projections it beats
-hipBLASLt up to 8 rows on the narrow products (q/k/v, o, down) but not on the
-wide ones (gate/up, LM head), so matmul routes 3-8 rows to it only for
-products of at most 8192 columns. The fused norm and SwiGLU inputs are
-routed at up to 2 rows only: the MFMA kernel takes a gate too, but every
-workgroup then evaluates the activation over its whole K-range for all 32
-padded rows before its first product, which measured slower (batch-8 decode
-step 1.043 ms) than torch's SiLU and multiply ahead of the plain product
-(0.885 ms).
+From 3 to 32 rows, products whose widths are multiples of 128 run on a second
+kernel that computes them on MFMA while W streams through registers, with the
+SwiGLU activation formed as x is loaded. Measured on MI355X over the
+LLaMA-3-8B decode projections at 8 and 32 rows (us, graph replays, weights
+that no cache holds), this kernel against hipBLASLt: q/k/v 13.5 and 16.4
+against 51.9 and 54.1, o 10.9 and 13.7 against 21.9 and 20.9, gate/up 42.3 and
+46.2 against 56.1 and 56.8, down 23.1 and 27.2 against 71.0 and 61.4, LM head
+165 and 177 against 190 and 198; so every such product goes to it, unless
+autograd, a tracer or autocast has to see the call (_library_only). The norm
+is folded into the launch at up to 2 rows only.
 
 Projections that share their input (a decoder's q/k/v, gate/up) go through
 matmul_shared_input, which runs them as one lsfa_gemv_group launch over their
@@ -45,6 +44,7 @@ going first. (A workspace first created inside a graph capture records its
 counter fill into the graph, which then clears the 256 KB on every replay.)
 """
 import collections
+import threading
 
 import torch
 
@@ -52,12 +52,10 @@ from .. import _lib
 
 SKINNY_MAX_ROWS = 32  # what lsfa_gemv takes (more than 8 rows: MFMA kernel only)
 AUTO_MAX_ROWS = 2    # rows that every product (and the fused norm / SwiGLU inputs) routes to it
-# From 3 to 8 rows, plain products whose matrices are multiples of 128 columns
-# wide and total at most this many columns run on the library's MFMA kernel
-# (faster than hipBLASLt there: the q/k/v, o and down projections of a
-# decoder); wider ones (gate/up, the LM head) stay on hipBLASLt.
-MFMA_AUTO_ROWS = 8
-MFMA_AUTO_MAX_COLS = 8192
+# From 3 to this many rows, products of up to this many columns in all, every
+# matrix a multiple of 128 wide, run on the library's MFMA kernel.
+MFMA_AUTO_ROWS = 32
+MFMA_AUTO_MAX_COLS = 128 * (_lib.GEMV_COUNTER_BYTES // 64)
 
 MAX_CACHED_STREAMS = 8
 
@@ -73,9 +71,15 @@ class _Entry:
 
 # (device index, stream handle) -> _Entry, least recently used first
 _workspaces = collections.OrderedDict()
+_workspaces_lock = threading.Lock()
 
 
 def _workspace(device, stream, nbytes):
+    with _workspaces_lock:
+        return _workspace_locked(device, stream, nbytes)
+
+
+def _workspace_locked(device, stream, nbytes):
     key = (device.index, stream)
     entry = _workspaces.pop(key, None) or _Entry()
     if entry.buf is None or entry.buf.numel() < nbytes:
@@ -99,7 +103,8 @@ def release_workspaces():
     """Frees every cached skinny-GEMM workspace. Call it once no captured HIP
     graph that ran a skinny product is alive (those graphs keep using the
     workspaces they recorded)."""
-    _workspaces.clear()
+    with _workspaces_lock:
+        _workspaces.clear()
 
 
 def _skinny_ok(a: torch.Tensor, b: torch.Tensor, max_rows: int = SKINNY_MAX_ROWS) -> bool:
@@ -179,6 +184,26 @@ def skinny_matmul_group(a: torch.Tensor, bs, outs=None, gate: torch.Tensor = Non
     return outs
 
 
+def _library_only(*tensors) -> bool:
+    """Whether a call on these tensors has to go through torch's own operators:
+    a gradient is recorded (reverse or forward mode), a subclass, mode or
+    transform looks at the operators, or autocast may change their types."""
+    return (any(type(t) not in (torch.Tensor, torch.nn.Parameter) for t in tensors)
+            or (torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
+            or torch.autograd.forward_ad._current_level >= 0
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch._C._len_torch_dispatch_stack() > 0 or torch._C._len_torch_function_stack() > 0
+            or torch.is_autocast_enabled("cuda") or torch._C._get_tracing_state() is not None
+            or torch.compiler.is_compiling())
+
+
+def _mfma_ok(a: torch.Tensor, bs) -> bool:
+    """Whether the MFMA kernel takes these products (beyond _skinny_ok)."""
+    return (AUTO_MAX_ROWS < a.shape[0] <= MFMA_AUTO_ROWS and sum(b.shape[1] for b in bs) <= MFMA_AUTO_MAX_COLS
+            and all(_skinny_ok(a, b) and b.shape[1] % 128 == 0 for b in bs)
+            and a.shape[1] % 8 == 0 and _rows_addressable(a))
+
+
 def _auto_skinny(a: torch.Tensor, bs) -> bool:
     """Whether matmul / matmul_shared_input route these products to the
     skinny kernels (see AUTO_MAX_ROWS and MFMA_AUTO_*)."""
@@ -187,9 +212,7 @@ def _auto_skinny(a: torch.Tensor, bs) -> bool:
         return False
     if a.shape[0] <= AUTO_MAX_ROWS:
         return all(_skinny_ok(a, b, AUTO_MAX_ROWS) for b in bs)
-    return (a.shape[0] <= MFMA_AUTO_ROWS and sum(b.shape[1] for b in bs) <= MFMA_AUTO_MAX_COLS
-            and all(_skinny_ok(a, b) and b.shape[1] % 128 == 0 for b in bs)
-            and a.shape[1] % 8 == 0 and a.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0)
+    return _mfma_ok(a, bs) and not _library_only(a, *bs)
 
 
 def matmul_shared_input(a: torch.Tensor, bs):
@@ -202,9 +225,11 @@ def matmul_shared_input(a: torch.Tensor, bs):
 
 def swiglu_matmul(gate: torch.Tensor, up: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     """matmul(F.silu(gate) * up, b), the activation folded into the skinny
-    kernel's load of its input when the product qualifies for it."""
+    kernels' load of their input when the product qualifies for them."""
     if (gate.ndim == 2 and gate.shape == up.shape and gate.dtype == up.dtype == b.dtype and gate.is_cuda
-            and b.ndim == 2 and b.shape[0] == up.shape[1] and gate.stride(1) == 1 and _skinny_ok(up, b, AUTO_MAX_ROWS)):
+            and up.is_cuda and b.is_cuda and b.ndim == 2 and b.shape[0] == up.shape[1] and gate.stride(1) == 1
+            and (_skinny_ok(up, b, AUTO_MAX_ROWS) or (
+                _mfma_ok(up, [b]) and _rows_addressable(gate) and not _library_only(gate, up, b)))):
         return skinny_matmul_group(up, [b], gate=gate)[0]
     return matmul(torch.nn.functional.silu(gate) * up, b)
 

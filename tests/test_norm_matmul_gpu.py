@@ -359,3 +359,50 @@ def test_gemv_abi_empty_k(M):
     _lib.gemv(args, _lib.current_stream(x.device))
     torch.cuda.synchronize()
     assert (y == 0).all()
+
+
+@pytest.mark.parametrize("M", [3, 15, 16, 17, 31, 32])
+@pytest.mark.parametrize("K,N", [(8, 128), (40, 128), (96, 256), (264, 4096), (1032, 128), (8200, 128), (4096, 32896)])
+def test_skinny_matmul_mfma_edges(M, K, N):
+    """The MFMA kernel at the edges of its 16-row blocks, 32-row steps and
+    K-ranges (steps that end inside a range, waves with no step, one split and
+    the most), with row strides on every operand, rows past the matrices that
+    hold NaN, and the gate: within one rounding of the fp64 product."""
+    from lightserve_amd.kernels.tiled_matmul import skinny_matmul, skinny_matmul_group
+    print(f"case gemv mfma edges M={M} K={K} N={N}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    xb = torch.full((M + 1, K + 8), float("nan"), device="cuda", dtype=torch.bfloat16)
+    wb = torch.full((K + 32, N + 16), float("nan"), device="cuda", dtype=torch.bfloat16)
+    x, w = xb[:M, :K], wb[:K, 8:N + 8]
+    x.copy_(torch.randn(M, K, device="cuda", generator=g))
+    w.copy_(torch.randn(K, N, device="cuda", generator=g) / K ** 0.5)
+    yb = torch.zeros(M, N + 3, device="cuda", dtype=torch.bfloat16)
+    y = skinny_matmul(x, w, out=yb[:, 1:N + 1])
+    torch.cuda.synchronize()
+    _assert_one_rounding(y, x, w)
+    assert (yb[:, :1] == 0).all() and (yb[:, N + 1:] == 0).all()
+    gate = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
+    act = torch.nn.functional.silu(gate) * x
+    assert torch.equal(skinny_matmul_group(x, [w], gate=gate)[0], skinny_matmul(act, w))
+
+
+@pytest.mark.parametrize("M", [3, 9, 32, 33])
+def test_matmul_routes_keep_torch_semantics(M):
+    """matmul, matmul_shared_input and swiglu_matmul at the row counts around
+    the MFMA kernel's range: equal to the fp64 product, and differentiable as
+    torch.matmul is (a recorded gradient keeps the call on torch's operators)."""
+    from lightserve_amd.kernels.tiled_matmul import matmul_shared_input, swiglu_matmul
+    print(f"case matmul routes M={M}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x, gate = (torch.randn(M, 512, device="cuda", generator=g).to(torch.bfloat16) for _ in range(2))
+    ws = [(torch.randn(512, n, device="cuda", generator=g) / 512 ** 0.5).to(torch.bfloat16) for n in (256, 128, 200)]
+    for c, w in zip(matmul_shared_input(x, ws), ws):
+        _assert_one_rounding(c, x, w)
+    act = torch.nn.functional.silu(gate) * x
+    _assert_one_rounding(swiglu_matmul(gate, x, ws[0]), act, ws[0])
+    leaf, up, wl = (t.clone().requires_grad_() for t in (gate, x, ws[0]))
+    for grads in (torch.autograd.grad(matmul(up, wl).float().sum(), (up, wl)),
+                  torch.autograd.grad(swiglu_matmul(leaf, up, wl).float().sum(), (leaf, up, wl))):
+        assert all(t is not None and torch.isfinite(t).all() for t in grads)
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert matmul(x, ws[0]).dtype == torch.float16
