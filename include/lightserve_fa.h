@@ -464,6 +464,15 @@ int lsfa_fwd_check(const lsfa_fwd_args* args);
  * stream is a hipStream_t (NULL = the default stream). */
 int lsfa_fwd(const lsfa_fwd_args* args, void* stream);
 
+/* The same forward with each query tile's keys shared out over several
+ * workgroups where the launch has too few tiles to fill the GPU (bf16/fp16).
+ * Needs lsfa_fwd_workspace_size() bytes of caller-allocated device memory,
+ * 256-byte aligned (0 bytes: the launch is not split and workspace may be
+ * NULL); its contents on entry do not matter and are scratch afterwards.
+ * Deterministic; the partial results are fp32. */
+int lsfa_fwd_workspace_size(const lsfa_fwd_args* args, uint64_t* bytes);
+int lsfa_fwd_split(const lsfa_fwd_args* args, void* workspace, uint64_t workspace_bytes, void* stream);
+
 /* Host-only validation of backward arguments; never touches the GPU. */
 int lsfa_bwd_check(const lsfa_bwd_args* args);
 
@@ -520,6 +529,11 @@ int lsfa_prefill_paged_check(const lsfa_prefill_paged_args* args);
  * forward kernel of lsfa_fwd with K/V tiles gathered through the block
  * tables. No reference counterpart. */
 int lsfa_prefill_paged(const lsfa_prefill_paged_args* args, void* stream);
+
+/* The same with the keys of each query tile split, as lsfa_fwd_split. */
+int lsfa_prefill_paged_workspace_size(const lsfa_prefill_paged_args* args, uint64_t* bytes);
+int lsfa_prefill_paged_split(const lsfa_prefill_paged_args* args, void* workspace, uint64_t workspace_bytes,
+                             void* stream);
 
 /* Host-only validation of skinny-GEMM arguments; never touches the GPU. */
 int lsfa_gemv_check(const lsfa_gemv_args* args);

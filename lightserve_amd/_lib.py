@@ -24,10 +24,12 @@ TORCH_TO_LSFA = {torch.float32: DTYPE_FP32, torch.float16: DTYPE_FP16, torch.bfl
 STATUS = {0: "LSFA_OK", -1: "LSFA_ERR_INVALID", -2: "LSFA_ERR_UNSUPPORTED", -3: "LSFA_ERR_LAUNCH"}
 
 EXPORTED_SYMBOLS = ("lsfa_abi_version", "lsfa_last_error", "lsfa_fwd_check", "lsfa_fwd",
+                    "lsfa_fwd_workspace_size", "lsfa_fwd_split",
                     "lsfa_bwd_check", "lsfa_bwd_workspace_size", "lsfa_bwd", "lsfa_bwd_noalloc",
                     "lsfa_decode_check", "lsfa_decode_workspace_size", "lsfa_decode",
                     "lsfa_rope_check", "lsfa_rope", "lsfa_rmsnorm_check", "lsfa_rmsnorm",
                     "lsfa_prefill_paged_check", "lsfa_prefill_paged",
+                    "lsfa_prefill_paged_workspace_size", "lsfa_prefill_paged_split",
                     "lsfa_gemv_check", "lsfa_gemv_workspace_size", "lsfa_gemv",
                     "lsfa_gemv_group_check", "lsfa_gemv_group_workspace_size", "lsfa_gemv_group",
                     "lsfa_greedy_check", "lsfa_greedy")
@@ -210,6 +212,11 @@ def load():
             fn = getattr(lib, name)
             fn.restype = ctypes.c_int
             fn.argtypes = [ctypes.POINTER(struct), ctypes.c_void_p]
+        for name, struct in (("lsfa_fwd", FwdArgs), ("lsfa_prefill_paged", PrefillPagedArgs)):
+            size, split = getattr(lib, name + "_workspace_size"), getattr(lib, name + "_split")
+            size.restype = split.restype = ctypes.c_int
+            size.argtypes = [ctypes.POINTER(struct), ctypes.POINTER(ctypes.c_uint64)]
+            split.argtypes = [ctypes.POINTER(struct), ctypes.c_void_p, ctypes.c_uint64, ctypes.c_void_p]
         lib.lsfa_bwd_workspace_size.restype = ctypes.c_int
         lib.lsfa_bwd_workspace_size.argtypes = [ctypes.POINTER(BwdArgs), ctypes.POINTER(ctypes.c_uint64)]
         lib.lsfa_gemv_group_workspace_size.restype = ctypes.c_int
@@ -278,6 +285,19 @@ def prefill_paged(args, stream):
     _raise_on(load().lsfa_prefill_paged(ctypes.byref(args), ctypes.c_void_p(stream)), "lsfa_prefill_paged")
 
 
+def prefill_paged_workspace_size(args):
+    """Bytes of device workspace lsfa_prefill_paged_split needs (host only; 0 when unsplit)."""
+    n = ctypes.c_uint64(0)
+    _raise_on(load().lsfa_prefill_paged_workspace_size(ctypes.byref(args), ctypes.byref(n)),
+              "lsfa_prefill_paged_workspace_size")
+    return n.value
+
+
+def prefill_paged_split(args, workspace, nbytes, stream):
+    _raise_on(load().lsfa_prefill_paged_split(ctypes.byref(args), ctypes.c_void_p(workspace), nbytes,
+                                              ctypes.c_void_p(stream)), "lsfa_prefill_paged_split")
+
+
 def gemv_check(args):
     """Host-only validation (no GPU access); returns (status, message)."""
     rc = load().lsfa_gemv_check(ctypes.byref(args))
@@ -344,6 +364,18 @@ def rmsnorm(args, stream):
 
 def fwd(args, stream):
     _raise_on(load().lsfa_fwd(ctypes.byref(args), ctypes.c_void_p(stream)), "lsfa_fwd")
+
+
+def fwd_workspace_size(args):
+    """Bytes of device workspace lsfa_fwd_split needs (host only; 0 when unsplit)."""
+    n = ctypes.c_uint64(0)
+    _raise_on(load().lsfa_fwd_workspace_size(ctypes.byref(args), ctypes.byref(n)), "lsfa_fwd_workspace_size")
+    return n.value
+
+
+def fwd_split(args, workspace, nbytes, stream):
+    _raise_on(load().lsfa_fwd_split(ctypes.byref(args), ctypes.c_void_p(workspace), nbytes, ctypes.c_void_p(stream)),
+              "lsfa_fwd_split")
 
 
 def bwd(args, stream):

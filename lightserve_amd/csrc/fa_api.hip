@@ -13,6 +13,8 @@
 
 namespace lsfa {
 hipError_t fwd_mfma(FwdParams p, bool is_bf16, int dp, bool causal, bool varlen, hipStream_t s);
+int fwd_splits(int B, int Hq, int Nq, int dp, long long max_keys);
+uint64_t fwd_part_bytes(int B, int Hq, int Nq, int dp, int splits);
 hipError_t fwd_paged(FwdParams p, bool is_bf16, int dp, bool causal, hipStream_t s);
 hipError_t bwd_mfma(const BwdParams& p, bool is_bf16, int dp, bool causal, int phases, hipStream_t s);
 hipError_t fwd_f32(const FwdParams& p, int dp, bool causal, bool varlen, float scale, hipStream_t s);
@@ -205,12 +207,37 @@ int lsfa_fwd_check(const lsfa_fwd_args* a) {
   return ok();
 }
 
-int lsfa_fwd(const lsfa_fwd_args* a, void* stream) {
-  int rc = lsfa_fwd_check(a);
+// Checks the workspace of a key-split forward of `need` bytes.
+static int check_split_workspace(const char* query, const void* workspace, uint64_t bytes, uint64_t need) {
+  if (need == 0) return ok();
+  if (!workspace) return fail(LSFA_ERR_INVALID, "workspace must be non-NULL");
+  if (bytes < need)
+    return fail(LSFA_ERR_INVALID, "workspace_bytes %llu is below the %llu bytes %s asks for", (unsigned long long)bytes,
+                (unsigned long long)need, query);
+  if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0)
+    return fail(LSFA_ERR_INVALID, "workspace is not 256-byte aligned");
+  return ok();
+}
+
+static int fwd_split_count(const lsfa_fwd_args* a) {
+  if (a->dtype == LSFA_DTYPE_FP32) return 1;
+  return lsfa::fwd_splits(a->batch, a->heads_q, a->seqlen_q, padded_dim(a->head_dim), a->seqlen_k);
+}
+
+int lsfa_fwd_workspace_size(const lsfa_fwd_args* a, uint64_t* bytes) {
+  if (a == nullptr || bytes == nullptr) return fail(LSFA_ERR_INVALID, "args or bytes is NULL");
+  int rc = check_common(a->dtype, a->batch, a->heads_q, a->heads_kv, a->seqlen_q, a->seqlen_k, a->head_dim, a->sm_scale);
   if (rc) return rc;
+  *bytes = lsfa::fwd_part_bytes(a->batch, a->heads_q, a->seqlen_q, padded_dim(a->head_dim), fwd_split_count(a));
+  return ok();
+}
+
+static int run_fwd(const lsfa_fwd_args* a, int splits, void* workspace, void* stream) {
   if ((long long)a->batch * a->heads_q * a->seqlen_q == 0) return ok();
   lsfa::FwdParams p;
   memset(&p, 0, sizeof(p));
+  p.splits = splits;
+  p.part = static_cast<float*>(workspace);
   p.q = a->q;
   p.k = a->k;
   p.v = a->v;
@@ -240,6 +267,20 @@ int lsfa_fwd(const lsfa_fwd_args* a, void* stream) {
     e = lsfa::fwd_mfma(p, a->dtype == LSFA_DTYPE_BF16, dp, a->causal != 0, varlen, s);
   if (e != hipSuccess) return fail(LSFA_ERR_LAUNCH, "forward launch failed: %s", hipGetErrorString(e));
   return ok();
+}
+
+int lsfa_fwd(const lsfa_fwd_args* a, void* stream) {
+  const int rc = lsfa_fwd_check(a);
+  return rc ? rc : run_fwd(a, 1, nullptr, stream);
+}
+
+int lsfa_fwd_split(const lsfa_fwd_args* a, void* workspace, uint64_t workspace_bytes, void* stream) {
+  int rc = lsfa_fwd_check(a);
+  if (rc) return rc;
+  uint64_t need = 0;
+  if ((rc = lsfa_fwd_workspace_size(a, &need))) return rc;
+  if ((rc = check_split_workspace("lsfa_fwd_workspace_size", workspace, workspace_bytes, need))) return rc;
+  return run_fwd(a, need > 0 ? fwd_split_count(a) : 1, workspace, stream);
 }
 
 int lsfa_bwd_check(const lsfa_bwd_args* a) {
@@ -546,12 +587,25 @@ int lsfa_prefill_paged_check(const lsfa_prefill_paged_args* a) {
   return ok();
 }
 
-int lsfa_prefill_paged(const lsfa_prefill_paged_args* a, void* stream) {
-  int rc = lsfa_prefill_paged_check(a);
-  if (rc) return rc;
+static int prefill_split_count(const lsfa_prefill_paged_args* a) {
+  if (a->batch <= 0 || a->max_seqlen_q <= 0 || a->heads_q <= 0 || a->max_blocks_per_seq <= 0 || a->block_size <= 0)
+    return 1;
+  return lsfa::fwd_splits(a->batch, a->heads_q, a->max_seqlen_q, padded_dim(a->head_dim),
+                          (long long)a->max_blocks_per_seq * a->block_size);
+}
+
+int lsfa_prefill_paged_workspace_size(const lsfa_prefill_paged_args* a, uint64_t* bytes) {
+  if (a == nullptr || bytes == nullptr) return fail(LSFA_ERR_INVALID, "args or bytes is NULL");
+  *bytes = lsfa::fwd_part_bytes(a->batch, a->heads_q, a->max_seqlen_q, padded_dim(a->head_dim), prefill_split_count(a));
+  return ok();
+}
+
+static int run_prefill_paged(const lsfa_prefill_paged_args* a, int splits, void* workspace, void* stream) {
   if (a->batch == 0 || a->max_seqlen_q == 0) return ok();
   lsfa::FwdParams p;
   memset(&p, 0, sizeof(p));
+  p.splits = splits;
+  p.part = static_cast<float*>(workspace);
   p.q = a->q; p.k = a->k_cache; p.v = a->v_cache; p.o = a->o; p.lse = a->lse;
   p.sqn = a->q_stride[0]; p.sqh = a->q_stride[1];
   p.skb = a->k_stride[0]; p.skn = a->k_stride[1]; p.skh = a->k_stride[2];
@@ -573,6 +627,20 @@ int lsfa_prefill_paged(const lsfa_prefill_paged_args* a, void* stream) {
                                  reinterpret_cast<hipStream_t>(stream));
   if (e != hipSuccess) return fail(LSFA_ERR_LAUNCH, "paged prefill launch failed: %s", hipGetErrorString(e));
   return ok();
+}
+
+int lsfa_prefill_paged(const lsfa_prefill_paged_args* a, void* stream) {
+  const int rc = lsfa_prefill_paged_check(a);
+  return rc ? rc : run_prefill_paged(a, 1, nullptr, stream);
+}
+
+int lsfa_prefill_paged_split(const lsfa_prefill_paged_args* a, void* workspace, uint64_t workspace_bytes, void* stream) {
+  int rc = lsfa_prefill_paged_check(a);
+  if (rc) return rc;
+  uint64_t need = 0;
+  if ((rc = lsfa_prefill_paged_workspace_size(a, &need))) return rc;
+  if ((rc = check_split_workspace("lsfa_prefill_paged_workspace_size", workspace, workspace_bytes, need))) return rc;
+  return run_prefill_paged(a, need > 0 ? prefill_split_count(a) : 1, workspace, stream);
 }
 
 }  // extern "C"

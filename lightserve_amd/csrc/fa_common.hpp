@@ -162,6 +162,10 @@ struct FwdParams {
   int heads_per_group;  // map_tile grouping
   float scale_log2;  // |sm_scale| * log2(e), at least 1e-30
   int neg_q;         // sm_scale < 0: q is negated on load so scale_log2 stays positive
+  // Key splits (more than one: each item's keys are shared out over that many
+  // workgroups, whose partial results meet in part).
+  int splits;
+  float* part;
 };
 
 struct BwdParams {

@@ -42,6 +42,7 @@
 // LDS tile is the same as for contiguous K/V. Block ids outside
 // [0, num_blocks) read as zeros.
 #include "fa_common.hpp"
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -53,10 +54,11 @@ constexpr float kLn2 = 0.6931471805599453f;
 template <typename T> constexpr float kMaxLog2P = 64.0f;
 template <> constexpr float kMaxLog2P<_Float16> = 15.0f;
 
-__device__ __forceinline__ int wave_sum_i(int v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
+// Sum over lanes 0 .. width-1 (a power of two; v is 0 in the lanes past it),
+// wave-uniform.
+__device__ __forceinline__ int wave_sum_i(int v, int width) {
+  for (int o = width >> 1; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  return __builtin_amdgcn_readfirstlane(v);
 }
 
 // Number of a sequence's query tiles (tq of them, BM rows each) whose key
@@ -79,6 +81,8 @@ __device__ __forceinline__ int tiles_above(int x, int tq, int nk, int off) {
 // Lane i holds sequence i (B <= 64). The key tile count of the item at the
 // rank is found by binary search on the number of items above a count, then
 // the item among those of that count by a prefix sum over the sequences.
+// The sums run over the lanes that hold a sequence only: each shuffle costs an
+// LDS round trip in a chain of about 10 log2(B), before the first load.
 // Wave-uniform result.
 template <bool CAUSAL, bool PAGED, int BM>
 __device__ __forceinline__ void varlen_item_at(const FwdParams& p, int rank, int lane, int& b_out, int& qt_out) {
@@ -90,16 +94,16 @@ __device__ __forceinline__ void varlen_item_at(const FwdParams& p, int rank, int
     tq = nq > 0 ? (nq + BM - 1) / BM : 0;
     off = nk - nq;
   }
+  const int width = p.B > 1 ? 1 << (32 - __builtin_clz(p.B - 1)) : 1;
   b_out = -1;
   qt_out = 0;
-  if (rank >= wave_sum_i(tq)) return;
+  if (rank >= wave_sum_i(tq, width)) return;
   int kmax = nk > 0 ? (nk + 63) >> 6 : 0;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) kmax = max(kmax, __shfl_xor(kmax, o));
+  for (int o = width >> 1; o > 0; o >>= 1) kmax = max(kmax, __shfl_xor(kmax, o));
   int lo = 0, hi = __builtin_amdgcn_readfirstlane(kmax);  // no item exceeds hi
   while (lo < hi) {
     const int mid = (lo + hi) >> 1;
-    if (__builtin_amdgcn_readfirstlane(wave_sum_i(tiles_above<CAUSAL, BM>(mid, tq, nk, off))) <= rank) hi = mid;
+    if (wave_sum_i(tiles_above<CAUSAL, BM>(mid, tq, nk, off), width) <= rank) hi = mid;
     else lo = mid + 1;
   }
   // rank lies among the items of exactly lo key tiles: tiles
@@ -107,10 +111,9 @@ __device__ __forceinline__ void varlen_item_at(const FwdParams& p, int rank, int
   const int a_hi = tiles_above<CAUSAL, BM>(lo - 1, tq, nk, off);
   const int a_lo = tiles_above<CAUSAL, BM>(lo, tq, nk, off);
   const int c = a_hi - a_lo;
-  const int k = rank - __builtin_amdgcn_readfirstlane(wave_sum_i(a_lo));
+  const int k = rank - wave_sum_i(a_lo, width);
   int inc = c;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
+  for (int o = 1; o < width; o <<= 1) {
     const int t = __shfl_up(inc, o);
     if (lane >= o) inc += t;
   }
@@ -121,11 +124,64 @@ __device__ __forceinline__ void varlen_item_at(const FwdParams& p, int rank, int
   qt_out = __builtin_amdgcn_readfirstlane(__shfl(tq - a_hi + k - pre, src));
 }
 
+// The (batch, head, query tile) of workgroup blockIdx.x; false past the last.
+template <bool CAUSAL, bool VARLEN, bool PAGED, int BM>
+__device__ __forceinline__ bool item_at(const FwdParams& p, int lane, int& b, int& h, int& qt) {
+  if (VARLEN && p.B <= 64) {
+    // Varlen sequences differ in length: workgroup L takes the item of rank
+    // L / Hq in longest-first order, for head slot L % Hq. Workgroups go to
+    // the XCDs round-robin, so with Hq a multiple of 8 XCD x gets slots
+    // x, x+8, ..., mapped to the adjacent heads x*Hq/8 .. (with GQA, query
+    // heads that share K/V), every rank in order.
+    const int L = blockIdx.x;
+    const int rank = L / p.Hq, u = L - rank * p.Hq;
+    h = (p.Hq & 7) == 0 ? (u & 7) * (p.Hq >> 3) + (u >> 3) : u;
+    varlen_item_at<CAUSAL, PAGED, BM>(p, rank, lane, b, qt);
+    return b >= 0;
+  } else {
+    int bh;
+    map_tile(p.num_q_tiles, gridDim.x, p.heads_per_group, bh, qt, CAUSAL);
+    // Longer varlen batches: the (sequence, head) index runs head-major, so
+    // each XCD's contiguous run of indices holds a few heads of every
+    // sequence instead of all heads of one sequence.
+    b = VARLEN ? bh % p.B : bh / p.Hq;
+    h = VARLEN ? bh / p.B : bh - b * p.Hq;
+  }
+  return true;
+}
+
+// Key tiles [lo, hi) of split `split` of an item of ntiles tiles over at most
+// `most` splits, and how many splits the item has: at least kSplitMinTiles
+// tiles each, an even number (the tiles' LDS buffers go by parity).
+constexpr int kSplitMinTiles = 4;
+__device__ __forceinline__ int split_tiles(int ntiles, int most, int split, int& lo, int& hi) {
+  const int want = max(1, min(most, ntiles / kSplitMinTiles));
+  const int per = ((ntiles + want - 1) / want + 1) & ~1;
+  lo = split * per;
+  hi = min(ntiles, lo + per);
+  return per > 0 ? max(1, (ntiles + per - 1) / per) : 1;
+}
+// Partials of an item's splits in p.part, in floats: per split the stats of
+// its BM rows (offset, sum for O, sum for the lse, unused), then O in the
+// accumulators' own order, [wave][32 columns][4 registers][lane] float4, so
+// that both sides move whole kilobytes. Behind all items, one int4 per item:
+// b, h, first query row (-1: no item), splits.
+template <int BM, int DP> constexpr int kPartFloats = BM * 4 + BM * DP;
+template <int BM, int DP>
+__device__ __forceinline__ u32x4* split_header(const FwdParams& p, int items, int item) {
+  return (u32x4*)(p.part + (int64_t)items * p.splits * kPartFloats<BM, DP>) + item;
+}
+
 // NW waves per workgroup (NW x 32 query rows): 4 (two workgroups per CU) or,
 // for long dense sequences and varlen batches with long query runs,
 // 8 (one per CU), so that every K/V tile brought into LDS serves twice the
 // rows.
-template <typename T, int DP, bool CAUSAL, bool VARLEN, bool LSE, bool PAGED, int NW>
+//
+// SPLIT: the item's key tiles are shared out over gridDim.y workgroups
+// (split_tiles); each leaves its unnormalised fp32 O, the exponent offset and
+// the row sums in p.part, and fa_fwd_combine_kernel merges them. An item of
+// too few tiles keeps one workgroup, which stores O itself.
+template <typename T, int DP, bool CAUSAL, bool VARLEN, bool LSE, bool PAGED, int NW, bool SPLIT>
 __global__ __launch_bounds__((NW * 64), (8 / NW)) void fa_fwd_kernel(const FwdParams p) {
   using X8 = typename VecT<T>::x8;
   using X4 = typename VecT<T>::x4;
@@ -162,25 +218,11 @@ __global__ __launch_bounds__((NW * 64), (8 / NW)) void fa_fwd_kernel(const FwdPa
   const bool loads = !kSecondLoads || wave >= NW / 2;  // wave-uniform
   const int lw = kSecondLoads ? (wave & (NW / 2 - 1)) : wave;  // this wave's chunk group
   int b, h, qt;
-  if (VARLEN && p.B <= 64) {
-    // Varlen sequences differ in length: workgroup L takes the item of rank
-    // L / Hq in longest-first order, for head slot L % Hq. Workgroups go to
-    // the XCDs round-robin, so with Hq a multiple of 8 XCD x gets slots
-    // x, x+8, ..., mapped to the adjacent heads x*Hq/8 .. (with GQA, query
-    // heads that share K/V), every rank in order.
-    const int L = blockIdx.x;
-    const int rank = L / p.Hq, u = L - rank * p.Hq;
-    h = (p.Hq & 7) == 0 ? (u & 7) * (p.Hq >> 3) + (u >> 3) : u;
-    varlen_item_at<CAUSAL, PAGED, BM>(p, rank, lane, b, qt);
-    if (b < 0) return;  // uniform, before any barrier
-  } else {
-    int bh;
-    map_tile(p.num_q_tiles, gridDim.x, p.heads_per_group, bh, qt, CAUSAL);
-    // Longer varlen batches: the (sequence, head) index runs head-major, so
-    // each XCD's contiguous run of indices holds a few heads of every
-    // sequence instead of all heads of one sequence.
-    b = VARLEN ? bh % p.B : bh / p.Hq;
-    h = VARLEN ? bh / p.B : bh - b * p.Hq;
+  if (!item_at<CAUSAL, VARLEN, PAGED, BM>(p, lane, b, h, qt)) {  // uniform, before any barrier
+    if constexpr (SPLIT)
+      if (blockIdx.y == 0 && tid == 0)
+        *split_header<BM, DP>(p, gridDim.x, blockIdx.x) = u32x4{0u, 0u, (uint32_t)-1, 1u};
+    return;
   }
   const int hk = h / (p.Hq / p.Hkv);
   int nq = p.Nq, nk = p.Nk;
@@ -196,7 +238,12 @@ __global__ __launch_bounds__((NW * 64), (8 / NW)) void fa_fwd_kernel(const FwdPa
     }
   }
   const int q0 = qt * BM;
-  if (q0 >= nq) return;  // uniform across the workgroup, before any barrier
+  if (q0 >= nq) {  // uniform across the workgroup, before any barrier
+    if constexpr (SPLIT)
+      if (blockIdx.y == 0 && tid == 0)
+        *split_header<BM, DP>(p, gridDim.x, blockIdx.x) = u32x4{0u, 0u, (uint32_t)-1, 1u};
+    return;
+  }
   const int off = nk - nq;  // bottom-right causal alignment
 
   const T* Q = (const T*)p.q + (VARLEN ? 0 : (int64_t)b * p.sqb) + (int64_t)h * p.sqh + rq0 * p.sqn;
@@ -208,7 +255,17 @@ __global__ __launch_bounds__((NW * 64), (8 / NW)) void fa_fwd_kernel(const FwdPa
 
   int kv_end = nk;
   if (CAUSAL) kv_end = min(nk, q0 + BM + off);
-  const int ntiles = kv_end > 0 ? (kv_end + BN - 1) / BN : 0;
+  int ntiles = kv_end > 0 ? (kv_end + BN - 1) / BN : 0;
+  // This workgroup's tiles are first .. ntiles - 1 (first is even).
+  int first = 0, splits = 1;
+  if constexpr (SPLIT) {
+    int hi;
+    splits = split_tiles(ntiles, gridDim.y, blockIdx.y, first, hi);
+    if ((int)blockIdx.y >= splits) return;  // uniform, before any barrier
+    ntiles = hi;
+    if (blockIdx.y == 0 && tid == 0)
+      *split_header<BM, DP>(p, gridDim.x, blockIdx.x) = u32x4{(uint32_t)b, (uint32_t)h, (uint32_t)q0, (uint32_t)splits};
+  }
 
   const int D = p.D;
   const int qw_lo = q0 + wave * 32;
@@ -448,13 +505,13 @@ __global__ __launch_bounds__((NW * 64), (8 / NW)) void fa_fwd_kernel(const FwdPa
   };
 
   // blk1, blk2: blocks of tiles t+1 and t+2 for the next pipelined step t.
-  const int blk0 = block_of(0);
-  int blk1 = block_of(1), blk2 = block_of(2);
-  if (ntiles > 0) {
-    tile_load(K, p.skn, p.skb, p.skh, kvo, 0, 0, blk0);
-    tile_load(V, p.svn, p.svb, p.svh, vvo, 0, 2, blk0);
+  const int blk0 = block_of(first);
+  int blk1 = block_of(first + 1), blk2 = block_of(first + 2);
+  if (ntiles > first) {
+    tile_load(K, p.skn, p.skb, p.skh, kvo, first, 0, blk0);
+    tile_load(V, p.svn, p.svb, p.svh, vvo, first, 2, blk0);
   }
-  if (ntiles > 1) tile_load(K, p.skn, p.skb, p.skh, kvo, 1, 1, blk1);
+  if (ntiles > first + 1) tile_load(K, p.skn, p.skb, p.skh, kvo, first + 1, 1, blk1);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
 
@@ -462,9 +519,9 @@ __global__ __launch_bounds__((NW * 64), (8 / NW)) void fa_fwd_kernel(const FwdPa
   // keys keep -1e30: their first visible tile then takes the check's slow
   // path, which raises the offset to that tile's max).
   f32x16 s0[KB], s1[KB];
-  if (ntiles > 0 && wave_sees(0)) {
+  if (ntiles > first && wave_sees(first)) {
     scores(kbuf(0), s0);
-    mask_tile(0, s0);
+    mask_tile(first, s0);
     m_run = fmaxf(row_max(s0), -1e30f);
   }
   __syncthreads();  // K buffer 0 is refilled by the first step
@@ -496,7 +553,7 @@ __global__ __launch_bounds__((NW * 64), (8 / NW)) void fa_fwd_kernel(const FwdPa
     }
     __syncthreads();
   };
-  int j = 0;
+  int j = first;
   for (; j + 1 < ntiles; j += 2) {
     pipe_step(j, s0, s1);
     pipe_step(j + 1, s1, s0);
@@ -504,6 +561,20 @@ __global__ __launch_bounds__((NW * 64), (8 / NW)) void fa_fwd_kernel(const FwdPa
   if (j < ntiles) pipe_step(j, s0, s1);
 
   const float lt = half_sum(l_run);
+  if constexpr (SPLIT) {
+    if (splits > 1) {
+      const float le = half_sum(l_lse);
+      float* part = p.part + ((int64_t)blockIdx.x * p.splits + blockIdx.y) * kPartFloats<BM, DP>;
+      if (hh == 0) *(f32x4*)(part + (wave * 32 + l32) * 4) = f32x4{m_run, lt, le, 0.f};
+      f32x4* po = (f32x4*)(part + BM * 4) + wave * DT * 4 * 64 + lane;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          po[(dt * 4 + g) * 64] = f32x4{acc[dt][4 * g], acc[dt][4 * g + 1], acc[dt][4 * g + 2], acc[dt][4 * g + 3]};
+      return;
+    }
+  }
   const float inv = lt > 0.f ? 1.f / lt : 0.f;
   // O leaves through LDS: a lane's accumulators hold 4-column pieces of one
   // query's row, so direct stores would scatter 8-byte pieces over 32 rows
@@ -536,11 +607,88 @@ __global__ __launch_bounds__((NW * 64), (8 / NW)) void fa_fwd_kernel(const FwdPa
   if (qrow < nq) {
     if constexpr (LSE) {
       const float le = half_sum(l_lse);
-      if (hh == 0) {
+      if (hh == 0 && (!SPLIT || p.lse != nullptr)) {
         float* L = p.lse + (VARLEN ? 0 : (int64_t)b * p.slb) + (int64_t)h * p.slh + (rq0 + qrow) * p.sln;
         *L = le > 0.f ? (m_run + __log2f(le)) * kLn2 : -INFINITY;
       }
     }
+  }
+}
+
+// Merges the key splits of fa_fwd_kernel<..., SPLIT>: workgroup (item, dt)
+// combines 32 columns of the item's rows, wave w rows 32 w .. 32 w + 31, in the
+// layout the accumulators had. Items that were not split are already stored.
+template <typename T, int DP, bool VARLEN, int NW>
+__global__ __launch_bounds__(NW * 64) void fa_fwd_combine_kernel(const FwdParams p) {
+  using X4 = typename VecT<T>::x4;
+  constexpr int BM = NW * 32, DT = DP / 32;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, hh = lane >> 5, dt = blockIdx.y;
+  const u32x4 head = *split_header<BM, DP>(p, gridDim.x, blockIdx.x);
+  const int b = head[0], h = head[1], q0 = head[2], splits = head[3];
+  if (splits <= 1) return;
+  int nq = p.Nq;
+  int64_t rq0 = 0;
+  if (VARLEN) {
+    rq0 = p.cu_q[b];
+    nq = p.cu_q[b + 1] - (int)rq0;
+  }
+  const int qrow = q0 + wave * 32 + l32;
+  const float* part = p.part + (int64_t)blockIdx.x * p.splits * kPartFloats<BM, DP>;
+  // Four splits at a time, their loads in flight together; the running offset
+  // M is the largest among the splits that saw a key of the row (a NaN sum
+  // counts as seen: O comes out NaN).
+  constexpr int SB = 4;
+  float M = -INFINITY, lt = 0.f, le = 0.f;
+  f32x4 acc[4];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) acc[g] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < splits; s0 += SB) {
+    f32x4 st[SB], v[SB][4];
+#pragma unroll
+    for (int i = 0; i < SB; ++i) {
+      const float* ps = part + (int64_t)min(s0 + i, splits - 1) * kPartFloats<BM, DP>;
+      st[i] = *(const f32x4*)(ps + (wave * 32 + l32) * 4);
+      const f32x4* po = (const f32x4*)(ps + BM * 4) + (wave * DT + dt) * 4 * 64 + lane;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) v[i][g] = po[g * 64];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    float mn = M;
+#pragma unroll
+    for (int i = 0; i < SB; ++i) mn = st[i][2] == 0.f ? mn : fmaxf(mn, st[i][0]);
+    const float a = M == -INFINITY ? 0.f : fast_exp2(M - mn);
+    M = mn;
+    lt *= a;
+    le *= a;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) acc[g] *= a;
+#pragma unroll
+    for (int i = 0; i < SB; ++i) {
+      const float w = (st[i][2] == 0.f || s0 + i >= splits) ? 0.f : fast_exp2(st[i][0] - M);
+      if (s0 + i < splits) {
+        lt += w * st[i][1];
+        le += w * st[i][2];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) acc[g] += w * v[i][g];
+      }
+    }
+  }
+  if (qrow >= nq) return;
+  const float inv = lt > 0.f ? 1.f / lt : 0.f;
+  T* O = (T*)p.o + (VARLEN ? 0 : (int64_t)b * p.sob) + (int64_t)h * p.soh + (rq0 + qrow) * p.son;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const int col = 32 * dt + 8 * g + 4 * hh;
+    X4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = (T)(acc[g][e] * inv);
+    if (col < p.D) *(X4*)(O + col) = v;  // D is a multiple of 8
+  }
+  if (dt == 0 && hh == 0 && p.lse != nullptr) {
+    float* L = p.lse + (VARLEN ? 0 : (int64_t)b * p.slb) + (int64_t)h * p.slh + (rq0 + qrow) * p.sln;
+    *L = le > 0.f ? (M + __log2f(le)) * kLn2 : -INFINITY;
   }
 }
 
@@ -1140,9 +1288,51 @@ static hipError_t launch_fwd_nw(FwdParams p, hipStream_t s) {
   p.num_q_tiles = (p.Nq + NW * 32 - 1) / (NW * 32);
   const int total = p.num_q_tiles * p.B * p.Hq;
   if (p.lse != nullptr)
-    hipLaunchKernelGGL((fa_fwd_kernel<T, DP, CAUSAL, VARLEN, true, PAGED, NW>), dim3(total), dim3(NW * 64), 0, s, p);
+    hipLaunchKernelGGL((fa_fwd_kernel<T, DP, CAUSAL, VARLEN, true, PAGED, NW, false>), dim3(total), dim3(NW * 64), 0, s, p);
   else
-    hipLaunchKernelGGL((fa_fwd_kernel<T, DP, CAUSAL, VARLEN, false, PAGED, NW>), dim3(total), dim3(NW * 64), 0, s, p);
+    hipLaunchKernelGGL((fa_fwd_kernel<T, DP, CAUSAL, VARLEN, false, PAGED, NW, false>), dim3(total), dim3(NW * 64), 0, s, p);
+  return hipGetLastError();
+}
+
+// Key splits (4-wave workgroups, two of which share a CU) of a launch of
+// B x Hq x ceil(Nq / 128) items over at most max_keys keys each: the count of
+// least estimated time, 1 where splitting does not pay. A 64-key step takes
+// about 1.2 us with one workgroup on its CU and 1.95 us with two; a split
+// launch adds 5 us (the combine launch and the partials' latency) and 23 ns per
+// workgroup for writing and reading its 64 KB of partials (head dim 128).
+// Measured, unsplit against split: 96 items of 100 tiles 154 -> 60 us (5
+// splits; 73 at 2), 128 of 64 87 -> 42 (4), 128 of 32 37 -> 30 (2; 29 at 4),
+// 252 of 125 167 -> 132 (2), but 128 of 8 14.5 -> 17.9 (2), 168 of 13 18.2 ->
+// 23.4 (3): both left unsplit by this rule.
+int fwd_splits(int B, int Hq, int Nq, int dp, long long max_keys) {
+  const long long items = (long long)B * Hq * ((Nq + 127) / 128);
+  const double tiles = (double)((max_keys + 63) / 64);
+  int best = 1;
+  double least = tiles * 1.2;
+  for (int s = 2; s <= 16 && items > 0 && items * s <= 512 && s * kSplitMinTiles <= tiles; ++s) {
+    const double us = tiles / s * (items * s <= 256 ? 1.2 : 1.95) + 5.0 + 0.023 * (double)(items * s) * dp / 128;
+    if (us < least) {
+      least = us;
+      best = s;
+    }
+  }
+  return best;
+}
+// Bytes of p.part for that launch.
+uint64_t fwd_part_bytes(int B, int Hq, int Nq, int dp, int splits) {
+  if (splits <= 1) return 0;
+  const uint64_t items = (uint64_t)B * Hq * ((Nq + 127) / 128);
+  return items * splits * (128 * 4 + 128 * dp) * 4 + items * 16;
+}
+
+template <typename T, int DP, bool CAUSAL, bool VARLEN, bool PAGED>
+static hipError_t launch_fwd_split(FwdParams p, hipStream_t s) {
+  p.num_q_tiles = (p.Nq + 127) / 128;
+  const int total = p.num_q_tiles * p.B * p.Hq;
+  hipLaunchKernelGGL((fa_fwd_kernel<T, DP, CAUSAL, VARLEN, true, PAGED, 4, true>), dim3(total, p.splits), dim3(256), 0, s, p);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((fa_fwd_combine_kernel<T, DP, VARLEN, 4>), dim3(total, DP / 32), dim3(256), 0, s, p);
   return hipGetLastError();
 }
 
@@ -1164,6 +1354,7 @@ static hipError_t launch_fwd_nw(FwdParams p, hipStream_t s) {
 // dim 64 it lost 1.7% there.
 template <typename T, int DP, bool CAUSAL, bool VARLEN, bool PAGED = false>
 static hipError_t launch_fwd(const FwdParams& p, hipStream_t s) {
+  if (p.splits > 1) return launch_fwd_split<T, DP, CAUSAL, VARLEN, PAGED>(p, s);
   if constexpr (!VARLEN && !PAGED && DP >= 64) {
     if (p.Nq >= (DP >= 128 ? 2048 : 4096)) {
       const int total = ((p.Nq + 255) / 256) * p.B * p.Hq;

@@ -20,6 +20,9 @@ import torch.nn.functional as F
 from .. import _lib
 
 SUPPORTED_DTYPES = (torch.float32, torch.float16, torch.bfloat16)
+# Launches of more 128-row query tiles, or of fewer keys, never split their
+# keys (lsfa_fwd_workspace_size is 0 there: no need to ask).
+SPLIT_MAX_TILES, SPLIT_MIN_KEYS = 256, 513
 
 
 def check_inputs(q, k, v):
@@ -66,6 +69,21 @@ def lse_args(lse):
     return lse.data_ptr(), _lib._i64x3(*lse.stride())
 
 
+def launch_forward(args, device):
+    """lsfa_fwd on the device's current stream, or lsfa_fwd_split with a
+    workspace where the launch has too few query tiles to fill the GPU."""
+    nbytes = 0
+    if (args.seqlen_k >= SPLIT_MIN_KEYS and args.dtype != _lib.DTYPE_FP32
+            and args.batch * args.heads_q * ((args.seqlen_q + 127) // 128) <= SPLIT_MAX_TILES):
+        nbytes = _lib.fwd_workspace_size(args)
+    with torch.cuda.device(device):
+        if nbytes > 0:
+            ws = torch.empty(nbytes, device=device, dtype=torch.uint8)  # 512-byte aligned blocks
+            _lib.fwd_split(args, ws.data_ptr(), nbytes, _lib.current_stream(device))
+        else:
+            _lib.fwd(args, _lib.current_stream(device))
+
+
 def forward_into(q, k, v, causal, scale, want_lse):
     """Runs the forward kernel; returns (o, lse or None). o is empty_like(q)."""
     B, H, N, D = q.shape
@@ -88,8 +106,7 @@ def forward_into(q, k, v, causal, scale, want_lse):
         dtype=_lib.TORCH_TO_LSFA[q.dtype], batch=B, heads_q=H, heads_kv=H, seqlen_q=N, seqlen_k=N,
         head_dim=dp, causal=int(bool(causal)), sm_scale=scale, reserved=0,
     )
-    with torch.cuda.device(q.device):
-        _lib.fwd(args, _lib.current_stream(q.device))
+    launch_forward(args, q.device)
     if ok is not o:
         o.copy_(ok[..., :D])
     return o, lse

@@ -17,7 +17,7 @@ import math
 import torch
 
 from .. import _lib
-from .flash_attention import SUPPORTED_DTYPES, as_kernel_layout, lse_args
+from .flash_attention import SUPPORTED_DTYPES, as_kernel_layout, launch_forward, lse_args
 
 
 def _check_varlen_inputs(q, k, v, cu_seqlens_q, cu_seqlens_k):
@@ -69,8 +69,7 @@ def flash_attention_varlen_forward(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seql
         seqlen_q=int(max_seqlen_q), seqlen_k=int(max_seqlen_k),
         head_dim=dp, causal=int(bool(causal)), sm_scale=scale, reserved=0,
     )
-    with torch.cuda.device(q.device):
-        _lib.fwd(args, _lib.current_stream(q.device))
+    launch_forward(args, q.device)
     if ok is not o:
         o.copy_(ok[..., :D])
     return o, lse

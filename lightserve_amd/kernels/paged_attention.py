@@ -40,6 +40,7 @@ import math
 import torch
 
 from .. import _lib
+from .flash_attention import SPLIT_MAX_TILES, SPLIT_MIN_KEYS
 
 
 def _check(q, k_cache, v_cache, block_tables, seq_lens):
@@ -136,6 +137,14 @@ def paged_prefill(q, k_cache, v_cache, block_tables, cu_seqlens_q, seq_lens_k, *
         max_seqlen_q=int(max_seqlen_q), causal=int(bool(causal)), sm_scale=scale, reserved=0,
     )
     if T > 0:
+        # few query tiles for the GPU: their keys are shared out over several workgroups
+        nbytes = 0
+        if bt.shape[1] * block_size >= SPLIT_MIN_KEYS and B * Hq * ((args.max_seqlen_q + 127) // 128) <= SPLIT_MAX_TILES:
+            nbytes = _lib.prefill_paged_workspace_size(args)
         with torch.cuda.device(q.device):
-            _lib.prefill_paged(args, _lib.current_stream(q.device))
+            if nbytes > 0:
+                ws = torch.empty(nbytes, device=q.device, dtype=torch.uint8)  # 512-byte aligned blocks
+                _lib.prefill_paged_split(args, ws.data_ptr(), nbytes, _lib.current_stream(q.device))
+            else:
+                _lib.prefill_paged(args, _lib.current_stream(q.device))
     return (o, lse) if return_lse else o

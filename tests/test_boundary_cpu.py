@@ -714,3 +714,44 @@ def test_integration_stub_binds_this_library(built_library):
     assert lib.lsfa_fwd_check(ctypes.byref(a)) == 0, lib.lsfa_last_error()
     a.head_dim = 12
     assert lib.lsfa_fwd_check(ctypes.byref(a)) != 0
+
+
+def test_abi_key_split_workspace(built_library):
+    """The key-split forward: workspace sizes are 0 where the launch is not
+    split (many query tiles, few keys, fp32, empty), positive and never above
+    512 workgroups' partials where it is; the entry points check the workspace
+    before any GPU call."""
+    def prefill(**kw):
+        return _prefill_args(**{**dict(batch=1, heads_q=32, heads_kv=8, head_dim=128, max_seqlen_q=333,
+                                       max_blocks_per_seq=400, block_table_stride=400), **kw})
+    most = 512 * (128 * 128 + 128 * 4) * 4 + 256 * 16
+    sizes = [_lib.prefill_paged_workspace_size(prefill(max_seqlen_q=n, max_blocks_per_seq=m, block_table_stride=m))
+             for n in (1, 16, 128, 333, 1024) for m in (40, 100, 400, 1000)]
+    assert any(sizes) and all(0 <= n <= most for n in sizes)
+    for kw in (dict(batch=16), dict(max_blocks_per_seq=8), dict(batch=0), dict(max_seqlen_q=0)):
+        assert _lib.prefill_paged_workspace_size(prefill(**kw)) == 0, kw
+    args = prefill()
+    need = _lib.prefill_paged_workspace_size(args)
+    for ws, n, word in ((None, need, "non-NULL"), (1 << 20, need - 1, "below"), ((1 << 20) + 64, need, "aligned")):
+        with pytest.raises(RuntimeError, match=word):
+            _lib.prefill_paged_split(args, ws, n, 0)
+
+    def dense(**kw):
+        base = dict(q=4096, k=4096, v=4096, o=4096, lse=None, dtype=_lib.DTYPE_BF16, batch=1, heads_q=4, heads_kv=4,
+                    seqlen_q=4096, seqlen_k=4096, head_dim=64, causal=1, sm_scale=0.125)
+        base.update(kw)
+        st = _lib._i64x4(1 << 20, 1 << 18, 64, 1)
+        return _lib.FwdArgs(q_stride=st, k_stride=st, v_stride=st, o_stride=st, lse_stride=_lib._i64x3(0, 0, 0), **base)
+    assert 0 < _lib.fwd_workspace_size(dense()) <= most
+    for kw in (dict(batch=64), dict(seqlen_q=0), dict(seqlen_k=512), dict(dtype=_lib.DTYPE_FP32)):
+        assert _lib.fwd_workspace_size(dense(**kw)) == 0, kw
+    with pytest.raises(RuntimeError, match="non-NULL"):
+        _lib.fwd_split(dense(), None, 1 << 30, 0)
+    # the Python wrappers ask only where the answer can be positive
+    from lightserve_amd.kernels.flash_attention import SPLIT_MAX_TILES, SPLIT_MIN_KEYS
+    for b in (1, 2, 5, 16):
+        for h in (1, 3, 16):
+            for n in (64, 300, SPLIT_MIN_KEYS - 1, 700, 2000, 5000):
+                tiles = b * h * ((n + 127) // 128)
+                if tiles > SPLIT_MAX_TILES or n < SPLIT_MIN_KEYS:
+                    assert _lib.fwd_workspace_size(dense(batch=b, heads_q=h, heads_kv=h, seqlen_q=n, seqlen_k=n)) == 0
