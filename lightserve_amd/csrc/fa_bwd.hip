@@ -62,9 +62,30 @@ __global__ __launch_bounds__(256, 2) void fa_bwd_dq_kernel(const BwdParams p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (SGPR)
   const int l32 = lane & 31, hh = lane >> 5;
-  int bh, qt;
-  map_tile(p.num_tiles, gridDim.x, p.heads_per_group, bh, qt, CAUSAL);
-  const int b = bh / p.H, h = bh - b * p.H;
+  int b, h, qt;
+  if (VARLEN && p.B <= 64) {
+    // Sequences differ in length: (sequence, query tile) items longest first,
+    // workgroup L taking rank L / H and head slot L % H (ranked_head).
+    const int rank = blockIdx.x / p.H;
+    h = ranked_head(blockIdx.x - rank * p.H, p.H);
+    int tq = 0, nk = 0, off = 0;
+    if (lane < p.B) {
+      const int nq = min(max(p.cu_q[lane + 1] - p.cu_q[lane], 0), p.Nq);
+      nk = min(max(p.cu_k[lane + 1] - p.cu_k[lane], 0), p.Nk);
+      tq = (nq + BM - 1) / BM;
+      off = nk - nq;
+    }
+    int d;
+    b = ranked_item(p.B, rank, lane, tq, (nk + 63) >> 6, [&](int x) { return tiles_above<CAUSAL, BM>(x, tq, nk, off); },
+                    d);
+    if (b < 0) return;  // uniform, before any barrier
+    qt = __builtin_amdgcn_readlane(tq, b) - 1 - d;
+  } else {
+    int bh;
+    map_tile(p.num_tiles, gridDim.x, p.heads_per_group, bh, qt, CAUSAL);
+    b = bh / p.H;
+    h = bh - b * p.H;
+  }
   int nq = p.Nq, nk = p.Nk;
   int64_t rq0 = 0, rk0 = 0;  // varlen: the sequence's first query / key row
   if (VARLEN) {  // lengths clamped to the longest the grid and the workspace were sized for
@@ -389,10 +410,37 @@ __global__ __launch_bounds__(256, 1) void fa_bwd_dkdv_kernel(const BwdParams p) 
   // ring one head after another, into the same dK/dV sums.
   static_assert(!((GQA || VARLEN) && DS), "the stored-dS path has no GQA or varlen");
   const int G = GQA ? p.G : 1, Hkv = p.H / G;
-  int bh, kt;
-  map_tile(p.num_tiles, gridDim.x, p.heads_per_group, bh, kt, false);  // low key tiles see the most queries
-  bh += p.bh0;
-  const int b = bh / Hkv, hk = bh - b * Hkv, h0 = hk * G;
+  int bh, kt, b, hk;
+  if (VARLEN && p.B <= 64) {
+    // Longest first, as in fa_bwd_dq_kernel: key tile kt of a sequence takes
+    // the query tiles from max(0, 128 kt - off) / 64 on, so more than x of
+    // them iff 128 kt < 64 (tiles - x) + off.
+    const int rank = blockIdx.x / Hkv;
+    hk = ranked_head(blockIdx.x - rank * Hkv, Hkv);
+    int tk = 0, tiles = 0, off = 0;
+    if (lane < p.B) {
+      const int nq = min(max(p.cu_q[lane + 1] - p.cu_q[lane], 0), p.Nq);
+      const int nk = min(max(p.cu_k[lane + 1] - p.cu_k[lane], 0), p.Nk);
+      tk = (nk + BNK - 1) / BNK;
+      tiles = (nq + BMQ - 1) / BMQ;
+      off = nk - nq;
+    }
+    b = ranked_item(p.B, rank, lane, tk, tiles, [&](int x) {
+      if (x < 0) return tk;
+      if (x >= tiles) return 0;
+      if (!CAUSAL) return tk;
+      const int y = BMQ * (tiles - x) + off;
+      return y <= 0 ? 0 : min(tk, (y + BNK - 1) / BNK);
+    }, kt);
+    if (b < 0) return;  // uniform, before any barrier
+    bh = b * Hkv + hk;
+  } else {
+    map_tile(p.num_tiles, gridDim.x, p.heads_per_group, bh, kt, false);  // low key tiles see the most queries
+    bh += p.bh0;
+    b = bh / Hkv;
+    hk = bh - b * Hkv;
+  }
+  const int h0 = hk * G;
   int nq = p.Nq, nk = p.Nk;
   int64_t rq0 = 0, rk0 = 0;  // varlen: the sequence's first query / key row
   if (VARLEN) {  // lengths clamped to the longest the grid and the workspace were sized for

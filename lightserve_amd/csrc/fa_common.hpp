@@ -341,6 +341,73 @@ __device__ __forceinline__ void map_tile(int num_tiles, int total, int heads_per
   tile = heavy_last_index ? (num_tiles - 1 - level) : level;
 }
 
+// Head of slot u (0 .. heads-1) of a launch whose workgroups are numbered
+// [rank][slot]: workgroups go to the XCDs round-robin, so with a multiple of 8
+// heads XCD x's slots x, x+8, ... map to adjacent heads (with GQA, query
+// heads that share K/V).
+__device__ __forceinline__ int ranked_head(int u, int heads) {
+  return (heads & 7) == 0 ? (u & 7) * (heads >> 3) + (u >> 3) : u;
+}
+
+// Sum over lanes 0 .. width-1 (a power of two; v is 0 in the lanes past it),
+// wave-uniform.
+__device__ __forceinline__ int wave_sum_i(int v, int width) {
+  for (int o = width >> 1; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  return __builtin_amdgcn_readfirstlane(v);
+}
+
+// Longest-first order of a varlen launch's items (a sequence's tiles), so that
+// the longest workgroups start first and the short ones fill the tail: the
+// sequence of the item of the given rank (rank 0 is the longest; ties go by
+// sequence), or -1 past the last item, and the item's position d among its
+// sequence's items in descending length. Lane i holds sequence i (B <= 64):
+// its number of items, the most steps one of them takes, and above(x), how
+// many of them take more than x steps (x = -1: all). The length at the rank
+// is found by binary search, the item among those of that length by a prefix
+// sum over the sequences. The sums run over the lanes that hold a sequence
+// only: each shuffle costs an LDS round trip in a chain of about 10 log2(B)
+// before the workgroup's first load. Wave-uniform results.
+template <typename F>
+__device__ __forceinline__ int ranked_item(int B, int rank, int lane, int items, int steps, F above, int& d) {
+  const int width = B > 1 ? 1 << (32 - __builtin_clz(B - 1)) : 1;
+  d = 0;
+  if (rank >= wave_sum_i(items, width)) return -1;
+  for (int o = width >> 1; o > 0; o >>= 1) steps = max(steps, __shfl_xor(steps, o));
+  int lo = 0, hi = __builtin_amdgcn_readfirstlane(steps);  // no item exceeds hi
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (wave_sum_i(above(mid), width) <= rank) hi = mid;
+    else lo = mid + 1;
+  }
+  // rank lies among the items of exactly lo steps: positions
+  // [above(lo), above(lo - 1)) of each sequence.
+  const int first = above(lo), c = above(lo - 1) - first;
+  const int k = rank - wave_sum_i(first, width);
+  int inc = c;
+  for (int o = 1; o < width; o <<= 1) {
+    const int t = __shfl_up(inc, o);
+    if (lane >= o) inc += t;
+  }
+  const int pre = inc - c;
+  const unsigned long long hit = __ballot(c > 0 && k >= pre && k < pre + c);
+  const int src = __builtin_amdgcn_readfirstlane((int)__builtin_ctzll(hit));
+  d = __builtin_amdgcn_readlane(first + k - pre, src);
+  return src;
+}
+
+// Number of a sequence's query tiles (tq of them, BM rows each) whose key
+// tile count (64 keys each) exceeds x; the tiles counted are always the last
+// ones, as causal work grows with the tile index. x = -1 counts every tile.
+template <bool CAUSAL, int BM>
+__device__ __forceinline__ int tiles_above(int x, int tq, int nk, int off) {
+  if (x < 0) return tq;
+  if (tq == 0 || nk <= 64 * x) return 0;  // the last tile sees all nk keys
+  if (!CAUSAL) return tq;
+  // tile t < tq-1 sees off + BM(t+1) keys: more than 64x iff t >= (64x-off)/BM
+  const long long y = 64LL * x - off;
+  return y < 0 ? tq : 1 + max(0, tq - 1 - (int)(y / BM));
+}
+
 // Heads per map_tile group: as many as keep a group's streamed operands
 // (bytes_per_head each: K and V for the query-stationary kernels, Q and dO
 // for the key-stationary one) within ~8 MiB, i.e. two XCD L2s, at most 16.

@@ -54,36 +54,8 @@ constexpr float kLn2 = 0.6931471805599453f;
 template <typename T> constexpr float kMaxLog2P = 64.0f;
 template <> constexpr float kMaxLog2P<_Float16> = 15.0f;
 
-// Sum over lanes 0 .. width-1 (a power of two; v is 0 in the lanes past it),
-// wave-uniform.
-__device__ __forceinline__ int wave_sum_i(int v, int width) {
-  for (int o = width >> 1; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return __builtin_amdgcn_readfirstlane(v);
-}
-
-// Number of a sequence's query tiles (tq of them, BM rows each) whose key
-// tile count (64 keys each) exceeds x; the tiles counted are always the last
-// ones, as causal work grows with the tile index. x = -1 counts every tile.
-template <bool CAUSAL, int BM>
-__device__ __forceinline__ int tiles_above(int x, int tq, int nk, int off) {
-  if (x < 0) return tq;
-  if (tq == 0 || nk <= 64 * x) return 0;  // the last tile sees all nk keys
-  if (!CAUSAL) return tq;
-  // tile t < tq-1 sees off + BM(t+1) keys: more than 64x iff t >= (64x-off)/BM
-  const long long y = 64LL * x - off;
-  return y < 0 ? tq : 1 + max(0, tq - 1 - (int)(y / BM));
-}
-
-// Longest-first order of a varlen launch's (sequence, query tile) items, so
-// that each XCD starts its longest workgroups first and the short ones fill
-// the tail: returns the item of the given rank (rank 0 has the most key
-// tiles; ties go by sequence, then tile), or b = -1 past the last item.
-// Lane i holds sequence i (B <= 64). The key tile count of the item at the
-// rank is found by binary search on the number of items above a count, then
-// the item among those of that count by a prefix sum over the sequences.
-// The sums run over the lanes that hold a sequence only: each shuffle costs an
-// LDS round trip in a chain of about 10 log2(B), before the first load.
-// Wave-uniform result.
+// Longest-first order of a varlen launch's (sequence, query tile) items
+// (ranked_item): the item of the given rank, b = -1 past the last item.
 template <bool CAUSAL, bool PAGED, int BM>
 __device__ __forceinline__ void varlen_item_at(const FwdParams& p, int rank, int lane, int& b_out, int& qt_out) {
   int tq = 0, nk = 0, off = 0;
@@ -94,34 +66,10 @@ __device__ __forceinline__ void varlen_item_at(const FwdParams& p, int rank, int
     tq = nq > 0 ? (nq + BM - 1) / BM : 0;
     off = nk - nq;
   }
-  const int width = p.B > 1 ? 1 << (32 - __builtin_clz(p.B - 1)) : 1;
-  b_out = -1;
-  qt_out = 0;
-  if (rank >= wave_sum_i(tq, width)) return;
-  int kmax = nk > 0 ? (nk + 63) >> 6 : 0;
-  for (int o = width >> 1; o > 0; o >>= 1) kmax = max(kmax, __shfl_xor(kmax, o));
-  int lo = 0, hi = __builtin_amdgcn_readfirstlane(kmax);  // no item exceeds hi
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (wave_sum_i(tiles_above<CAUSAL, BM>(mid, tq, nk, off), width) <= rank) hi = mid;
-    else lo = mid + 1;
-  }
-  // rank lies among the items of exactly lo key tiles: tiles
-  // [tq - above(lo-1), tq - above(lo)) of each sequence.
-  const int a_hi = tiles_above<CAUSAL, BM>(lo - 1, tq, nk, off);
-  const int a_lo = tiles_above<CAUSAL, BM>(lo, tq, nk, off);
-  const int c = a_hi - a_lo;
-  const int k = rank - wave_sum_i(a_lo, width);
-  int inc = c;
-  for (int o = 1; o < width; o <<= 1) {
-    const int t = __shfl_up(inc, o);
-    if (lane >= o) inc += t;
-  }
-  const int pre = inc - c;
-  const unsigned long long hit = __ballot(c > 0 && k >= pre && k < pre + c);
-  const int src = __builtin_amdgcn_readfirstlane((int)__builtin_ctzll(hit));
-  b_out = src;
-  qt_out = __builtin_amdgcn_readfirstlane(__shfl(tq - a_hi + k - pre, src));
+  int d;
+  b_out = ranked_item(p.B, rank, lane, tq, nk > 0 ? (nk + 63) >> 6 : 0,
+                      [&](int x) { return tiles_above<CAUSAL, BM>(x, tq, nk, off); }, d);
+  qt_out = b_out < 0 ? 0 : __builtin_amdgcn_readlane(tq, b_out) - 1 - d;  // the last tile is the longest
 }
 
 // The (batch, head, query tile) of workgroup blockIdx.x; false past the last.
@@ -129,13 +77,10 @@ template <bool CAUSAL, bool VARLEN, bool PAGED, int BM>
 __device__ __forceinline__ bool item_at(const FwdParams& p, int lane, int& b, int& h, int& qt) {
   if (VARLEN && p.B <= 64) {
     // Varlen sequences differ in length: workgroup L takes the item of rank
-    // L / Hq in longest-first order, for head slot L % Hq. Workgroups go to
-    // the XCDs round-robin, so with Hq a multiple of 8 XCD x gets slots
-    // x, x+8, ..., mapped to the adjacent heads x*Hq/8 .. (with GQA, query
-    // heads that share K/V), every rank in order.
+    // L / Hq in longest-first order, for head slot L % Hq (ranked_head).
     const int L = blockIdx.x;
     const int rank = L / p.Hq, u = L - rank * p.Hq;
-    h = (p.Hq & 7) == 0 ? (u & 7) * (p.Hq >> 3) + (u >> 3) : u;
+    h = ranked_head(u, p.Hq);
     varlen_item_at<CAUSAL, PAGED, BM>(p, rank, lane, b, qt);
     return b >= 0;
   } else {

@@ -280,3 +280,42 @@ def test_varlen_backward_validation(gpu):
     with torch.no_grad():  # no gradient wanted: the fp32 forward runs
         o = flash_attention_varlen(qf, kf, kf, cu_q, cu_k, 20, 30)
     assert o.shape == qf.shape
+
+
+@pytest.mark.parametrize("heads", [(8, 8), (6, 2), (16, 8)])
+@pytest.mark.parametrize("B", [1, 2, 5, 64, 65])
+@pytest.mark.parametrize("causal", [True, False])
+def test_varlen_order_does_not_change_results(B, heads, causal):
+    """Batches of up to 64 sequences run their tiles longest first, longer ones
+    in launch order: forward and gradients of a batch (empty sequences, empty
+    key or query sides, more keys than queries and fewer) equal the same
+    sequences run one at a time, bit for bit."""
+    import random
+    from lightserve_amd.kernels.flash_attention_varlen import flash_attention_varlen_backward
+    print(f"case varlen order B={B} heads={heads} causal={causal}", flush=True)
+    rng = random.Random(B)
+    lq = [rng.choice([0, 1, 63, 64, 129, 200, 300]) for _ in range(B)]
+    lk = [rng.choice([0, 1, 64, 65, 128, 257, n, n]) for n in lq]
+    if B == 1:
+        lq, lk = [300], [257]
+    g = torch.Generator(device="cuda").manual_seed(B)
+    Hq, Hkv = heads
+    q, do = (torch.randn(sum(lq), Hq, 64, device="cuda", generator=g).to(torch.bfloat16) for _ in range(2))
+    k, v = (torch.randn(sum(lk), Hkv, 64, device="cuda", generator=g).to(torch.bfloat16) for _ in range(2))
+
+    def run(q, k, v, do, lq, lk):
+        cu = [torch.tensor([0] + n, device="cuda").cumsum(0).to(torch.int32) for n in (lq, lk)]
+        o, lse = flash_attention_varlen_forward(q, k, v, *cu, max(lq), max(lk), causal=causal)
+        return (o, *flash_attention_varlen_backward(do, q, k, v, o, lse, *cu, max(lq), max(lk), causal=causal))
+    got = run(q, k, v, do, lq, lk)
+    parts, a, c = [], 0, 0
+    for nq, nk in zip(lq, lk):
+        s, t = slice(a, a + nq), slice(c, c + nk)
+        if nq == 0 or nk == 0:  # no query sees a key
+            parts.append(tuple(torch.zeros_like(x) for x in (q[s], q[s], k[t], v[t])))
+        else:
+            parts.append(run(q[s], k[t], v[t], do[s], [nq], [nk]))
+        a, c = a + nq, c + nk
+    for i, t in enumerate(got):
+        want = torch.cat([p[i] for p in parts])
+        assert torch.equal(t, want), i
