@@ -435,6 +435,9 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const void* base, in
 __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t rs, LDS_AS void* dst, int voff) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, dst, 16, voff, 0, 0, 0);
 }
+__device__ __forceinline__ void dma4(__amdgpu_buffer_rsrc_t rs, LDS_AS void* dst, int voff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, dst, 4, voff, 0, 0, 0);
+}
 __device__ __forceinline__ void store16(u32x4 v, __amdgpu_buffer_rsrc_t rs, int voff) {
   __builtin_amdgcn_raw_buffer_store_b128(v, rs, voff, 0, 0);
 }
