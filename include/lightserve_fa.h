@@ -551,6 +551,13 @@ int lsfa_gemv_group_check(const lsfa_gemv_group_args* args);
 int lsfa_gemv_group_workspace_size(const lsfa_gemv_group_args* args, uint64_t* bytes);
 int lsfa_gemv_group(const lsfa_gemv_group_args* args, void* stream);
 
+/* The same product above 32 rows (no gate, no norm; every width a multiple of
+ * 128, k % 8 == 0, x rows 16-byte aligned) for launches of at most 256 tiles
+ * of 64 rows x 128 columns, where a general GEMM's tiles leave CUs idle. */
+int lsfa_gemm_group_check(const lsfa_gemv_group_args* args);
+int lsfa_gemm_group_workspace_size(const lsfa_gemv_group_args* args, uint64_t* bytes);
+int lsfa_gemm_group(const lsfa_gemv_group_args* args, void* stream);
+
 /* Host-only validation of greedy-token arguments; never touches the GPU. */
 int lsfa_greedy_check(const lsfa_greedy_args* args);
 

@@ -32,6 +32,7 @@ EXPORTED_SYMBOLS = ("lsfa_abi_version", "lsfa_last_error", "lsfa_fwd_check", "ls
                     "lsfa_prefill_paged_workspace_size", "lsfa_prefill_paged_split",
                     "lsfa_gemv_check", "lsfa_gemv_workspace_size", "lsfa_gemv",
                     "lsfa_gemv_group_check", "lsfa_gemv_group_workspace_size", "lsfa_gemv_group",
+                    "lsfa_gemm_group_check", "lsfa_gemm_group_workspace_size", "lsfa_gemm_group",
                     "lsfa_greedy_check", "lsfa_greedy")
 
 _i64x4 = ctypes.c_int64 * 4
@@ -200,6 +201,7 @@ def load():
                              ("lsfa_decode_check", DecodeArgs), ("lsfa_rope_check", RopeArgs),
                              ("lsfa_rmsnorm_check", RmsNormArgs), ("lsfa_prefill_paged_check", PrefillPagedArgs),
                              ("lsfa_gemv_check", GemvArgs), ("lsfa_gemv_group_check", GemvGroupArgs),
+                             ("lsfa_gemm_group_check", GemvGroupArgs),
                              ("lsfa_greedy_check", GreedyArgs)):
             fn = getattr(lib, name)
             fn.restype = ctypes.c_int
@@ -208,7 +210,8 @@ def load():
                              ("lsfa_decode", DecodeArgs),
                              ("lsfa_rope", RopeArgs), ("lsfa_rmsnorm", RmsNormArgs),
                              ("lsfa_prefill_paged", PrefillPagedArgs), ("lsfa_gemv", GemvArgs),
-                             ("lsfa_gemv_group", GemvGroupArgs), ("lsfa_greedy", GreedyArgs)):
+                             ("lsfa_gemv_group", GemvGroupArgs), ("lsfa_gemm_group", GemvGroupArgs),
+                             ("lsfa_greedy", GreedyArgs)):
             fn = getattr(lib, name)
             fn.restype = ctypes.c_int
             fn.argtypes = [ctypes.POINTER(struct), ctypes.c_void_p]
@@ -219,8 +222,9 @@ def load():
             split.argtypes = [ctypes.POINTER(struct), ctypes.c_void_p, ctypes.c_uint64, ctypes.c_void_p]
         lib.lsfa_bwd_workspace_size.restype = ctypes.c_int
         lib.lsfa_bwd_workspace_size.argtypes = [ctypes.POINTER(BwdArgs), ctypes.POINTER(ctypes.c_uint64)]
-        lib.lsfa_gemv_group_workspace_size.restype = ctypes.c_int
-        lib.lsfa_gemv_group_workspace_size.argtypes = [ctypes.POINTER(GemvGroupArgs), ctypes.POINTER(ctypes.c_uint64)]
+        for size in (lib.lsfa_gemv_group_workspace_size, lib.lsfa_gemm_group_workspace_size):
+            size.restype = ctypes.c_int
+            size.argtypes = [ctypes.POINTER(GemvGroupArgs), ctypes.POINTER(ctypes.c_uint64)]
         lib.lsfa_gemv_workspace_size.restype = ctypes.c_int
         lib.lsfa_gemv_workspace_size.argtypes = [ctypes.POINTER(GemvArgs), ctypes.POINTER(ctypes.c_uint64)]
         lib.lsfa_decode_workspace_size.restype = ctypes.c_int
@@ -330,6 +334,23 @@ def gemv_group_workspace_size(args):
 
 def gemv_group(args, stream):
     _raise_on(load().lsfa_gemv_group(ctypes.byref(args), ctypes.c_void_p(stream)), "lsfa_gemv_group")
+
+
+def gemm_group_check(args):
+    """Host-only validation (no GPU access); returns (status, message)."""
+    rc = load().lsfa_gemm_group_check(ctypes.byref(args))
+    return rc, load().lsfa_last_error().decode(errors="replace")
+
+
+def gemm_group_workspace_size(args):
+    n = ctypes.c_uint64(0)
+    _raise_on(load().lsfa_gemm_group_workspace_size(ctypes.byref(args), ctypes.byref(n)),
+              "lsfa_gemm_group_workspace_size")
+    return n.value
+
+
+def gemm_group(args, stream):
+    _raise_on(load().lsfa_gemm_group(ctypes.byref(args), ctypes.c_void_p(stream)), "lsfa_gemm_group")
 
 
 def greedy_check(args):

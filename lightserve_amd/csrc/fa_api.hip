@@ -688,12 +688,12 @@ GemvSplit gemv_split_mfma(long long M, long long K, long long N) {
   M = std::max(M, 0LL); K = std::max(K, 0LL); N = std::max(N, 0LL);
   const long long blocks = std::max(1LL, N / 128);
   const long long most = std::max(1LL, (K + 255) / 256);
-  const long long want = std::max(1LL, std::min(256 / blocks, most));
+  const long long want = std::max(1LL, std::min(256 / (blocks * std::max(1LL, (M + 63) / 64)), most));
   g.kc = (int)std::max(32LL, ((K + want - 1) / want + 31) / 32 * 32);
   g.splits = (int)std::max(1LL, (K + g.kc - 1) / g.kc);
   if (g.splits > 1) {
     g.counter_bytes = LSFA_GEMV_COUNTER_BYTES;
-    g.bytes = g.counter_bytes + align256((uint64_t)std::min(512 / blocks, most) * M * N * 4);
+    g.bytes = g.counter_bytes + align256((uint64_t)std::max(want, std::min(512 / blocks, M <= 32 ? most : 1)) * M * N * 4);
   }
   return g;
 }
@@ -810,13 +810,7 @@ int lsfa_gemv_group_workspace_size(const lsfa_gemv_group_args* a, uint64_t* byte
   return ok();
 }
 
-int lsfa_gemv_group(const lsfa_gemv_group_args* a, void* stream) {
-  int rc = lsfa_gemv_group_check(a);
-  if (rc) return rc;
-  const long long N = gemv_total_n(a);
-  if (a->m == 0 || N == 0) return ok();
-  const bool mfma = gemv_uses_mfma(a);
-  const GemvSplit g = mfma ? gemv_split_mfma(a->m, a->k, N) : gemv_split(a->m, a->k, N);
+static int run_gemv_group(const lsfa_gemv_group_args* a, bool mfma, const GemvSplit& g, long long N, void* stream) {
   lsfa::GemvParams p;
   memset(&p, 0, sizeof(p));
   p.x = a->x;
@@ -850,6 +844,50 @@ int lsfa_gemv_group(const lsfa_gemv_group_args* a, void* stream) {
                       : lsfa::gemv(p, a->dtype == LSFA_DTYPE_BF16, reinterpret_cast<hipStream_t>(stream));
   if (e != hipSuccess) return fail(LSFA_ERR_LAUNCH, "gemv launch failed: %s", hipGetErrorString(e));
   return ok();
+}
+
+int lsfa_gemv_group(const lsfa_gemv_group_args* a, void* stream) {
+  int rc = lsfa_gemv_group_check(a);
+  if (rc) return rc;
+  const long long N = gemv_total_n(a);
+  if (a->m == 0 || N == 0) return ok();
+  const bool mfma = gemv_uses_mfma(a);
+  return run_gemv_group(a, mfma, mfma ? gemv_split_mfma(a->m, a->k, N) : gemv_split(a->m, a->k, N), N, stream);
+}
+
+// Above 32 rows: the MFMA kernel over row blocks, for launches of at most one
+// workgroup per CU (column blocks x 64-row blocks <= 256).
+int lsfa_gemm_group_check(const lsfa_gemv_group_args* a) {
+  if (a == nullptr) return fail(LSFA_ERR_INVALID, "args is NULL");
+  if (a->m <= 32 || a->x_gate || a->norm_weight)
+    return fail(LSFA_ERR_UNSUPPORTED, "gemm takes more than 32 rows and no gate or norm (m=%d); use lsfa_gemv_group", a->m);
+  lsfa_gemv_group_args few = *a;
+  few.m = 32;
+  few.workspace = reinterpret_cast<void*>(uintptr_t{256});  // (checked below, for m rows)
+  few.workspace_bytes = ~uint64_t{0};
+  int rc = lsfa_gemv_group_check(&few);
+  if (rc) return rc;
+  const long long N = gemv_total_n(a);
+  if (N == 0) return ok();
+  if (N / 128 * (((long long)a->m + 63) / 64) > 256)
+    return fail(LSFA_ERR_UNSUPPORTED, "gemm takes at most 256 tiles of 64 x 128 (m=%d n=%lld)", a->m, N);
+  if (a->x_stride > (1 << 23)) return fail(LSFA_ERR_UNSUPPORTED, "x_stride must be at most 2^23");
+  return check_split_workspace("lsfa_gemm_group_workspace_size", a->workspace, a->workspace_bytes,
+                               gemv_split_mfma(a->m, a->k, N).bytes);
+}
+
+int lsfa_gemm_group_workspace_size(const lsfa_gemv_group_args* a, uint64_t* bytes) {
+  if (a == nullptr || bytes == nullptr) return fail(LSFA_ERR_INVALID, "args or bytes is NULL");
+  *bytes = gemv_split_mfma(a->m, a->k, gemv_total_n(a)).bytes;
+  return ok();
+}
+
+int lsfa_gemm_group(const lsfa_gemv_group_args* a, void* stream) {
+  const int rc = lsfa_gemm_group_check(a);
+  if (rc) return rc;
+  const long long N = gemv_total_n(a);
+  if (N == 0) return ok();
+  return run_gemv_group(a, true, gemv_split_mfma(a->m, a->k, N), N, stream);
 }
 
 int lsfa_gemv_check(const lsfa_gemv_args* a) {

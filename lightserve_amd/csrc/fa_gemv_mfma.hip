@@ -1,4 +1,4 @@
-// Skinny GEMM on MFMA for 3..32 rows: y[M, N] = x[M, K] @ W[K, N] (W in the
+// Skinny GEMM on MFMA, 3 rows and more: y[M, N] = x[M, K] @ W[K, N] (W in the
 // model's [in, out] row-major layout, bf16/fp16, fp32 accumulate, one rounding),
 // for the decode steps of a batch, where the VALU kernel (fa_gemv.hip) spends
 // more time on its products than on the weight bytes.
@@ -32,12 +32,25 @@
 // and at 32 rows 37.1 -> 16.4, 31.3 -> 13.7, 99.4 -> 46.2, 85.5 -> 27.2, 406 -> 177.
 // Three or four steps in flight, or eight waves, change nothing (+-3%): what is
 // left on the small products is the launch's own latency and the reduction.
+//
+// Above 32 rows (grid z, blocks of 64 rows, eight waves) the same kernel serves
+// products whose tiles fit the GPU once, where a library GEMM's larger tiles
+// leave most CUs idle: us against hipBLASLt at 64 / 128 / 256 / 512 rows,
+//   4096 -> 4096+1024+1024: 22.5 / 28 / 37.5 / - against 82 / 78 / 64 (three launches)
+//   4096 -> 4096: 18.9 / 20.5 / 26.0 / 35.4 against 28.2 / 39.6 / 25.7 / 39.4
+//   14336 -> 4096: 36.5 / 46.5 / 68.0 / 110 against 103 / 124 / 98.5 / 124
+//   2048 -> 2048: 15.7 / 15.7 / 14.2 / 16.4 against 15.6 / 12.6 / 13.0 / 14.1: left to
+//   the library, as is what has more tiles than CUs (4096 -> 2 x 14336 at 128 rows 92
+//   against 86, at 512 288 against 148).
+// There it is bound by its loads: every wave reads x rows of its own steps, in
+// 64-byte pieces, and W passes L1 once per row block (with both from L1 the same
+// loop runs at 950 TFLOP/s). Four waves of twice the steps: 4% slower; 128-row
+// blocks (512 VGPRs): slower everywhere.
 #include "fa_common.hpp"
 
 namespace lsfa {
 
 constexpr int kMfmaCols = 128;   // columns per workgroup
-constexpr int kMfmaWaves = 4;    // waves per workgroup
 constexpr int kMfmaStep = 32;    // rows of W per step
 constexpr int kMfmaDepth = 2;    // steps of a wave in flight
 constexpr int kMfmaLd = kMfmaCols + 4;  // row stride of the wave sums in LDS (floats)
@@ -49,15 +62,19 @@ __device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
 __device__ __forceinline__ f32x4 mfma16(f16x8 a, f16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
-// 16-byte read-once load (non-temporal); lanes whose offset is out of range read zero.
+// 16-byte loads, the first non-temporal; lanes whose offset is out of range read zero.
 __device__ __forceinline__ u32x4 load16_nt(__amdgpu_buffer_rsrc_t rs, int voff, int soff) {
   return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, voff, soff, 2));
 }
+__device__ __forceinline__ u32x4 load16(__amdgpu_buffer_rsrc_t rs, int voff, int soff) {
+  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, voff, soff, 0));
+}
 
 // MT: blocks of 16 rows (M <= 16 MT). GATE: x stands for silu(xg) * x.
-template <typename T, int MT, bool GATE>
-__global__ __launch_bounds__(64 * kMfmaWaves, 2) void fa_gemv_mfma_kernel(const GemvParams p) {
-  constexpr int NW = kMfmaWaves, DEPTH = kMfmaDepth;
+template <typename T, int MT, int NW, bool GATE>
+__global__ __launch_bounds__(64 * NW, 2) void fa_gemv_mfma_kernel(const GemvParams p) {
+  constexpr int DEPTH = kMfmaDepth;
+  constexpr bool WNT = MT <= 2;  // one row block: W is read once
   using X8 = typename VecT<T>::x8;
   extern __shared__ __attribute__((aligned(16))) float wave_sums[];  // [NW / 2][16 MT][kMfmaLd]
   __shared__ int last_arrival;
@@ -65,6 +82,8 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void fa_gemv_mfma_kernel(const 
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, kg = lane >> 4;
   const int split = blockIdx.y;
+  const int m0 = blockIdx.z * 16 * MT;  // first row of the row block
+  const int rows = min(p.M - m0, 16 * MT);
   const int k_begin = split * p.kc;
   const int k_len = max(0, min(p.K, k_begin + p.kc) - k_begin);
 
@@ -79,14 +98,15 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void fa_gemv_mfma_kernel(const 
   const int n_local = n_blk - col_off;
 
   // Rows of x past M repeat the last one: their sums are never stored.
-  const T* xr[MT];
-  const T* gr[MT];
+  int xo[MT], go[GATE ? MT : 1];
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
-    const int m = min(16 * t + c, p.M - 1);
-    xr[t] = (const T*)p.x + (int64_t)m * p.sx + k_begin;
-    gr[t] = GATE ? (const T*)p.xg + (int64_t)m * p.sxg + k_begin : nullptr;
+    const int m = min(16 * t + c, rows - 1);
+    xo[t] = (int)(m * p.sx * 2) + 16 * kg;
+    if (GATE) go[t] = (int)(m * p.sxg * 2) + 16 * kg;
   }
+  const T* xk = (const T*)p.x + (int64_t)m0 * p.sx + k_begin;
+  const T* gk = GATE ? (const T*)p.xg + (int64_t)m0 * p.sxg + k_begin : nullptr;
   const T* wk = w + (int64_t)k_begin * sw + n_local;
   const int row_bytes = (int)(sw * 2);
   const int lane_off = 8 * kg * row_bytes + 16 * c;
@@ -99,20 +119,23 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void fa_gemv_mfma_kernel(const 
   // The loads of one step, always the same number of them, so that the wait
   // before a step's use counts the next step's loads as still in flight. K is
   // a multiple of 8, so a lane's eight rows are inside the K-range or past it
-  // together; past it W reads as zero (offset out of range: no memory access)
-  // and x, read at its row's start, is masked on use.
+  // together; past it W and x read as zero (offset out of range: no memory
+  // access).
   auto load = [&](int step, Step& s) {
-    const int k = step * kMfmaStep;
-    const bool in = k + 8 * kg < k_len;
-    const __amdgpu_buffer_rsrc_t rs = tile_rsrc(wk + (int64_t)min(k, k_len) * sw, 0x7fffffff);
-    const int voff = in ? lane_off : (int)0x80000000;
+    const int k = step * kMfmaStep, kc = min(k, k_len);
+    // (or-ed into the offsets: a select of offsets turns into branches around the loads)
+    const int past = k + 8 * kg < k_len ? 0 : (int)0x80000000;
+    const __amdgpu_buffer_rsrc_t rs = tile_rsrc(wk + (int64_t)kc * sw, 0x7fffffff);
+    const int voff = lane_off | past;
 #pragma unroll
-    for (int r = 0; r < 8; ++r) s.w[r] = load16_nt(rs, voff, r * row_bytes);
-    const int kx = in ? k + 8 * kg : 0;
+    for (int r = 0; r < 8; ++r) s.w[r] = WNT ? load16_nt(rs, voff, r * row_bytes) : load16(rs, voff, r * row_bytes);
+    const __amdgpu_buffer_rsrc_t xs = tile_rsrc(xk + kc, 0x7fffffff);
 #pragma unroll
-    for (int t = 0; t < MT; ++t) {
-      s.x[t] = ldg16(xr[t] + kx);
-      if (GATE) s.g[t] = ldg16(gr[t] + kx);
+    for (int t = 0; t < MT; ++t) s.x[t] = load16(xs, xo[t] | past, 0);
+    if constexpr (GATE) {
+      const __amdgpu_buffer_rsrc_t gs = tile_rsrc(gk + kc, 0x7fffffff);
+#pragma unroll
+      for (int t = 0; t < MT; ++t) s.g[t] = load16(gs, go[t] | past, 0);
     }
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -121,8 +144,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void fa_gemv_mfma_kernel(const 
   for (int t = 0; t < MT; ++t)
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto use = [&](int step, const Step& s) {
-    const bool in = step * kMfmaStep + 8 * kg < k_len;
+  auto use = [&](const Step& s) {
     X8 xb[MT];
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
@@ -140,8 +162,6 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void fa_gemv_mfma_kernel(const 
         }
         raw = __builtin_bit_cast(u32x4, o);
       }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) raw[e] = in ? raw[e] : 0u;
       xb[t] = __builtin_bit_cast(X8, raw);
     }
 #pragma unroll
@@ -169,7 +189,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void fa_gemv_mfma_kernel(const 
     for (int st = wave; st < steps; st += DEPTH * NW) {
 #pragma unroll
       for (int d = 0; d < DEPTH; ++d) {
-        use(st + d * NW, s[d]);
+        use(s[d]);
         load(st + (DEPTH + d) * NW, s[d]);
       }
     }
@@ -203,11 +223,11 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void fa_gemv_mfma_kernel(const 
   // The block's sums in pairs of columns, row by row: thread tid takes pairs
   // tid, tid + 64 NW, ...
   constexpr int IT = 16 * MT * (kMfmaCols / 2) / (64 * NW);
-  const int pairs = p.M * (kMfmaCols / 2);
+  const int pairs = rows * (kMfmaCols / 2);
   const int64_t sstride = (int64_t)p.N * p.M / 2;
-  uint64_t* base = (uint64_t*)(p.partial + (int64_t)n_blk * p.M);
+  uint64_t* base = (uint64_t*)(p.partial + (int64_t)n_blk * p.M + (int64_t)m0 * kMfmaCols);
   auto put = [&](int pair, float s0, float s1) {
-    T* dst = y + (int64_t)(pair / (kMfmaCols / 2)) * sy + n_local + 2 * (pair % (kMfmaCols / 2));
+    T* dst = y + (int64_t)(m0 + pair / (kMfmaCols / 2)) * sy + n_local + 2 * (pair % (kMfmaCols / 2));
     dst[0] = (T)s0;
     dst[1] = (T)s1;
   };
@@ -246,7 +266,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void fa_gemv_mfma_kernel(const 
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the partials have reached device scope
   __syncthreads();
   if (tid == 0) {
-    int* ctr = p.counters + blockIdx.x * kMfmaCounterSlots;
+    int* ctr = p.counters + (blockIdx.z * gridDim.x + blockIdx.x) * kMfmaCounterSlots;
     // One counter for up to eight splits (the arrivals are spread over more
     // than the 175 ns that each takes), two levels above.
     bool last = true;
@@ -269,7 +289,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void fa_gemv_mfma_kernel(const 
   float t0[IT], t1[IT];
 #pragma unroll
   for (int it = 0; it < IT; ++it) t0[it] = t1[it] = 0.f;
-  constexpr int SB = IT <= 2 ? 8 : 4;
+  constexpr int SB = IT <= 2 ? 8 : (IT <= 4 ? 4 : 2);
   for (int s0 = 0; s0 < p.splits; s0 += SB) {
     uint64_t v[SB][IT];
 #pragma unroll
@@ -295,23 +315,27 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void fa_gemv_mfma_kernel(const 
     if (tid + it * 64 * NW < pairs) put(tid + it * 64 * NW, t0[it], t1[it]);
 }
 
-template <typename T, int MT>
+template <typename T, int MT, int NW, bool GATE>
 static hipError_t launch_gemv_mfma(const GemvParams& p, hipStream_t s) {
-  const dim3 grid((unsigned)(p.N / kMfmaCols), (unsigned)p.splits);
-  const size_t lds = (size_t)(kMfmaWaves / 2) * 16 * MT * kMfmaLd * 4;
-  if (p.xg != nullptr)
-    hipLaunchKernelGGL((fa_gemv_mfma_kernel<T, MT, true>), grid, dim3(64 * kMfmaWaves), lds, s, p);
-  else
-    hipLaunchKernelGGL((fa_gemv_mfma_kernel<T, MT, false>), grid, dim3(64 * kMfmaWaves), lds, s, p);
+  const dim3 grid((unsigned)(p.N / kMfmaCols), (unsigned)p.splits, (unsigned)((p.M + 16 * MT - 1) / (16 * MT)));
+  const size_t lds = (size_t)(NW / 2) * 16 * MT * kMfmaLd * 4;
+  hipLaunchKernelGGL((fa_gemv_mfma_kernel<T, MT, NW, GATE>), grid, dim3(64 * NW), lds, s, p);
   return hipGetLastError();
 }
 
+template <typename T>
+static hipError_t dispatch_gemv_mfma(const GemvParams& p, hipStream_t s) {
+  if (p.M <= 16) return p.xg ? launch_gemv_mfma<T, 1, 4, true>(p, s) : launch_gemv_mfma<T, 1, 4, false>(p, s);
+  if (p.M <= 32) return p.xg ? launch_gemv_mfma<T, 2, 4, true>(p, s) : launch_gemv_mfma<T, 2, 4, false>(p, s);
+  return launch_gemv_mfma<T, 4, 8, false>(p, s);
+}
+
 // Host entry used by the C ABI layer: arguments validated, every matrix's
-// width a multiple of 128, K and kc multiples of 8, 3 <= M <= 32.
+// width a multiple of 128, K and kc multiples of 8, M >= 3, no gate above 32
+// rows.
 hipError_t gemv_mfma(const GemvParams& p, bool is_bf16, hipStream_t s) {
   if (p.M == 0 || p.N == 0) return hipSuccess;
-  if (p.M <= 16) return is_bf16 ? launch_gemv_mfma<__bf16, 1>(p, s) : launch_gemv_mfma<_Float16, 1>(p, s);
-  return is_bf16 ? launch_gemv_mfma<__bf16, 2>(p, s) : launch_gemv_mfma<_Float16, 2>(p, s);
+  return is_bf16 ? dispatch_gemv_mfma<__bf16>(p, s) : dispatch_gemv_mfma<_Float16>(p, s);
 }
 
 }  // namespace lsfa

@@ -22,7 +22,10 @@ against 51.9 and 54.1, o 10.9 and 13.7 against 21.9 and 20.9, gate/up 42.3 and
 46.2 against 56.1 and 56.8, down 23.1 and 27.2 against 71.0 and 61.4, LM head
 165 and 177 against 190 and 198; so every such product goes to it, unless
 autograd, a tracer or autocast has to see the call (_library_only). The norm
-is folded into the launch at up to 2 rows only.
+is folded into the launch at up to 2 rows only. Above 32 rows the same kernel
+runs over blocks of 64 rows (lsfa_gemm_group) as long as the launch has at most
+one tile of 64 x 128 per CU (GEMM_*); there it beats hipBLASLt's larger tiles
+(figures in csrc/fa_gemv_mfma.hip), beyond that it loses to them.
 
 Projections that share their input (a decoder's q/k/v, gate/up) go through
 matmul_shared_input, which runs them as one lsfa_gemv_group launch over their
@@ -56,6 +59,11 @@ AUTO_MAX_ROWS = 2    # rows that every product (and the fused norm / SwiGLU inpu
 # matrix a multiple of 128 wide, run on the library's MFMA kernel.
 MFMA_AUTO_ROWS = 32
 MFMA_AUTO_MAX_COLS = 128 * (_lib.GEMV_COUNTER_BYTES // 64)
+# Above MFMA_AUTO_ROWS rows, lsfa_gemm_group runs launches of this many tiles of
+# 64 x 128 whose K is at least GEMM_MIN_K or which group several matrices (a
+# short K alone: 2048 -> 2048 at 128 rows 15.7 us against hipBLASLt's 12.6; few
+# tiles: 4096 -> 1024 at 48 rows 19.0 against 14.6).
+GEMM_MIN_TILES, GEMM_MAX_TILES, GEMM_MIN_K = 16, 256, 4096
 
 MAX_CACHED_STREAMS = 8
 
@@ -146,6 +154,16 @@ def skinny_matmul(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor = None) ->
     return out
 
 
+def _group_args(a, bs, outs):
+    """lsfa_gemv_group_args of [a @ b for b in bs] into outs, no workspace yet."""
+    args = _lib.GemvGroupArgs(x=a.data_ptr(), x_stride=a.stride(0), dtype=_lib.TORCH_TO_LSFA[a.dtype], m=a.shape[0],
+                              k=a.shape[1], count=len(bs))
+    for i, (b, o) in enumerate(zip(bs, outs)):
+        args.w[i], args.y[i] = b.data_ptr(), o.data_ptr()
+        args.w_stride[i], args.y_stride[i], args.n[i] = b.stride(0), o.stride(0), b.shape[1]
+    return args
+
+
 def skinny_matmul_group(a: torch.Tensor, bs, outs=None, gate: torch.Tensor = None):
     """[a @ b for b in bs] for up to four b sharing a (each as for
     skinny_matmul) in one lsfa_gemv_group launch. With gate (a's shape and
@@ -167,13 +185,9 @@ def skinny_matmul_group(a: torch.Tensor, bs, outs=None, gate: torch.Tensor = Non
         return outs
     if K == 0:
         return [o.zero_() for o in outs]
-    args = _lib.GemvGroupArgs(x=a.data_ptr(), x_stride=a.stride(0), dtype=_lib.TORCH_TO_LSFA[a.dtype], m=M, k=K,
-                              count=len(bs))
+    args = _group_args(a, bs, outs)
     if gate is not None:
         args.x_gate, args.x_gate_stride = gate.data_ptr(), gate.stride(0)
-    for i, (b, o) in enumerate(zip(bs, outs)):
-        args.w[i], args.y[i] = b.data_ptr(), o.data_ptr()
-        args.w_stride[i], args.y_stride[i], args.n[i] = b.stride(0), o.stride(0), b.shape[1]
     nbytes = _lib.gemv_group_workspace_size(args)
     with torch.cuda.device(a.device):
         stream = _lib.current_stream(a.device)
@@ -215,11 +229,39 @@ def _auto_skinny(a: torch.Tensor, bs) -> bool:
     return _mfma_ok(a, bs) and not _library_only(a, *bs)
 
 
+def _gemm_ok(a: torch.Tensor, bs) -> bool:
+    """Whether lsfa_gemm_group takes these products and is the faster route."""
+    return (len(bs) <= _lib.GEMV_MAX_GROUP and a.ndim == 2 and a.is_cuda and a.shape[0] > MFMA_AUTO_ROWS
+            and a.dtype in (torch.bfloat16, torch.float16) and a.shape[1] > 0 and a.shape[1] % 8 == 0
+            and _rows_addressable(a) and a.shape[1] <= a.stride(0) <= 1 << 23 and all(
+                b.ndim == 2 and b.is_cuda and b.dtype == a.dtype and b.shape[0] == a.shape[1] and b.shape[1] % 128 == 0
+                and b.shape[1] > 0 and _rows_addressable(b) and b.stride(0) >= b.shape[1] for b in bs)
+            and GEMM_MIN_TILES <= sum(b.shape[1] for b in bs) // 128 * ((a.shape[0] + 63) // 64) <= GEMM_MAX_TILES
+            and (len(bs) > 1 or a.shape[1] >= GEMM_MIN_K)
+            and not _library_only(a, *bs))
+
+
+def _gemm_group(a: torch.Tensor, bs):
+    """[a @ b for b in bs] through lsfa_gemm_group (_gemm_ok holds)."""
+    outs = [torch.empty(a.shape[0], b.shape[1], dtype=a.dtype, device=a.device) for b in bs]
+    args = _group_args(a, bs, outs)
+    nbytes = _lib.gemm_group_workspace_size(args)
+    with torch.cuda.device(a.device):
+        stream = _lib.current_stream(a.device)
+        if nbytes:
+            ws = _workspace(a.device, stream, nbytes)
+            args.workspace, args.workspace_bytes = ws.data_ptr(), ws.numel()
+        _lib.gemm_group(args, stream)
+    return outs
+
+
 def matmul_shared_input(a: torch.Tensor, bs):
-    """[matmul(a, b) for b in bs]: one grouped skinny launch when the
-    products qualify for the skinny kernels, else one matmul each."""
+    """[matmul(a, b) for b in bs]: one grouped launch when the products
+    qualify for the library's kernels together, else one matmul each."""
     if _auto_skinny(a, bs):
         return skinny_matmul_group(a, bs)
+    if _gemm_ok(a, bs):
+        return _gemm_group(a, bs)
     return [matmul(a, b) for b in bs]
 
 
@@ -290,4 +332,6 @@ def matmul(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     assert a.dtype == b.dtype, f"dtype mismatch: a={a.dtype} b={b.dtype}"
     if _auto_skinny(a, [b]):
         return skinny_matmul(a, b)
+    if _gemm_ok(a, [b]):
+        return _gemm_group(a, [b])[0]
     return torch.matmul(a, b)

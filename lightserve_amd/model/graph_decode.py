@@ -33,7 +33,7 @@ from ..kernels.paged_attention import paged_attention_decode, paged_prefill
 from ..kernels.rope import apply_rope_
 from ..kernels.fused_rmsnorm_residual import fused_add_rmsnorm
 from ..kernels.greedy import greedy_next_token
-from ..kernels.tiled_matmul import add_rmsnorm_matmul_shared_input, matmul, swiglu_matmul
+from ..kernels.tiled_matmul import add_rmsnorm_matmul_shared_input, matmul, matmul_shared_input, swiglu_matmul
 from .minimal_llama import add_norm, init_weights, llama3_8b_shape, llama_forward, precompute_rope
 
 SEED_TOKEN_ID = 1
@@ -185,9 +185,7 @@ class KVCacheDecoder:
             pending = None
             for i, layer in enumerate(self.w.layers):
                 h, residual = add_norm(pending, residual, layer.input_layernorm_weight, cfg.rms_eps)
-                q = matmul(h, layer.q_proj)
-                k = matmul(h, layer.k_proj)
-                v = matmul(h, layer.v_proj)
+                q, k, v = matmul_shared_input(h, (layer.q_proj, layer.k_proj, layer.v_proj))
                 apply_rope_(q.view(B, c, nh, hd).transpose(1, 2), k.view(B, c, nkv, hd).transpose(1, 2),
                             self.cos, self.sin, positions=pos, v=v.view(B, c, nkv, hd).transpose(1, 2),
                             k_cache=self.k_cache[i], v_cache=self.v_cache[i], slots=slot)
@@ -195,8 +193,8 @@ class KVCacheDecoder:
                                   max_seqlen_q=c)
                 h2, residual = fused_add_rmsnorm(matmul(o.view(B * c, nh * hd), layer.o_proj), residual,
                                                  layer.post_attention_layernorm_weight, cfg.rms_eps)
-                mlp = F.silu(matmul(h2, layer.gate_proj)) * matmul(h2, layer.up_proj)
-                pending = matmul(mlp, layer.down_proj)
+                gate, up = matmul_shared_input(h2, (layer.gate_proj, layer.up_proj))
+                pending = swiglu_matmul(gate, up, layer.down_proj)
             last = slice(c - 1, B * c, c)  # each sequence's last token of the chunk
             final, _ = add_norm(pending[last].contiguous() if pending is not None else None,
                                 residual[last].contiguous(), self.w.norm_weight, cfg.rms_eps)

@@ -34,7 +34,7 @@ from ..kernels.fused_rmsnorm_residual import fused_add_rmsnorm
 from ..kernels.fused_rmsnorm_residual import rmsnorm as rmsnorm_kernel
 from ..kernels.flash_attention_varlen import flash_attention_varlen_forward
 from ..kernels.rope import apply_rope_
-from ..kernels.tiled_matmul import matmul
+from ..kernels.tiled_matmul import matmul, matmul_shared_input, swiglu_matmul
 
 
 @dataclass
@@ -152,9 +152,8 @@ def add_norm(x, residual, weight, eps):
 def attention_block(layer, config, normed_2d, B, N, cos, sin, causal, positions=None):
     """q/k/v projections, in-place RoPE, attention; returns [B*N, n_heads*head_dim]."""
     nh, nkv, hd = config.n_heads, config.kv_heads, config.head_dim
-    q = matmul(normed_2d, layer.q_proj)   # [B*N, nh*hd]
-    k = matmul(normed_2d, layer.k_proj)   # [B*N, nkv*hd]
-    v = matmul(normed_2d, layer.v_proj)
+    # [B*N, nh*hd], [B*N, nkv*hd] twice
+    q, k, v = matmul_shared_input(normed_2d, (layer.q_proj, layer.k_proj, layer.v_proj))
     q4 = q.view(B, N, nh, hd).transpose(1, 2)   # [B, nh, N, hd] views, no copies
     k4 = k.view(B, N, nkv, hd).transpose(1, 2)
     apply_rope_(q4, k4, cos, sin, positions)
@@ -181,7 +180,7 @@ def llama_forward(weights: LlamaWeights, config: LlamaConfig, input_ids: torch.T
         attn = attention_block(layer, config, normed, B, N, cos, sin, causal)
         normed2, residual = fused_add_rmsnorm(matmul(attn, layer.o_proj), residual,
                                               layer.post_attention_layernorm_weight, config.rms_eps)
-        mlp = F.silu(matmul(normed2, layer.gate_proj)) * matmul(normed2, layer.up_proj)
-        pending = matmul(mlp, layer.down_proj)
+        gate, up = matmul_shared_input(normed2, (layer.gate_proj, layer.up_proj))
+        pending = swiglu_matmul(gate, up, layer.down_proj)
     final, _ = add_norm(pending, residual, weights.norm_weight, config.rms_eps)
     return matmul(final, weights.lm_head).reshape(B, N, config.vocab_size)

@@ -755,3 +755,26 @@ def test_abi_key_split_workspace(built_library):
                 tiles = b * h * ((n + 127) // 128)
                 if tiles > SPLIT_MAX_TILES or n < SPLIT_MIN_KEYS:
                     assert _lib.fwd_workspace_size(dense(batch=b, heads_q=h, heads_kv=h, seqlen_q=n, seqlen_k=n)) == 0
+
+
+def test_abi_gemm_group_validation(built_library):
+    """lsfa_gemm_group: more than 32 rows, at most 256 tiles of 64 x 128; other
+    checks as lsfa_gemv_group's; the workspace checked for its own row count."""
+    def args(**kw):
+        return _group_args([4096, 1024, 1024], **{**dict(m=200), **kw})
+    assert _lib.gemm_group_check(args())[0] == 0
+    for kw, code in ((dict(m=32), -2), (dict(m=0), -2), (dict(m=-5), -2), (dict(m=400), -2), (dict(x=None), -1), (dict(k=4092), -2),
+                     (dict(x_gate=8192, x_gate_stride=4096), -2), (dict(norm_weight=1 << 23), -2), (dict(x=4104), -2),
+                     (dict(x_stride=1 << 24), -2), (dict(x_stride=104), -1), (dict(dtype=_lib.DTYPE_FP32), -2)):
+        assert _lib.gemm_group_check(args(**kw))[0] == code, kw
+    one = _group_args([4096], m=64)
+    need = _lib.gemm_group_workspace_size(one)
+    assert need >= _lib.GEMV_COUNTER_BYTES + 8 * 64 * 4096 * 4  # 32 column blocks: eight splits
+    for kw, word in ((dict(workspace=None), "non-NULL"), (dict(workspace_bytes=need - 1), "below"),
+                     (dict(workspace=(1 << 20) + 64), "aligned")):
+        rc, msg = _lib.gemm_group_check(_group_args([4096], m=64, **kw))
+        assert rc == -1 and word in msg
+    for m in (0, -1, 33, 1 << 20):
+        _lib.gemm_group_workspace_size(args(m=m))
+    with pytest.raises(RuntimeError, match="32 rows"):
+        _lib.gemm_group(args(m=8), 0)

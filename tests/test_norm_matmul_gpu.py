@@ -406,3 +406,51 @@ def test_matmul_routes_keep_torch_semantics(M):
         assert all(t is not None and torch.isfinite(t).all() for t in grads)
     with torch.autocast("cuda", dtype=torch.float16):
         assert matmul(x, ws[0]).dtype == torch.float16
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K,ns", [(33, 8, (128,)), (64, 4096, (4096, 1024, 1024)), (65, 1000, (256, 128)), (127, 2056, (384,)),
+                                    (128, 14336, (4096,)), (500, 4096, (4096,)), (1000, 264, (128, 128, 128, 128)),
+                                    (4096, 512, (512,))])
+def test_gemm_group_row_blocks(M, K, ns, dtype):
+    """Above 32 rows: the MFMA kernel over 64-row blocks at the edges of rows,
+    K-ranges and splits, on strided operands beside NaN, within one rounding of
+    the fp64 product; the counters return to zero, and a repeat is identical."""
+    from lightserve_amd.kernels import tiled_matmul as tm
+    print(f"case gemm M={M} K={K} N={ns} {dtype}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    xb = torch.full((M + 1, K + 8), float("nan"), device="cuda", dtype=dtype)
+    x = xb[:M, :K].copy_(torch.randn(M, K, device="cuda", generator=g))
+    ws = []
+    for n in ns:
+        wb = torch.full((K + 32, n + 16), float("nan"), device="cuda", dtype=dtype)
+        ws.append(wb[:K, 8:n + 8].copy_(torch.randn(K, n, device="cuda", generator=g) / K ** 0.5))
+    got = tm._gemm_group(x, ws)
+    again = tm._gemm_group(x, ws)
+    torch.cuda.synchronize()
+    for c, c2, w in zip(got, again, ws):
+        _assert_one_rounding(c, x, w)
+        assert torch.equal(c, c2)
+    entry = tm._workspaces.get((0, torch.cuda.current_stream().cuda_stream))
+    assert entry is None or (entry.buf[:_lib.GEMV_COUNTER_BYTES] == 0).all()
+
+
+def test_gemm_route(monkeypatch):
+    """matmul and matmul_shared_input take lsfa_gemm_group inside its range and
+    torch's GEMM outside it or where a gradient is recorded."""
+    from lightserve_amd.kernels import tiled_matmul as tm
+    print("case gemm route", flush=True)
+    calls = []
+    real = _lib.gemm_group
+    monkeypatch.setattr(_lib, "gemm_group", lambda *a: (calls.append(1), real(*a)))
+
+    def run(M, K, ns, grad=False):
+        x = torch.randn(M, K, device="cuda").to(torch.bfloat16).requires_grad_(grad)
+        ws = [(torch.randn(K, n, device="cuda") / K ** 0.5).to(torch.bfloat16) for n in ns]
+        calls.clear()
+        for c, w in zip(tm.matmul_shared_input(x, ws) if len(ws) > 1 else [matmul(x, ws[0])], ws):
+            _assert_one_rounding(c.detach(), x.detach(), w)
+        return len(calls)
+    assert run(33, 4096, (2048,)) == 1 and run(200, 2048, (1024, 512)) == 1 and run(512, 4096, (4096,)) == 1
+    assert run(48, 4096, (1024,)) == 0 and run(200, 2048, (1024,)) == 0 and run(513, 4096, (4096,)) == 0
+    assert run(64, 4096, (4096,), grad=True) == 0 and run(32, 4096, (4096,)) == 0 and run(64, 4096, (2048, 1000)) == 1
