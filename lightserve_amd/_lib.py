@@ -7,6 +7,7 @@ machine where it is missing raise RuntimeError; there is no fallback path.
 """
 import ctypes
 import os
+import struct
 import threading
 
 import torch
@@ -176,6 +177,42 @@ class RmsNormArgs(ctypes.Structure):
     ]
 
 
+# Packed forms of the argument structs: filling one from Python costs a call
+# per field and per stride array (7.8 us for lsfa_fwd_args), packing the same
+# fields in one call and copying the bytes 2.7 us. "=" is the structs' own
+# layout (test_struct_layouts compares the sizes), as their fields are aligned
+# without gaps.
+_PACK = {cls: struct.Struct(fmt) for cls, fmt in (
+    (FwdArgs, "=5Q19q2Q8ifi"), (BwdArgs, "=10QQ35q2Q8ifi"), (DecodeArgs, "=8QQ17q9if"),
+    (PrefillPagedArgs, "=8Q13q10ifi"), (GemvGroupArgs, "=3QqQq4Q4Q4q4q4i4i3Q2qfi"),
+    (RmsNormArgs, "=5Q4q3if"), (RopeArgs, "=6Q9q8i4Q7qQq2i"))}
+
+
+def pack(cls, *fields):
+    """cls (an args structure) with these values in field order, arrays spread
+    out and null pointers as 0."""
+    return cls.from_buffer_copy(_PACK[cls].pack(*fields))
+
+
+class _Here:
+    """The device guard where the tensors' device is current already."""
+    __slots__ = ()
+
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        return False
+
+
+_HERE = _Here()
+
+
+def device_guard(device):
+    """torch.cuda.device(device), at a tenth of its cost where that is current."""
+    return _HERE if torch.cuda.current_device() == device.index else torch.cuda.device(device)
+
+
 def library_path():
     return _LIB_PATH
 
@@ -276,7 +313,7 @@ def decode_workspace_size(args):
 
 
 def decode(args, stream):
-    _raise_on(load().lsfa_decode(ctypes.byref(args), ctypes.c_void_p(stream)), "lsfa_decode")
+    _raise_on(load().lsfa_decode(ctypes.byref(args), stream), "lsfa_decode")
 
 
 def prefill_paged_check(args):
@@ -286,7 +323,7 @@ def prefill_paged_check(args):
 
 
 def prefill_paged(args, stream):
-    _raise_on(load().lsfa_prefill_paged(ctypes.byref(args), ctypes.c_void_p(stream)), "lsfa_prefill_paged")
+    _raise_on(load().lsfa_prefill_paged(ctypes.byref(args), stream), "lsfa_prefill_paged")
 
 
 def prefill_paged_workspace_size(args):
@@ -316,7 +353,7 @@ def gemv_workspace_size(args):
 
 
 def gemv(args, stream):
-    _raise_on(load().lsfa_gemv(ctypes.byref(args), ctypes.c_void_p(stream)), "lsfa_gemv")
+    _raise_on(load().lsfa_gemv(ctypes.byref(args), stream), "lsfa_gemv")
 
 
 def gemv_group_check(args):
@@ -333,7 +370,7 @@ def gemv_group_workspace_size(args):
 
 
 def gemv_group(args, stream):
-    _raise_on(load().lsfa_gemv_group(ctypes.byref(args), ctypes.c_void_p(stream)), "lsfa_gemv_group")
+    _raise_on(load().lsfa_gemv_group(ctypes.byref(args), stream), "lsfa_gemv_group")
 
 
 def gemm_group_check(args):
@@ -350,7 +387,7 @@ def gemm_group_workspace_size(args):
 
 
 def gemm_group(args, stream):
-    _raise_on(load().lsfa_gemm_group(ctypes.byref(args), ctypes.c_void_p(stream)), "lsfa_gemm_group")
+    _raise_on(load().lsfa_gemm_group(ctypes.byref(args), stream), "lsfa_gemm_group")
 
 
 def greedy_check(args):
@@ -360,7 +397,7 @@ def greedy_check(args):
 
 
 def greedy(args, stream):
-    _raise_on(load().lsfa_greedy(ctypes.byref(args), ctypes.c_void_p(stream)), "lsfa_greedy")
+    _raise_on(load().lsfa_greedy(ctypes.byref(args), stream), "lsfa_greedy")
 
 
 def rope_check(args):
@@ -370,7 +407,7 @@ def rope_check(args):
 
 
 def rope(args, stream):
-    _raise_on(load().lsfa_rope(ctypes.byref(args), ctypes.c_void_p(stream)), "lsfa_rope")
+    _raise_on(load().lsfa_rope(ctypes.byref(args), stream), "lsfa_rope")
 
 
 def rmsnorm_check(args):
@@ -380,11 +417,11 @@ def rmsnorm_check(args):
 
 
 def rmsnorm(args, stream):
-    _raise_on(load().lsfa_rmsnorm(ctypes.byref(args), ctypes.c_void_p(stream)), "lsfa_rmsnorm")
+    _raise_on(load().lsfa_rmsnorm(ctypes.byref(args), stream), "lsfa_rmsnorm")
 
 
 def fwd(args, stream):
-    _raise_on(load().lsfa_fwd(ctypes.byref(args), ctypes.c_void_p(stream)), "lsfa_fwd")
+    _raise_on(load().lsfa_fwd(ctypes.byref(args), stream), "lsfa_fwd")
 
 
 def fwd_workspace_size(args):
@@ -400,13 +437,13 @@ def fwd_split(args, workspace, nbytes, stream):
 
 
 def bwd(args, stream):
-    _raise_on(load().lsfa_bwd(ctypes.byref(args), ctypes.c_void_p(stream)), "lsfa_bwd")
+    _raise_on(load().lsfa_bwd(ctypes.byref(args), stream), "lsfa_bwd")
 
 
 def bwd_noalloc(args, stream):
     """lsfa_bwd_noalloc: the backward with the library's own scratch array as
     workspace (args.workspace is ignored)."""
-    _raise_on(load().lsfa_bwd_noalloc(ctypes.byref(args), ctypes.c_void_p(stream)), "lsfa_bwd_noalloc")
+    _raise_on(load().lsfa_bwd_noalloc(ctypes.byref(args), stream), "lsfa_bwd_noalloc")
 
 
 def strides4(t):
@@ -424,10 +461,14 @@ def fast_layout_ok(t):
     """Whether the bf16/fp16 kernels can address t in place: unit head-dim
     stride, head_dim and every other stride a multiple of 8 elements, 16-byte
     aligned base (the requirements lsfa_fwd_check/lsfa_bwd_check enforce)."""
-    if t.stride(-1) != 1 or t.shape[-1] % 8 != 0 or t.data_ptr() % 16 != 0:
+    *outer, inner = t.stride()
+    if inner != 1 or t.shape[-1] % 8 != 0 or t.data_ptr() % 16 != 0:
         return False
-    return all(s % 8 == 0 for s in t.stride()[:-1])
+    bits = 0
+    for s in outer:
+        bits |= s
+    return bits & 7 == 0
 
 
 def current_stream(device):
-    return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)

@@ -76,7 +76,7 @@ def launch_forward(args, device):
     if (args.seqlen_k >= SPLIT_MIN_KEYS and args.dtype != _lib.DTYPE_FP32
             and args.batch * args.heads_q * ((args.seqlen_q + 127) // 128) <= SPLIT_MAX_TILES):
         nbytes = _lib.fwd_workspace_size(args)
-    with torch.cuda.device(device):
+    with _lib.device_guard(device):
         if nbytes > 0:
             ws = torch.empty(nbytes, device=device, dtype=torch.uint8)  # 512-byte aligned blocks
             _lib.fwd_split(args, ws.data_ptr(), nbytes, _lib.current_stream(device))
@@ -97,15 +97,11 @@ def forward_into(q, k, v, causal, scale, want_lse):
     qk, kk, vk = (as_kernel_layout(t, dp) for t in (q, k, v))
     direct = q.dtype == torch.float32 or (dp == D and _lib.fast_layout_ok(o))
     ok = o if direct else torch.empty(B, H, N, dp, device=q.device, dtype=q.dtype)
-    lse_ptr, lse_stride = lse_args(lse)
-    args = _lib.FwdArgs(
-        q=qk.data_ptr(), k=kk.data_ptr(), v=vk.data_ptr(), o=ok.data_ptr(), lse=lse_ptr,
-        q_stride=_lib.strides4(qk), k_stride=_lib.strides4(kk), v_stride=_lib.strides4(vk),
-        o_stride=_lib.strides4(ok), lse_stride=lse_stride,
-        cu_seqlens_q=None, cu_seqlens_k=None,
-        dtype=_lib.TORCH_TO_LSFA[q.dtype], batch=B, heads_q=H, heads_kv=H, seqlen_q=N, seqlen_k=N,
-        head_dim=dp, causal=int(bool(causal)), sm_scale=scale, reserved=0,
-    )
+    args = _lib.pack(
+        _lib.FwdArgs, qk.data_ptr(), kk.data_ptr(), vk.data_ptr(), ok.data_ptr(), lse.data_ptr() if want_lse else 0,
+        *qk.stride(), *kk.stride(), *vk.stride(), *ok.stride(), *(lse.stride() if want_lse else (0, 0, 0)),
+        0, 0,  # no cu_seqlens
+        _lib.TORCH_TO_LSFA[q.dtype], B, H, H, N, N, dp, bool(causal), scale, 0)
     launch_forward(args, q.device)
     if ok is not o:
         o.copy_(ok[..., :D])

@@ -49,17 +49,12 @@ def _backward_args(do: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.
     dqk, dkk, dvk = outs
     L = L.contiguous()
     assert L.shape == (B, H, N) and L.dtype == torch.float32, "L must be fp32 [B, H, N]"
-    args = _lib.BwdArgs(
-        q=qk.data_ptr(), k=kk.data_ptr(), v=vk.data_ptr(), o=ok_.data_ptr(), dout=dok.data_ptr(),
-        lse=L.data_ptr(), dq=dqk.data_ptr(), dk=dkk.data_ptr(), dv=dvk.data_ptr(), workspace=None,
-        workspace_bytes=0,
-        q_stride=_lib.strides4(qk), k_stride=_lib.strides4(kk), v_stride=_lib.strides4(vk),
-        o_stride=_lib.strides4(ok_), do_stride=_lib.strides4(dok), dq_stride=_lib.strides4(dqk),
-        dk_stride=_lib.strides4(dkk), dv_stride=_lib.strides4(dvk), lse_stride=_lib._i64x3(*L.stride()),
-        cu_seqlens_q=None, cu_seqlens_k=None,
-        dtype=_lib.TORCH_TO_LSFA[q.dtype], batch=B, heads_q=H, heads_kv=H, seqlen_q=N, seqlen_k=N,
-        head_dim=dp, causal=int(bool(causal)), sm_scale=scale, flags=flags,
-    )
+    args = _lib.pack(
+        _lib.BwdArgs, qk.data_ptr(), kk.data_ptr(), vk.data_ptr(), ok_.data_ptr(), dok.data_ptr(), L.data_ptr(),
+        dqk.data_ptr(), dkk.data_ptr(), dvk.data_ptr(), 0, 0,  # the workspace follows
+        *qk.stride(), *kk.stride(), *vk.stride(), *ok_.stride(), *dok.stride(), *dqk.stride(), *dkk.stride(),
+        *dvk.stride(), *L.stride(), 0, 0,  # no cu_seqlens
+        _lib.TORCH_TO_LSFA[q.dtype], B, H, H, N, N, dp, bool(causal), scale, flags)
     nbytes = _lib.bwd_workspace_size(args)
     # The caching allocator hands out 512-byte aligned blocks (the ABI asks for 256).
     workspace = torch.empty(nbytes, device=q.device, dtype=torch.uint8)
@@ -74,7 +69,7 @@ def _flash_attention_backward(do: torch.Tensor, q: torch.Tensor, k: torch.Tensor
     dq, dk, dv = keep[:3]
     if args is None:
         return dq, dk, dv
-    with torch.cuda.device(q.device):
+    with _lib.device_guard(q.device):
         _lib.bwd(args, _lib.current_stream(q.device))
     D = q.shape[-1]
     for t, tk in zip((dq, dk, dv), keep[3]):

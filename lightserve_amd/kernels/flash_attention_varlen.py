@@ -17,7 +17,13 @@ import math
 import torch
 
 from .. import _lib
-from .flash_attention import SUPPORTED_DTYPES, as_kernel_layout, launch_forward, lse_args
+from .flash_attention import SUPPORTED_DTYPES, as_kernel_layout, launch_forward
+
+
+def _thd(t):
+    """Strides of a packed [tokens, heads, d] tensor in ABI order (b, h, n, d)."""
+    n, h, d = t.stride()
+    return 0, h, n, d
 
 
 def _check_varlen_inputs(q, k, v, cu_seqlens_q, cu_seqlens_k):
@@ -59,16 +65,10 @@ def flash_attention_varlen_forward(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seql
     ok = o if direct else torch.empty(Tq, Hq, dp, device=q.device, dtype=q.dtype)
     cu_q = cu_seqlens_q.contiguous()
     cu_k = cu_seqlens_k.contiguous()
-    lse_ptr, _ = lse_args(lse)
-    args = _lib.FwdArgs(
-        q=qk.data_ptr(), k=kk.data_ptr(), v=vk.data_ptr(), o=ok.data_ptr(), lse=lse_ptr,
-        q_stride=_lib.strides_thd(qk), k_stride=_lib.strides_thd(kk), v_stride=_lib.strides_thd(vk),
-        o_stride=_lib.strides_thd(ok), lse_stride=_lib._i64x3(0, lse.stride(0), lse.stride(1)),
-        cu_seqlens_q=cu_q.data_ptr(), cu_seqlens_k=cu_k.data_ptr(),
-        dtype=_lib.TORCH_TO_LSFA[q.dtype], batch=batch, heads_q=Hq, heads_kv=Hkv,
-        seqlen_q=int(max_seqlen_q), seqlen_k=int(max_seqlen_k),
-        head_dim=dp, causal=int(bool(causal)), sm_scale=scale, reserved=0,
-    )
+    args = _lib.pack(
+        _lib.FwdArgs, qk.data_ptr(), kk.data_ptr(), vk.data_ptr(), ok.data_ptr(), lse.data_ptr(),
+        *_thd(qk), *_thd(kk), *_thd(vk), *_thd(ok), 0, *lse.stride(), cu_q.data_ptr(), cu_k.data_ptr(),
+        _lib.TORCH_TO_LSFA[q.dtype], batch, Hq, Hkv, int(max_seqlen_q), int(max_seqlen_k), dp, bool(causal), scale, 0)
     launch_forward(args, q.device)
     if ok is not o:
         o.copy_(ok[..., :D])
@@ -103,20 +103,16 @@ def flash_attention_varlen_backward(do, q, k, v, o, lse, cu_seqlens_q, cu_seqlen
     lse = lse.contiguous()
     cu_q = cu_seqlens_q.contiguous()
     cu_k = cu_seqlens_k.contiguous()
-    th = _lib.strides_thd
-    args = _lib.BwdArgs(
-        q=qk.data_ptr(), k=kk.data_ptr(), v=vk.data_ptr(), o=ok_.data_ptr(), dout=dok.data_ptr(),
-        lse=lse.data_ptr(), dq=dqk.data_ptr(), dk=dkk.data_ptr(), dv=dvk.data_ptr(), workspace=None,
-        workspace_bytes=0, q_stride=th(qk), k_stride=th(kk), v_stride=th(vk), o_stride=th(ok_), do_stride=th(dok),
-        dq_stride=th(dqk), dk_stride=th(dkk), dv_stride=th(dvk),
-        lse_stride=_lib._i64x3(0, lse.stride(0), lse.stride(1)),
-        cu_seqlens_q=cu_q.data_ptr(), cu_seqlens_k=cu_k.data_ptr(), dtype=_lib.TORCH_TO_LSFA[q.dtype],
-        batch=batch, heads_q=Hq, heads_kv=Hkv, seqlen_q=int(max_seqlen_q), seqlen_k=int(max_seqlen_k),
-        head_dim=dp, causal=int(bool(causal)), sm_scale=scale, flags=0)
+    args = _lib.pack(
+        _lib.BwdArgs, qk.data_ptr(), kk.data_ptr(), vk.data_ptr(), ok_.data_ptr(), dok.data_ptr(), lse.data_ptr(),
+        dqk.data_ptr(), dkk.data_ptr(), dvk.data_ptr(), 0, 0,  # the workspace follows
+        *_thd(qk), *_thd(kk), *_thd(vk), *_thd(ok_), *_thd(dok), *_thd(dqk), *_thd(dkk), *_thd(dvk), 0, *lse.stride(),
+        cu_q.data_ptr(), cu_k.data_ptr(), _lib.TORCH_TO_LSFA[q.dtype], batch, Hq, Hkv, int(max_seqlen_q),
+        int(max_seqlen_k), dp, bool(causal), scale, 0)
     n = _lib.bwd_workspace_size(args)
     ws = torch.empty(max(n, 1), device=q.device, dtype=torch.uint8)
     args.workspace, args.workspace_bytes = ws.data_ptr(), n
-    with torch.cuda.device(q.device):
+    with _lib.device_guard(q.device):
         _lib.bwd(args, _lib.current_stream(q.device))
     for t, tk in zip((dq, dk, dv), outs):
         if tk is not t:

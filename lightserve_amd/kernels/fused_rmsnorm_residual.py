@@ -17,15 +17,12 @@ from .. import _lib
 
 def _launch(x, residual, weight, eps, out, residual_out):
     M, N = x.shape
-    args = _lib.RmsNormArgs(
-        x=x.data_ptr(), residual=residual.data_ptr() if residual is not None else None,
-        weight=weight.data_ptr(), out=out.data_ptr(),
-        residual_out=residual_out.data_ptr() if residual_out is not None else None,
-        x_stride=x.stride(0), residual_stride=residual.stride(0) if residual is not None else 0,
-        out_stride=out.stride(0), residual_out_stride=residual_out.stride(0) if residual_out is not None else 0,
-        dtype=_lib.TORCH_TO_LSFA[x.dtype], rows=M, cols=N, eps=float(eps),
-    )
-    with torch.cuda.device(x.device):
+    args = _lib.pack(
+        _lib.RmsNormArgs, x.data_ptr(), residual.data_ptr() if residual is not None else 0, weight.data_ptr(),
+        out.data_ptr(), residual_out.data_ptr() if residual_out is not None else 0, x.stride(0),
+        residual.stride(0) if residual is not None else 0, out.stride(0),
+        residual_out.stride(0) if residual_out is not None else 0, _lib.TORCH_TO_LSFA[x.dtype], M, N, float(eps))
+    with _lib.device_guard(x.device):
         _lib.rmsnorm(args, _lib.current_stream(x.device))
 
 

@@ -28,6 +28,6 @@ def greedy_next_token(logits: torch.Tensor, out: torch.Tensor = None, seq_lens: 
                            seq_lens=seq_lens.data_ptr() if seq_lens is not None else None,
                            logits_stride=logits.stride(0), dtype=_lib.TORCH_TO_LSFA[logits.dtype], rows=rows,
                            cols=cols)
-    with torch.cuda.device(logits.device):
+    with _lib.device_guard(logits.device):
         _lib.greedy(args, _lib.current_stream(logits.device))
     return out

@@ -74,23 +74,18 @@ def paged_attention_decode(q, k_cache, v_cache, block_tables, seq_lens, *, max_s
     sl = seq_lens.contiguous()
     o = torch.empty(B, Hq, D, device=q.device, dtype=q.dtype)
     lse = torch.empty(B, Hq, device=q.device, dtype=torch.float32) if return_lse else None
-    args = _lib.DecodeArgs(
-        q=q_.data_ptr(), k_cache=k_cache.data_ptr(), v_cache=v_cache.data_ptr(), o=o.data_ptr(),
-        lse=lse.data_ptr() if lse is not None else None, block_tables=bt.data_ptr(), seq_lens=sl.data_ptr(),
-        workspace=None, workspace_bytes=0,
-        q_stride=_lib._i64x3(*q_.stride()), k_stride=_lib._i64x4(*k_cache.stride()),
-        v_stride=_lib._i64x4(*v_cache.stride()), o_stride=_lib._i64x3(*o.stride()),
-        lse_stride=_lib._i64x2(*(lse.stride() if lse is not None else (0, 0))),
-        block_table_stride=bt.stride(0), dtype=_lib.TORCH_TO_LSFA[q.dtype], batch=B, heads_q=Hq,
-        heads_kv=Hkv, head_dim=D, block_size=block_size, num_blocks=num_blocks,
-        max_blocks_per_seq=bt.shape[1], max_seq_len=int(max_seq_len), sm_scale=scale,
-    )
+    args = _lib.pack(
+        _lib.DecodeArgs, q_.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), o.data_ptr(),
+        lse.data_ptr() if return_lse else 0, bt.data_ptr(), sl.data_ptr(), 0, 0,  # the workspace follows
+        *q_.stride(), *k_cache.stride(), *v_cache.stride(), *o.stride(), *(lse.stride() if return_lse else (0, 0)),
+        bt.stride(0), _lib.TORCH_TO_LSFA[q.dtype], B, Hq, Hkv, D, block_size, num_blocks, bt.shape[1],
+        int(max_seq_len), scale)
     nbytes = _lib.decode_workspace_size(args)
     ws = None
     if nbytes > 0:
         ws = torch.empty(nbytes, device=q.device, dtype=torch.uint8)  # 512-byte aligned blocks
         args.workspace, args.workspace_bytes = ws.data_ptr(), nbytes
-    with torch.cuda.device(q.device):
+    with _lib.device_guard(q.device):
         _lib.decode(args, _lib.current_stream(q.device))
     return (o, lse) if return_lse else o
 
@@ -125,23 +120,18 @@ def paged_prefill(q, k_cache, v_cache, block_tables, cu_seqlens_q, seq_lens_k, *
     cu, sl = cu_seqlens_q.contiguous(), seq_lens_k.contiguous()  # kept alive until the launch
     o = torch.empty(T, Hq, D, device=q.device, dtype=q.dtype)
     lse = torch.empty(Hq, T, device=q.device, dtype=torch.float32) if return_lse else None
-    args = _lib.PrefillPagedArgs(
-        q=q_.data_ptr(), k_cache=k_cache.data_ptr(), v_cache=v_cache.data_ptr(), o=o.data_ptr(),
-        lse=lse.data_ptr() if lse is not None else None, cu_seqlens_q=cu.data_ptr(),
-        seq_lens_k=sl.data_ptr(), block_tables=bt.data_ptr(),
-        q_stride=_lib._i64x2(*q_.stride()[:2]), k_stride=_lib._i64x3(*k_cache.stride()[:3]),
-        v_stride=_lib._i64x3(*v_cache.stride()[:3]), o_stride=_lib._i64x2(*o.stride()[:2]),
-        lse_stride=_lib._i64x2(*(lse.stride() if lse is not None else (0, 0))),
-        block_table_stride=bt.stride(0), dtype=_lib.TORCH_TO_LSFA[q.dtype], batch=B, heads_q=Hq,
-        heads_kv=Hkv, head_dim=D, block_size=block_size, num_blocks=num_blocks, max_blocks_per_seq=bt.shape[1],
-        max_seqlen_q=int(max_seqlen_q), causal=int(bool(causal)), sm_scale=scale, reserved=0,
-    )
+    args = _lib.pack(
+        _lib.PrefillPagedArgs, q_.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), o.data_ptr(),
+        lse.data_ptr() if return_lse else 0, cu.data_ptr(), sl.data_ptr(), bt.data_ptr(),
+        *q_.stride()[:2], *k_cache.stride()[:3], *v_cache.stride()[:3], *o.stride()[:2],
+        *(lse.stride() if return_lse else (0, 0)), bt.stride(0), _lib.TORCH_TO_LSFA[q.dtype], B, Hq, Hkv, D,
+        block_size, num_blocks, bt.shape[1], int(max_seqlen_q), bool(causal), scale, 0)
     if T > 0:
         # few query tiles for the GPU: their keys are shared out over several workgroups
         nbytes = 0
         if bt.shape[1] * block_size >= SPLIT_MIN_KEYS and B * Hq * ((args.max_seqlen_q + 127) // 128) <= SPLIT_MAX_TILES:
             nbytes = _lib.prefill_paged_workspace_size(args)
-        with torch.cuda.device(q.device):
+        with _lib.device_guard(q.device):
             if nbytes > 0:
                 ws = torch.empty(nbytes, device=q.device, dtype=torch.uint8)  # 512-byte aligned blocks
                 _lib.prefill_paged_split(args, ws.data_ptr(), nbytes, _lib.current_stream(q.device))

@@ -25,6 +25,9 @@ import torch
 from .. import _lib
 
 
+_ZEROS = (0, 0, 0, 0)
+
+
 def _check(q, k, cos, sin):
     assert q.dim() == 4, "q must be [batch, heads, seqlen, head_dim]"
     assert q.is_cuda, "q must be a GPU tensor"
@@ -78,25 +81,18 @@ def apply_rope_(q, k, cos, sin, positions=None, *, v=None, k_cache=None, v_cache
             "positions must be an int32 GPU tensor of shape [batch]"
         positions = positions.contiguous()
     c, s = cos.contiguous(), sin.contiguous()  # no copies for precompute_rope's tables
-    args = _lib.RopeArgs(
-        q=q.data_ptr(), k=k.data_ptr() if k is not None else None, cos=c.data_ptr(), sin=s.data_ptr(),
-        positions=positions.data_ptr() if positions is not None else None, cu_seqlens=None,
-        q_stride=_lib.strides4(q), k_stride=_lib.strides4(k) if k is not None else _lib._i64x4(0, 0, 0, 0),
-        table_stride=c.stride(0), dtype=_lib.TORCH_TO_LSFA[q.dtype], batch=B, seqlen=N, heads_q=Hq,
-        heads_kv=k.shape[1] if k is not None else 0, head_dim=D, max_pos=c.shape[0], reserved=0,
-    )
+    cache = (0, 0, 0, 0, *_ZEROS, 0, 0, 0, 0, 0, 0, 0)
     if k_cache is not None:
         sl = slots.contiguous() if slots is not None else None
-        args.v, args.k_cache, args.v_cache = v.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr()
-        if sl is not None:
-            args.slots = sl.data_ptr()
-        else:
-            args.block_tables, args.block_table_stride = block_tables.data_ptr(), block_tables.stride(0)
-            args.block_size, args.max_blocks_per_seq = k_cache.shape[1], block_tables.shape[1]
-        args.v_stride = _lib.strides4(v)
-        args.cache_stride[0], args.cache_stride[1] = k_cache.stride(1), k_cache.stride(2)
-        args.num_slots = k_cache.shape[0] * k_cache.shape[1]
-    with torch.cuda.device(q.device):
+        cache = (v.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), sl.data_ptr() if sl is not None else 0,
+                 *v.stride(), k_cache.stride(1), k_cache.stride(2), k_cache.shape[0] * k_cache.shape[1],
+                 *((0, 0, 0, 0) if sl is not None else (block_tables.data_ptr(), block_tables.stride(0),
+                                                        k_cache.shape[1], block_tables.shape[1])))
+    args = _lib.pack(
+        _lib.RopeArgs, q.data_ptr(), k.data_ptr() if k is not None else 0, c.data_ptr(), s.data_ptr(),
+        positions.data_ptr() if positions is not None else 0, 0, *q.stride(), *(k.stride() if k is not None else _ZEROS),
+        c.stride(0), _lib.TORCH_TO_LSFA[q.dtype], B, N, Hq, k.shape[1] if k is not None else 0, D, c.shape[0], 0, *cache)
+    with _lib.device_guard(q.device):
         _lib.rope(args, _lib.current_stream(q.device))
     return q, k
 

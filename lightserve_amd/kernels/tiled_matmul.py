@@ -50,8 +50,13 @@ import collections
 import threading
 
 import torch
+from torch.autograd import forward_ad
 
 from .. import _lib
+
+_interpreter = torch._C._functorch.peek_interpreter_stack
+_dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
+_tracing = torch._C._get_tracing_state
 
 SKINNY_MAX_ROWS = 32  # what lsfa_gemv takes (more than 8 rows: MFMA kernel only)
 AUTO_MAX_ROWS = 2    # rows that every product (and the fused norm / SwiGLU inputs) routes to it
@@ -145,7 +150,7 @@ def skinny_matmul(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor = None) ->
                          x_stride=a.stride(0), w_stride=b.stride(0), y_stride=out.stride(0),
                          dtype=_lib.TORCH_TO_LSFA[a.dtype], m=M, k=K, n=N)
     nbytes = _lib.gemv_workspace_size(args)
-    with torch.cuda.device(a.device):
+    with _lib.device_guard(a.device):
         stream = _lib.current_stream(a.device)
         if nbytes:
             ws = _workspace(a.device, stream, nbytes)
@@ -154,14 +159,32 @@ def skinny_matmul(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor = None) ->
     return out
 
 
-def _group_args(a, bs, outs):
-    """lsfa_gemv_group_args of [a @ b for b in bs] into outs, no workspace yet."""
-    args = _lib.GemvGroupArgs(x=a.data_ptr(), x_stride=a.stride(0), dtype=_lib.TORCH_TO_LSFA[a.dtype], m=a.shape[0],
-                              k=a.shape[1], count=len(bs))
-    for i, (b, o) in enumerate(zip(bs, outs)):
-        args.w[i], args.y[i] = b.data_ptr(), o.data_ptr()
-        args.w_stride[i], args.y_stride[i], args.n[i] = b.stride(0), o.stride(0), b.shape[1]
-    return args
+_ZEROS = (0, 0, 0, 0)
+
+
+def _group_args(a, bs, outs, gate=None, norm=(0, 0, 0, 0, 0, 0.0)):
+    """lsfa_gemv_group_args of [a @ b for b in bs] into outs, no workspace yet;
+    norm: (weight, residual, residual_out, their strides, eps)."""
+    pad = _ZEROS[len(bs):]
+    return _lib.pack(
+        _lib.GemvGroupArgs, a.data_ptr(), 0, 0, a.stride(0), *((0, 0) if gate is None else (gate.data_ptr(), gate.stride(0))),
+        *[b.data_ptr() for b in bs], *pad, *[o.data_ptr() for o in outs], *pad, *[b.stride(0) for b in bs], *pad,
+        *[o.stride(0) for o in outs], *pad, *[b.shape[1] for b in bs], *pad, _lib.TORCH_TO_LSFA[a.dtype], a.shape[0],
+        a.shape[1], len(bs), *norm, 0)
+
+
+def _run_group(args, device, size=_lib.gemv_group_workspace_size, launch=_lib.gemv_group):
+    nbytes = size(args)
+    with _lib.device_guard(device):
+        stream = _lib.current_stream(device)
+        if nbytes:
+            ws = _workspace(device, stream, nbytes)
+            args.workspace, args.workspace_bytes = ws.data_ptr(), ws.numel()
+        launch(args, stream)
+
+
+def _empty_outs(a, bs):
+    return [torch.empty(a.shape[0], b.shape[1], dtype=a.dtype, device=a.device) for b in bs]
 
 
 def skinny_matmul_group(a: torch.Tensor, bs, outs=None, gate: torch.Tensor = None):
@@ -185,16 +208,7 @@ def skinny_matmul_group(a: torch.Tensor, bs, outs=None, gate: torch.Tensor = Non
         return outs
     if K == 0:
         return [o.zero_() for o in outs]
-    args = _group_args(a, bs, outs)
-    if gate is not None:
-        args.x_gate, args.x_gate_stride = gate.data_ptr(), gate.stride(0)
-    nbytes = _lib.gemv_group_workspace_size(args)
-    with torch.cuda.device(a.device):
-        stream = _lib.current_stream(a.device)
-        if nbytes:
-            ws = _workspace(a.device, stream, nbytes)
-            args.workspace, args.workspace_bytes = ws.data_ptr(), ws.numel()
-        _lib.gemv_group(args, stream)
+    _run_group(_group_args(a, bs, outs, gate), a.device)
     return outs
 
 
@@ -202,12 +216,13 @@ def _library_only(*tensors) -> bool:
     """Whether a call on these tensors has to go through torch's own operators:
     a gradient is recorded (reverse or forward mode), a subclass, mode or
     transform looks at the operators, or autocast may change their types."""
-    return (any(type(t) not in (torch.Tensor, torch.nn.Parameter) for t in tensors)
-            or (torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
-            or torch.autograd.forward_ad._current_level >= 0
-            or torch._C._functorch.peek_interpreter_stack() is not None
-            or torch._C._len_torch_dispatch_stack() > 0 or torch._C._len_torch_function_stack() > 0
-            or torch.is_autocast_enabled("cuda") or torch._C._get_tracing_state() is not None
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        kind = type(t)
+        if (kind is not torch.Tensor and kind is not torch.nn.Parameter) or (grad and t.requires_grad):
+            return True
+    return (forward_ad._current_level >= 0 or _interpreter() is not None or _dispatch_modes() > 0
+            or _function_modes() > 0 or _tracing() is not None or torch.is_autocast_enabled("cuda")
             or torch.compiler.is_compiling())
 
 
@@ -229,6 +244,15 @@ def _auto_skinny(a: torch.Tensor, bs) -> bool:
     return _mfma_ok(a, bs) and not _library_only(a, *bs)
 
 
+def _skinny_run(a: torch.Tensor, bs):
+    """skinny_matmul_group where _auto_skinny holds (its conditions are checked)."""
+    if 0 in a.shape or sum(b.shape[1] for b in bs) == 0:
+        return skinny_matmul_group(a, bs)
+    outs = _empty_outs(a, bs)
+    _run_group(_group_args(a, bs, outs), a.device)
+    return outs
+
+
 def _gemm_ok(a: torch.Tensor, bs) -> bool:
     """Whether lsfa_gemm_group takes these products and is the faster route."""
     return (len(bs) <= _lib.GEMV_MAX_GROUP and a.ndim == 2 and a.is_cuda and a.shape[0] > MFMA_AUTO_ROWS
@@ -243,15 +267,8 @@ def _gemm_ok(a: torch.Tensor, bs) -> bool:
 
 def _gemm_group(a: torch.Tensor, bs):
     """[a @ b for b in bs] through lsfa_gemm_group (_gemm_ok holds)."""
-    outs = [torch.empty(a.shape[0], b.shape[1], dtype=a.dtype, device=a.device) for b in bs]
-    args = _group_args(a, bs, outs)
-    nbytes = _lib.gemm_group_workspace_size(args)
-    with torch.cuda.device(a.device):
-        stream = _lib.current_stream(a.device)
-        if nbytes:
-            ws = _workspace(a.device, stream, nbytes)
-            args.workspace, args.workspace_bytes = ws.data_ptr(), ws.numel()
-        _lib.gemm_group(args, stream)
+    outs = _empty_outs(a, bs)
+    _run_group(_group_args(a, bs, outs), a.device, _lib.gemm_group_workspace_size, _lib.gemm_group)
     return outs
 
 
@@ -259,7 +276,7 @@ def matmul_shared_input(a: torch.Tensor, bs):
     """[matmul(a, b) for b in bs]: one grouped launch when the products
     qualify for the library's kernels together, else one matmul each."""
     if _auto_skinny(a, bs):
-        return skinny_matmul_group(a, bs)
+        return _skinny_run(a, bs)
     if _gemm_ok(a, bs):
         return _gemm_group(a, bs)
     return [matmul(a, b) for b in bs]
@@ -305,22 +322,9 @@ def add_rmsnorm_matmul_shared_input(x, residual, weight, eps, bs, write_residual
     outs = [torch.empty(M, b.shape[1], dtype=x.dtype, device=x.device) for b in bs]
     if M == 0:
         return outs, (h if residual is not None else x)
-    args = _lib.GemvGroupArgs(x=x.data_ptr(), x_stride=x.stride(0), dtype=_lib.TORCH_TO_LSFA[x.dtype], m=M, k=K,
-                              count=len(bs), norm_weight=weight.data_ptr(), eps=float(eps))
-    if residual is not None:
-        args.residual, args.residual_stride = residual.data_ptr(), residual.stride(0)
-    if h is not None:
-        args.residual_out, args.residual_out_stride = h.data_ptr(), h.stride(0)
-    for i, (b, o) in enumerate(zip(bs, outs)):
-        args.w[i], args.y[i] = b.data_ptr(), o.data_ptr()
-        args.w_stride[i], args.y_stride[i], args.n[i] = b.stride(0), o.stride(0), b.shape[1]
-    nbytes = _lib.gemv_group_workspace_size(args)
-    with torch.cuda.device(x.device):
-        stream = _lib.current_stream(x.device)
-        if nbytes:
-            ws = _workspace(x.device, stream, nbytes)
-            args.workspace, args.workspace_bytes = ws.data_ptr(), ws.numel()
-        _lib.gemv_group(args, stream)
+    _run_group(_group_args(x, bs, outs, norm=(
+        weight.data_ptr(), residual.data_ptr() if residual is not None else 0, h.data_ptr() if h is not None else 0,
+        residual.stride(0) if residual is not None else 0, h.stride(0) if h is not None else 0, float(eps))), x.device)
     return outs, (h if residual is not None else x)
 
 
@@ -331,7 +335,7 @@ def matmul(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     assert a.is_cuda and b.is_cuda, "the gfx950 path needs GPU tensors"
     assert a.dtype == b.dtype, f"dtype mismatch: a={a.dtype} b={b.dtype}"
     if _auto_skinny(a, [b]):
-        return skinny_matmul(a, b)
+        return _skinny_run(a, [b])[0]
     if _gemm_ok(a, [b]):
         return _gemm_group(a, [b])[0]
     return torch.matmul(a, b)

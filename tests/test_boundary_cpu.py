@@ -778,3 +778,16 @@ def test_abi_gemm_group_validation(built_library):
         _lib.gemm_group_workspace_size(args(m=m))
     with pytest.raises(RuntimeError, match="32 rows"):
         _lib.gemm_group(args(m=8), 0)
+
+
+def test_packed_structs_fill_every_field_in_order():
+    """_lib.pack: the packed form of each args struct has its size and puts the
+    values into the fields in order, arrays spread out."""
+    for cls, packing in _lib._PACK.items():
+        assert packing.size == ctypes.sizeof(cls)
+        values = list(range(1, 1 + len(packing.unpack(bytes(packing.size)))))
+        got = []
+        for name, _ in cls._fields_:
+            v = getattr(_lib.pack(cls, *values), name)
+            got += list(v) if hasattr(v, "__len__") else [v]
+        assert got == values, cls.__name__
