@@ -150,14 +150,17 @@ DecodeSplit decode_split(const lsfa_decode_args* a) {
   DecodeSplit d;
   const int maxs = std::max(a->max_seq_len, 0);
   const long long units = std::max(1LL, (long long)a->batch * a->heads_kv);
-  // Lane-group kernel: splits of about 512 tokens while fewer than ~16
-  // workgroups per CU exist (sequence lengths vary, and short splits keep the
-  // longest sequences from setting the tail). MFMA kernel (one workgroup per
-  // CU): splits only below one workgroup per CU, of at least 4096 tokens, so
-  // that each workgroup's first-load latency is amortised.
+  // Lane-group kernel: up to ~16 workgroups per CU, splits of at least 256
+  // tokens (128 where 256 would leave CUs idle; none up to 512 tokens where the
+  // sequences alone fill half the GPU: 16 x 500 x 8 KV heads 11.1 us unsplit, 14.0
+  // split in two). Each sequence gets splits by its own length (kernel). MFMA
+  // kernel (one workgroup per CU): up to one workgroup per CU, splits of at least
+  // 512 tokens: 16 sequences of 1000..3000 with 4 KV heads of group 7, 64
+  // workgroups unsplit, 39.0 -> 23.5 us (1024 and 256 the same).
   const int g = a->heads_kv > 0 ? a->heads_q / a->heads_kv : 1;
   const bool mfma = lsfa::decode_uses_mfma(g, std::max(0, log2_exact(std::max(1, a->block_size))));
-  const long long target = mfma ? 256 : 4096, min_split = mfma ? 4096 : 512;
+  const long long target = mfma ? 256 : 4096;
+  const long long min_split = mfma ? 512 : (units * ((maxs + 255) / 256) < 256 ? 128 : (units >= 128 && maxs <= 512 ? 512 : 256));
   long long ns = 1;
   if (units < target && maxs > min_split)
     ns = std::min<long long>((target + units - 1) / units, (maxs + min_split - 1) / min_split);

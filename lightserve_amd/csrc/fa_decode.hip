@@ -79,6 +79,45 @@ __device__ __forceinline__ float dot8(const X8& a, const X8& b) {
   return dot2(__builtin_shufflevector(a, a, 6, 7), __builtin_shufflevector(b, b, 6, 7), d);
 }
 
+// Tokens per split of a sequence of seq tokens. The host sizes the grid and the
+// workspace for the longest sequence it was told of (num_splits splits of at
+// most split_tokens); each sequence shares those splits out by its own length,
+// in splits of at least 512 tokens, or 256 or 128 where longer ones would leave
+// CUs without a workgroup. 64 sequences of 100..1000 tokens under a limit of
+// 16384 took splits of 2048, one workgroup for each longest sequence: 165 -> 42 us
+// (with the order below); 4 of 2000..6000 44.5 -> 27.9, 1 x 1000 x 32 heads 18.9 ->
+// 10.8.
+__device__ __forceinline__ int decode_split_tokens(const DecodeParams& p, int seq) {
+  if (p.num_splits == 1) return p.split_tokens;
+  const int64_t units = (int64_t)p.B * p.Hkv;
+  const int least = units * ((seq + 511) >> 9) >= 256 ? 512 : (units * ((seq + 255) >> 8) >= 256 ? 256 : 128);
+  const int even = __builtin_amdgcn_readfirstlane((seq + p.num_splits - 1) / p.num_splits);
+  return min((max(even, least) + 63) & ~63, p.split_tokens);
+}
+
+// Workgroups are numbered [split][sequence][KV head]: the heads of a token range
+// run side by side, so that the 256-byte rows they read of a token (adjacent in
+// the cache) are requested together (with the splits innermost, 32 sequences of
+// 1024..8192 tokens read 4.3 instead of 4.7 TB/s, 64 of 3000..4000 with 32 KV heads
+// 6.0 instead of 6.5), and the splits that no sequence has come last. Splits past
+// the grid's 65535 go on along x.
+__device__ __forceinline__ void decode_item(const DecodeParams& p, int& hk, int& b, int& split) {
+  hk = blockIdx.x;
+  b = blockIdx.y;
+  split = blockIdx.z;
+  if (hk >= p.Hkv) {
+    // (integer division runs on the VALU: back to a scalar, or every address
+    // that follows is computed per lane, which cost the loop a quarter)
+    const int round = __builtin_amdgcn_readfirstlane(hk / p.Hkv);
+    split += round * gridDim.z;
+    hk -= round * p.Hkv;
+  }
+}
+static dim3 decode_grid(const DecodeParams& p) {
+  const int rounds = (p.num_splits + 65534) / 65535;
+  return dim3(p.Hkv * rounds, p.B, (p.num_splits + rounds - 1) / rounds);
+}
+
 template <typename T, int DP, int G>
 __global__ __launch_bounds__(256) void fa_decode_split_kernel(const DecodeParams p) {
   using X8 = typename VecT<T>::x8;
@@ -88,13 +127,16 @@ __global__ __launch_bounds__(256) void fa_decode_split_kernel(const DecodeParams
   constexpr int TPI = NW * TPW;  // tokens per workgroup per load instruction
   constexpr int CH = 4;          // tokens per lane group between offset updates
 
-  const int split = blockIdx.x, hk = blockIdx.y, b = blockIdx.z;
+  int hk, b, split;
+  decode_item(p, hk, b, split);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane % LPT, tq = lane / LPT;
   const int seq = min(max(p.seq_lens[b], 0), min(p.max_seq_len, p.max_blocks << p.block_shift));
-  const int t0 = split * p.split_tokens;
-  const int t1 = min(seq, t0 + p.split_tokens);
+  const int st = decode_split_tokens(p, seq);
+  const int t0 = split * st;
+  if (split > 0 && t0 >= seq) return;  // uniform, before any barrier
+  const int t1 = min(seq, t0 + st);
 
   __shared__ int s_blk[kDecodeMaxTableSlots];
   __shared__ float st_m[NW][G], st_l[NW][G];
@@ -129,28 +171,39 @@ __global__ __launch_bounds__(256) void fa_decode_split_kernel(const DecodeParams
     for (int e = 0; e < 8; ++e) acc[g][e] = 0.f;
   }
 
-  const T* kbase = (const T*)p.kc + (int64_t)hk * p.skh + 8 * c;
-  const T* vbase = (const T*)p.vc + (int64_t)hk * p.svh + 8 * c;
-  const bool col_ok = 8 * c < p.D;
+  // Rows that do not exist (tokens past the split, block ids outside the cache,
+  // columns past D) read as zero: their loads go to a row that does exist and
+  // are masked on use. A branch around each load instead made the compiler wait
+  // for it at the join wherever its registers differed there.
+  const bool col_ok = 8 * c < p.D, any = p.num_blocks > 0;
+  const int col = col_ok ? 8 * c : 0;
+  const T* kbase = any ? (const T*)p.kc + (int64_t)hk * p.skh + col : (const T*)p.q;
+  const T* vbase = any ? (const T*)p.vc + (int64_t)hk * p.svh + col : (const T*)p.q;
   const int bmask = (1 << p.block_shift) - 1;
 
   // Every lane group (wave, tq) walks its own tokens in chunks of CH; the
   // loads of the next chunk are in flight while the current one is used.
-  auto load_chunk = [&](int tb, u32x4* kr, u32x4* vr) {
+  auto load_chunk = [&](int tb, u32x4* kr, u32x4* vr, bool* ok) {
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
-      const int t = tb + u * TPI;
-      kr[u] = u32x4{0, 0, 0, 0};
-      vr[u] = u32x4{0, 0, 0, 0};
-      const int blk = t < t1 ? s_blk[(t >> p.block_shift) - first_slot] : -1;
-      if (t < t1 && col_ok && (unsigned)blk < (unsigned)p.num_blocks) {
-        const int slot = t & bmask;
-        kr[u] = __builtin_nontemporal_load((const u32x4*)(kbase + (int64_t)blk * p.skb + (int64_t)slot * p.sks));
-        vr[u] = __builtin_nontemporal_load((const u32x4*)(vbase + (int64_t)blk * p.svb + (int64_t)slot * p.svs));
-      }
+      const int t = tb + u * TPI, tc = min(t, t1 - 1);
+      const int blk = s_blk[(tc >> p.block_shift) - first_slot];
+      const bool in = (unsigned)blk < (unsigned)p.num_blocks;
+      const int slot = in ? tc & bmask : 0, row = in ? blk : 0;
+      kr[u] = __builtin_nontemporal_load((const u32x4*)(kbase + (int64_t)row * p.skb + (int64_t)slot * p.sks));
+      vr[u] = __builtin_nontemporal_load((const u32x4*)(vbase + (int64_t)row * p.svb + (int64_t)slot * p.svs));
+      ok[u] = in && col_ok && t < t1;
     }
+    __builtin_amdgcn_sched_barrier(0);
   };
-  auto use_chunk = [&](int tb, const u32x4* kr, const u32x4* vr) {
+  auto use_chunk = [&](int tb, u32x4* kr, u32x4* vr, const bool* in) {
+#pragma unroll
+    for (int u = 0; u < CH; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        kr[u][e] = in[u] ? kr[u][e] : 0u;
+        vr[u][e] = in[u] ? vr[u][e] : 0u;
+      }
     float s[CH][G];
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
@@ -175,6 +228,9 @@ __global__ __launch_bounds__(256) void fa_decode_split_kernel(const DecodeParams
         m[g] = mx;
       }
     }
+    float mu[G];  // (a lane group that has seen no token keeps m = -inf)
+#pragma unroll
+    for (int g = 0; g < G; ++g) mu[g] = m[g] == -INFINITY ? 0.f : m[g];
     // P V two tokens at a time on v_dot2 (each pair of V rows interleaved by
     // v_perm_b32, shared by the G heads), with p rounded to the input dtype
     // as the forward's PV operands are. The row sums stay fp32: the offset
@@ -191,8 +247,8 @@ __global__ __launch_bounds__(256) void fa_decode_split_kernel(const DecodeParams
       }
 #pragma unroll
       for (int g = 0; g < G; ++g) {
-        const float p0 = fast_exp2(s[u][g] - m[g]);  // exp2(-inf) = 0 past the end
-        const float p1 = fast_exp2(s[u + 1][g] - m[g]);
+        const float p0 = fast_exp2(s[u][g] - mu[g]);  // exp2(-inf) = 0 past the end
+        const float p1 = fast_exp2(s[u + 1][g] - mu[g]);
         const T2 pp = T2{(T)p0, (T)p1};
         l[g] += p0 + p1;
 #pragma unroll
@@ -201,17 +257,25 @@ __global__ __launch_bounds__(256) void fa_decode_split_kernel(const DecodeParams
     }
   };
   u32x4 ka[CH], va[CH], kb[CH], vb[CH];
-  int tb = t0 + wave * TPW + tq;
-  if (tb < t1) load_chunk(tb, ka, va);
-  while (tb < t1) {
-    const int tn = tb + CH * TPI;
-    if (tn < t1) load_chunk(tn, kb, vb);
-    use_chunk(tb, ka, va);
-    if (tn >= t1) break;
-    const int tn2 = tn + CH * TPI;
-    if (tn2 < t1) load_chunk(tn2, ka, va);
-    use_chunk(tn, kb, vb);
-    tb = tn2;
+  bool oa[CH], ob[CH];
+  // Wave-uniform, with a chunk's loads always issued (rows past the split are
+  // the last one again, from cache): the wait before a chunk's use then counts
+  // the next chunk's loads as still in flight. Where the compiler could not
+  // know, it waited for all of them: 32 sequences of 1024..8192 tokens 136 -> 126
+  // us (5.3 TB/s), 16 of 500 22.5 -> 16.3.
+  int tw = t0 + wave * TPW;  // the wave's first token
+  if (tw < t1) {
+    load_chunk(tw + tq, ka, va, oa);
+    for (;;) {
+      const int tn = tw + CH * TPI, tn2 = tn + CH * TPI;
+      load_chunk(tn + tq, kb, vb, ob);
+      use_chunk(tw + tq, ka, va, oa);
+      if (tn >= t1) break;
+      load_chunk(tn2 + tq, ka, va, oa);
+      use_chunk(tn + tq, kb, vb, ob);
+      if (tn2 >= t1) break;
+      tw = tn2;
+    }
   }
 
   // Merge the wave's TPW lane groups (lanes with equal c) with shuffles, then
@@ -261,7 +325,7 @@ __global__ __launch_bounds__(256) void fa_decode_split_kernel(const DecodeParams
     const int h = hk * G + g;
     const float on = L > 0.f ? O / L : 0.f;
     const float lse2 = L > 0.f ? M + __log2f(L) : -INFINITY;  // log2 units
-    if (p.num_splits == 1) {
+    if (seq <= st) {  // the sequence's only split
       if (d < p.D) ((T*)p.o)[(int64_t)b * p.sob + (int64_t)h * p.soh + d] = (T)on;
       if (d == 0 && p.lse != nullptr) p.lse[(int64_t)b * p.slb + (int64_t)h * p.slh] = lse2 * kDecLn2;
     } else {
@@ -303,14 +367,17 @@ __global__ __launch_bounds__(256) void fa_decode_mfma_kernel(const DecodeParams 
   __shared__ float st_m[NW][32], st_l[NW][32], st_le[NW][32];
   LDS_AS char* smem = (LDS_AS char*)smem_raw;
 
-  const int split = blockIdx.x, hk = blockIdx.y, b = blockIdx.z;
+  int hk, b, split;
+  decode_item(p, hk, b, split);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hh = lane >> 5;
   const int G = p.Hq / p.Hkv;
   const int seq = min(max(p.seq_lens[b], 0), min(p.max_seq_len, p.max_blocks << p.block_shift));
-  const int t0 = split * p.split_tokens;
-  const int t1 = min(seq, t0 + p.split_tokens);
+  const int st = decode_split_tokens(p, seq);
+  const int t0 = split * st;
+  if (split > 0 && t0 >= seq) return;  // uniform, before any barrier
+  const int t1 = min(seq, t0 + st);
   const int ntile = t1 > t0 ? (t1 - t0 + BT - 1) / BT : 0;
   const int D = p.D;
   const float sl2 = p.scale_log2;
@@ -493,7 +560,7 @@ __global__ __launch_bounds__(256) void fa_decode_mfma_kernel(const DecodeParams 
     const int h = hk * G + g;
     const float on = L > 0.f ? O / L : 0.f;
     const float lse2 = LE > 0.f ? M + __log2f(LE) : -INFINITY;  // log2 units
-    if (p.num_splits == 1) {
+    if (seq <= st) {  // the sequence's only split
       if (d < p.D) ((T*)p.o)[(int64_t)b * p.sob + (int64_t)h * p.soh + d] = (T)on;
       if (d == 0 && p.lse != nullptr) p.lse[(int64_t)b * p.slb + (int64_t)h * p.slh] = lse2 * kDecLn2;
     } else {
@@ -520,7 +587,9 @@ __global__ __launch_bounds__(DP) void fa_decode_combine_kernel(const DecodeParam
   const int h = blockIdx.x, b = blockIdx.y, d = threadIdx.x;
   const int64_t row0 = ((int64_t)b * p.Hq + h) * p.num_splits;
   const int seq = min(max(p.seq_lens[b], 0), min(p.max_seq_len, p.max_blocks << p.block_shift));
-  const int ns = min(p.num_splits, (seq + p.split_tokens - 1) / p.split_tokens);
+  const int st = decode_split_tokens(p, seq);
+  if (seq <= st) return;  // one split, already in o
+  const int ns = (seq + st - 1) / st;
   float M = -INFINITY, W = 0.f, O = 0.f;
   for (int c0 = 0; c0 < ns; c0 += kCombineBatch) {
     const int cn = min(kCombineBatch, ns - c0);
@@ -564,7 +633,7 @@ __global__ __launch_bounds__(DP) void fa_decode_combine_kernel(const DecodeParam
 
 template <typename T, int DP, int G>
 static hipError_t launch_decode(const DecodeParams& p, hipStream_t s) {
-  hipLaunchKernelGGL((fa_decode_split_kernel<T, DP, G>), dim3(p.num_splits, p.Hkv, p.B), dim3(256), 0, s, p);
+  hipLaunchKernelGGL((fa_decode_split_kernel<T, DP, G>), decode_grid(p), dim3(256), 0, s, p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || p.num_splits == 1) return e;
   hipLaunchKernelGGL((fa_decode_combine_kernel<T, DP>), dim3(p.Hq, p.B), dim3(DP), 0, s, p);
@@ -584,7 +653,7 @@ static hipError_t dispatch_decode_g(const DecodeParams& p, hipStream_t s) {
 
 template <typename T, int DP>
 static hipError_t launch_decode_mfma(const DecodeParams& p, hipStream_t s) {
-  hipLaunchKernelGGL((fa_decode_mfma_kernel<T, DP>), dim3(p.num_splits, p.Hkv, p.B), dim3(256), 0, s, p);
+  hipLaunchKernelGGL((fa_decode_mfma_kernel<T, DP>), decode_grid(p), dim3(256), 0, s, p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || p.num_splits == 1) return e;
   hipLaunchKernelGGL((fa_decode_combine_kernel<T, DP>), dim3(p.Hq, p.B), dim3(DP), 0, s, p);

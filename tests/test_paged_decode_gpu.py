@@ -12,6 +12,8 @@ block and tile boundaries, shuffled physical blocks, split and unsplit
 launches, the device-side clamp of seq_lens to max_seq_len, and 20 seeded
 random batches over all of these.
 """
+import math
+
 import pytest
 import torch
 
@@ -147,3 +149,37 @@ def test_decode_random_batches(gpu, seed):
     print(f"case {label} lens={lens}", flush=True)
     q, kc, vc, table, sl = _make_case(lens, hq, hkv, d, bs, dtype, "cuda", 500 + seed)
     _check(q, kc, vc, table, sl, label)
+
+
+@pytest.mark.parametrize("heads", [(8, 2), (4, 4), (14, 2)])
+@pytest.mark.parametrize("limit", [None, 600, 4096, 16384])
+def test_decode_limit_does_not_change_results(gpu, heads, limit):
+    """Sequences split by their own lengths under a larger limit: lengths around
+    the split sizes (0, one token, the edges of 128, 256 and 512), NaN in the
+    cache rows that no sequence holds; each result is float64's whatever the limit sizes the grid for."""
+    print(f"case decode limit {limit} heads={heads}", flush=True)
+    lens = [0, 1, 127, 128, 129, 255, 257, 511, 513, 577]
+    q, kc, vc, bt, sl = (t.to(gpu) for t in _make_case(lens, heads[0], heads[1], 64, 16, torch.bfloat16, gpu, seed=7))
+    free = torch.ones(kc.shape[0] + 1, dtype=torch.bool, device=gpu)
+    for b, n in enumerate(lens):
+        free[bt[b, :(n + 15) // 16].long()] = False
+    kc[free[:-1]] = float("nan")
+    vc[free[:-1]] = float("nan")
+    for b, n in enumerate(lens):
+        if n % 16:  # rows of the last block past the sequence
+            last = bt[b, n // 16].long()
+            kc[last, n % 16:] = float("nan")
+            vc[last, n % 16:] = float("nan")
+    want, lse_want = paged_attention_decode(q, kc, vc, bt, sl, max_seq_len=577, return_lse=True)
+    got, lse = paged_attention_decode(q, kc, vc, bt, sl, max_seq_len=limit, return_lse=True)
+    torch.cuda.synchronize()
+    assert got.isfinite().all() and (got[0] == 0).all() and (lse[0] == -math.inf).all()
+    assert (got.float() - want.float()).abs().max() < 2e-2
+    torch.testing.assert_close(lse[1:], lse_want[1:], atol=1e-4, rtol=1e-5)
+    for b, n in enumerate(lens[1:], 1):
+        rows = torch.arange(n, device=gpu)
+        slot = bt[b].long()[rows // 16] * 16 + rows % 16
+        k, v = (c.flatten(0, 1)[slot].double().repeat_interleave(heads[0] // heads[1], 1) for c in (kc, vc))
+        s = (q[b].double() * k).sum(2).T / 8.0
+        assert (got[b].double() - (s.softmax(1).T[:, :, None] * v).sum(0)).abs().max() < 2e-2, n
+        assert (lse[b].double() - s.logsumexp(1)).abs().max() < 1e-3, n
