@@ -541,7 +541,7 @@ int lsfa_gemv_check(const lsfa_gemv_args* args);
 /* Workspace bytes lsfa_gemv needs (m, k and n matter); no GPU work. */
 int lsfa_gemv_workspace_size(const lsfa_gemv_args* args, uint64_t* bytes);
 
-/* y = x @ w for m <= 8 rows (see lsfa_gemv_args): one launch on the stream,
+/* y = x @ w for m <= 32 rows (see lsfa_gemv_args): one launch on the stream,
  * a K-split pass over w whose last-arriving workgroup per column block sums
  * the splits (in split order: deterministic) and rounds once into y. */
 int lsfa_gemv(const lsfa_gemv_args* args, void* stream);
