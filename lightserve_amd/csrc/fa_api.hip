@@ -674,7 +674,7 @@ bool gemv_uses_mfma(const lsfa_gemv_group_args* a) {
   if (a->x_gate && (a->x_gate_stride % 8 != 0 || !aligned16(a->x_gate))) return false;
   long long n = 0;
   for (int i = 0; i < a->count; ++i) {
-    if (a->n[i] % 128 != 0) return false;
+    if (a->n[i] % 128 != 0 || a->w_stride[i] > (1 << 25)) return false;  // 32 rows of W in 31 bits of byte offset
     n += a->n[i];
   }
   return n / 128 <= LSFA_GEMV_COUNTER_BYTES / 64;
@@ -813,6 +813,13 @@ int lsfa_gemv_group_workspace_size(const lsfa_gemv_group_args* a, uint64_t* byte
   return ok();
 }
 
+// Rows of x, stride elements apart, whose byte offsets stay below 2^31
+// (above 32 rows the stride is at most 2^23 and a launch takes 64 at a time).
+static int gemv_mfma_rows(int64_t stride) {
+  if (stride <= (1 << 23)) return 1 << 30;
+  return (int)(1 + (0x7fffffffLL - 128) / (2 * stride));
+}
+
 static int run_gemv_group(const lsfa_gemv_group_args* a, bool mfma, const GemvSplit& g, long long N, void* stream) {
   lsfa::GemvParams p;
   memset(&p, 0, sizeof(p));
@@ -843,8 +850,21 @@ static int run_gemv_group(const lsfa_gemv_group_args* a, bool mfma, const GemvSp
   p.sx = a->x_stride;
   p.M = a->m; p.K = a->k; p.N = (int)N;
   p.kc = g.kc; p.splits = g.splits;
-  hipError_t e = mfma ? lsfa::gemv_mfma(p, a->dtype == LSFA_DTYPE_BF16, reinterpret_cast<hipStream_t>(stream))
-                      : lsfa::gemv(p, a->dtype == LSFA_DTYPE_BF16, reinterpret_cast<hipStream_t>(stream));
+  hipError_t e = hipSuccess;
+  if (!mfma) {
+    e = lsfa::gemv(p, a->dtype == LSFA_DTYPE_BF16, reinterpret_cast<hipStream_t>(stream));
+  } else {
+    // The kernel's offsets of x rows (and of the gate's) are 31 bits of bytes:
+    // rows further apart (the last token of each long sequence) go in several launches.
+    const int most = gemv_mfma_rows(std::max(a->x_stride, a->x_gate ? a->x_gate_stride : 0));
+    for (int m = 0; m < a->m && e == hipSuccess; m += most) {
+      p.M = std::min(most, a->m - m);
+      e = lsfa::gemv_mfma(p, a->dtype == LSFA_DTYPE_BF16, reinterpret_cast<hipStream_t>(stream));
+      p.x = static_cast<const char*>(p.x) + (int64_t)most * a->x_stride * 2;
+      if (p.xg) p.xg = static_cast<const char*>(p.xg) + (int64_t)most * a->x_gate_stride * 2;
+      for (int i = 0; i < a->count; ++i) p.y[i] = static_cast<char*>(p.y[i]) + (int64_t)most * a->y_stride[i] * 2;
+    }
+  }
   if (e != hipSuccess) return fail(LSFA_ERR_LAUNCH, "gemv launch failed: %s", hipGetErrorString(e));
   return ok();
 }

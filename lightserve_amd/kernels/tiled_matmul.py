@@ -64,6 +64,7 @@ AUTO_MAX_ROWS = 2    # rows that every product (and the fused norm / SwiGLU inpu
 # matrix a multiple of 128 wide, run on the library's MFMA kernel.
 MFMA_AUTO_ROWS = 32
 MFMA_AUTO_MAX_COLS = 128 * (_lib.GEMV_COUNTER_BYTES // 64)
+MFMA_MAX_STRIDE = 1 << 25  # of W's rows: 32 of them in a 31-bit byte offset
 # Above MFMA_AUTO_ROWS rows, lsfa_gemm_group runs launches of this many tiles of
 # 64 x 128 whose K is at least GEMM_MIN_K or which group several matrices (a
 # short K alone: 2048 -> 2048 at 128 rows 15.7 us against hipBLASLt's 12.6; few
@@ -229,15 +230,15 @@ def _library_only(*tensors) -> bool:
 def _mfma_ok(a: torch.Tensor, bs) -> bool:
     """Whether the MFMA kernel takes these products (beyond _skinny_ok)."""
     return (AUTO_MAX_ROWS < a.shape[0] <= MFMA_AUTO_ROWS and sum(b.shape[1] for b in bs) <= MFMA_AUTO_MAX_COLS
-            and all(_skinny_ok(a, b) and b.shape[1] % 128 == 0 for b in bs)
-            and a.shape[1] % 8 == 0 and _rows_addressable(a))
+            and all(_skinny_ok(a, b) and b.shape[1] % 128 == 0 and b.stride(0) <= MFMA_MAX_STRIDE for b in bs)
+            and a.shape[1] % 8 == 0 and _rows_addressable(a) and a.stride(0) >= a.shape[1])
 
 
 def _auto_skinny(a: torch.Tensor, bs) -> bool:
     """Whether matmul / matmul_shared_input route these products to the
     skinny kernels (see AUTO_MAX_ROWS and MFMA_AUTO_*)."""
     if not (len(bs) <= _lib.GEMV_MAX_GROUP and a.ndim == 2 and a.is_cuda and all(
-            b.ndim == 2 and b.is_cuda and b.dtype == a.dtype and b.shape[0] == a.shape[1] for b in bs)):
+            b.ndim == 2 and b.device == a.device and b.dtype == a.dtype and b.shape[0] == a.shape[1] for b in bs)):
         return False
     if a.shape[0] <= AUTO_MAX_ROWS:
         return all(_skinny_ok(a, b, AUTO_MAX_ROWS) for b in bs)
@@ -258,8 +259,9 @@ def _gemm_ok(a: torch.Tensor, bs) -> bool:
     return (len(bs) <= _lib.GEMV_MAX_GROUP and a.ndim == 2 and a.is_cuda and a.shape[0] > MFMA_AUTO_ROWS
             and a.dtype in (torch.bfloat16, torch.float16) and a.shape[1] > 0 and a.shape[1] % 8 == 0
             and _rows_addressable(a) and a.shape[1] <= a.stride(0) <= 1 << 23 and all(
-                b.ndim == 2 and b.is_cuda and b.dtype == a.dtype and b.shape[0] == a.shape[1] and b.shape[1] % 128 == 0
-                and b.shape[1] > 0 and _rows_addressable(b) and b.stride(0) >= b.shape[1] for b in bs)
+                b.ndim == 2 and b.device == a.device and b.dtype == a.dtype and b.shape[0] == a.shape[1]
+                and b.shape[1] % 128 == 0 and b.shape[1] > 0 and _rows_addressable(b)
+                and b.shape[1] <= b.stride(0) <= MFMA_MAX_STRIDE for b in bs)
             and GEMM_MIN_TILES <= sum(b.shape[1] for b in bs) // 128 * ((a.shape[0] + 63) // 64) <= GEMM_MAX_TILES
             and (len(bs) > 1 or a.shape[1] >= GEMM_MIN_K)
             and not _library_only(a, *bs))
@@ -286,9 +288,10 @@ def swiglu_matmul(gate: torch.Tensor, up: torch.Tensor, b: torch.Tensor) -> torc
     """matmul(F.silu(gate) * up, b), the activation folded into the skinny
     kernels' load of their input when the product qualifies for them."""
     if (gate.ndim == 2 and gate.shape == up.shape and gate.dtype == up.dtype == b.dtype and gate.is_cuda
-            and up.is_cuda and b.is_cuda and b.ndim == 2 and b.shape[0] == up.shape[1] and gate.stride(1) == 1
-            and (_skinny_ok(up, b, AUTO_MAX_ROWS) or (
-                _mfma_ok(up, [b]) and _rows_addressable(gate) and not _library_only(gate, up, b)))):
+            and up.device == gate.device and b.device == gate.device and b.ndim == 2 and b.shape[0] == up.shape[1]
+            and gate.stride(1) == 1 and (_skinny_ok(up, b, AUTO_MAX_ROWS) or (
+                _mfma_ok(up, [b]) and _rows_addressable(gate) and gate.stride(0) >= gate.shape[1]
+                and not _library_only(gate, up, b)))):
         return skinny_matmul_group(up, [b], gate=gate)[0]
     return matmul(torch.nn.functional.silu(gate) * up, b)
 

@@ -791,3 +791,29 @@ def test_packed_structs_fill_every_field_in_order():
             v = getattr(_lib.pack(cls, *values), name)
             got += list(v) if hasattr(v, "__len__") else [v]
         assert got == values, cls.__name__
+
+
+def test_matmul_routes_need_one_device_and_plain_rows():
+    """The routes to the skinny kernels, on stand-ins for tensors: operands on
+    two GPUs, repeated rows and W rows too far apart stay with torch."""
+    from types import SimpleNamespace
+    from lightserve_amd.kernels import tiled_matmul as tm
+
+    def tensor(rows, cols, device="cuda:0", stride=None):
+        strides = (cols if stride is None else stride, 1)
+        return SimpleNamespace(shape=(rows, cols), ndim=2, is_cuda=True, device=torch.device(device), requires_grad=False,
+                               dtype=torch.bfloat16, data_ptr=lambda: 4096,
+                               stride=lambda i=None: strides if i is None else strides[i])
+
+    library_only, tm._library_only = tm._library_only, lambda *t: False
+    try:
+        for m in (2, 3, 8, 32):
+            assert tm._auto_skinny(tensor(m, 4096), [tensor(4096, 256)])
+            assert not tm._auto_skinny(tensor(m, 4096), [tensor(4096, 256, "cuda:1")])
+        assert tm._gemm_ok(tensor(64, 4096), [tensor(4096, 4096)])
+        assert not tm._gemm_ok(tensor(64, 4096), [tensor(4096, 4096, "cuda:1")])
+        for m, ok in ((8, tm._auto_skinny), (32, tm._auto_skinny), (64, tm._gemm_ok)):
+            assert not ok(tensor(m, 4096, stride=0), [tensor(4096, 4096)])
+            assert not ok(tensor(m, 4096), [tensor(4096, 4096, stride=(1 << 25) + 8)])
+    finally:
+        tm._library_only = library_only

@@ -435,6 +435,34 @@ def test_gemm_group_row_blocks(M, K, ns, dtype):
     assert entry is None or (entry.buf[:_lib.GEMV_COUNTER_BYTES] == 0).all()
 
 
+def test_rows_far_apart():
+    """x rows (and a gate's) more than 31 bits of byte offset apart, as the last
+    tokens of long sequences are: the same bits as from packed rows."""
+    from lightserve_amd.kernels.tiled_matmul import swiglu_matmul
+    print("case rows far apart", flush=True)
+    M, K, N, stride = 9, 512, 256, (1 << 27) + 8
+    g = torch.Generator(device="cuda").manual_seed(9)
+    far = torch.empty((M - 1) * stride + K, device="cuda", dtype=torch.bfloat16).as_strided((M, K), (stride, 1))
+    near, gate = (torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16) for _ in range(2))
+    w = (torch.randn(K, N, device="cuda", generator=g) / K ** 0.5).to(torch.bfloat16)
+    far.copy_(near)
+    assert torch.equal(matmul(far, w), matmul(near, w))
+    assert torch.equal(swiglu_matmul(gate, far, w), swiglu_matmul(gate, near, w))
+    assert torch.equal(swiglu_matmul(far, gate, w), swiglu_matmul(near, gate, w))
+
+
+@pytest.mark.parametrize("M", [3, 16, 64])
+def test_repeated_rows(M):
+    """One row expanded (row stride 0), as x or as the gate: torch's operators take it."""
+    from lightserve_amd.kernels.tiled_matmul import swiglu_matmul
+    x = torch.randn(1, 512, device="cuda").to(torch.bfloat16)
+    full = torch.randn(M, 512, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(512, 256, device="cuda") / 512 ** 0.5).to(torch.bfloat16)
+    _assert_one_rounding(matmul(x.expand(M, 512), w), x.expand(M, 512), w)
+    for gate, up in ((x.expand(M, 512), full), (full, x.expand(M, 512))):
+        _assert_one_rounding(swiglu_matmul(gate, up, w), torch.nn.functional.silu(gate) * up, w)
+
+
 def test_gemm_route(monkeypatch):
     """matmul and matmul_shared_input take lsfa_gemm_group inside its range and
     torch's GEMM outside it or where a gradient is recorded."""
