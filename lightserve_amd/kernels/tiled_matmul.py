@@ -216,15 +216,18 @@ def skinny_matmul_group(a: torch.Tensor, bs, outs=None, gate: torch.Tensor = Non
 def _library_only(*tensors) -> bool:
     """Whether a call on these tensors has to go through torch's own operators:
     a gradient is recorded (reverse or forward mode), a subclass, mode or
-    transform looks at the operators, or autocast may change their types."""
+    transform looks at the operators, or autocast may change their types. To be
+    asked before anything reads an address: what a transform or tracer passes
+    has none."""
+    if torch.compiler.is_compiling():
+        return True
     grad = torch.is_grad_enabled()
     for t in tensors:
         kind = type(t)
         if (kind is not torch.Tensor and kind is not torch.nn.Parameter) or (grad and t.requires_grad):
             return True
     return (forward_ad._current_level >= 0 or _interpreter() is not None or _dispatch_modes() > 0
-            or _function_modes() > 0 or _tracing() is not None or torch.is_autocast_enabled("cuda")
-            or torch.compiler.is_compiling())
+            or _function_modes() > 0 or _tracing() is not None or torch.is_autocast_enabled("cuda"))
 
 
 def _mfma_ok(a: torch.Tensor, bs) -> bool:
@@ -235,14 +238,14 @@ def _mfma_ok(a: torch.Tensor, bs) -> bool:
 
 
 def _auto_skinny(a: torch.Tensor, bs) -> bool:
-    """Whether matmul / matmul_shared_input route these products to the
-    skinny kernels (see AUTO_MAX_ROWS and MFMA_AUTO_*)."""
+    """Whether matmul / matmul_shared_input route these products, which are not
+    _library_only, to the skinny kernels (see AUTO_MAX_ROWS and MFMA_AUTO_*)."""
     if not (len(bs) <= _lib.GEMV_MAX_GROUP and a.ndim == 2 and a.is_cuda and all(
             b.ndim == 2 and b.device == a.device and b.dtype == a.dtype and b.shape[0] == a.shape[1] for b in bs)):
         return False
     if a.shape[0] <= AUTO_MAX_ROWS:
         return all(_skinny_ok(a, b, AUTO_MAX_ROWS) for b in bs)
-    return _mfma_ok(a, bs) and not _library_only(a, *bs)
+    return _mfma_ok(a, bs)
 
 
 def _skinny_run(a: torch.Tensor, bs):
@@ -255,7 +258,8 @@ def _skinny_run(a: torch.Tensor, bs):
 
 
 def _gemm_ok(a: torch.Tensor, bs) -> bool:
-    """Whether lsfa_gemm_group takes these products and is the faster route."""
+    """Whether lsfa_gemm_group takes these products, which are not
+    _library_only, and is the faster route."""
     return (len(bs) <= _lib.GEMV_MAX_GROUP and a.ndim == 2 and a.is_cuda and a.shape[0] > MFMA_AUTO_ROWS
             and a.dtype in (torch.bfloat16, torch.float16) and a.shape[1] > 0 and a.shape[1] % 8 == 0
             and _rows_addressable(a) and a.shape[1] <= a.stride(0) <= 1 << 23 and all(
@@ -263,8 +267,7 @@ def _gemm_ok(a: torch.Tensor, bs) -> bool:
                 and b.shape[1] % 128 == 0 and b.shape[1] > 0 and _rows_addressable(b)
                 and b.shape[1] <= b.stride(0) <= MFMA_MAX_STRIDE for b in bs)
             and GEMM_MIN_TILES <= sum(b.shape[1] for b in bs) // 128 * ((a.shape[0] + 63) // 64) <= GEMM_MAX_TILES
-            and (len(bs) > 1 or a.shape[1] >= GEMM_MIN_K)
-            and not _library_only(a, *bs))
+            and (len(bs) > 1 or a.shape[1] >= GEMM_MIN_K))
 
 
 def _gemm_group(a: torch.Tensor, bs):
@@ -277,10 +280,11 @@ def _gemm_group(a: torch.Tensor, bs):
 def matmul_shared_input(a: torch.Tensor, bs):
     """[matmul(a, b) for b in bs]: one grouped launch when the products
     qualify for the library's kernels together, else one matmul each."""
-    if _auto_skinny(a, bs):
-        return _skinny_run(a, bs)
-    if _gemm_ok(a, bs):
-        return _gemm_group(a, bs)
+    if a.ndim == 2 and (a.shape[0] <= AUTO_MAX_ROWS or not _library_only(a, *bs)):
+        if _auto_skinny(a, bs):
+            return _skinny_run(a, bs)
+        if _gemm_ok(a, bs):
+            return _gemm_group(a, bs)
     return [matmul(a, b) for b in bs]
 
 
@@ -289,9 +293,9 @@ def swiglu_matmul(gate: torch.Tensor, up: torch.Tensor, b: torch.Tensor) -> torc
     kernels' load of their input when the product qualifies for them."""
     if (gate.ndim == 2 and gate.shape == up.shape and gate.dtype == up.dtype == b.dtype and gate.is_cuda
             and up.device == gate.device and b.device == gate.device and b.ndim == 2 and b.shape[0] == up.shape[1]
+            and (gate.shape[0] <= AUTO_MAX_ROWS or not _library_only(gate, up, b))
             and gate.stride(1) == 1 and (_skinny_ok(up, b, AUTO_MAX_ROWS) or (
-                _mfma_ok(up, [b]) and _rows_addressable(gate) and gate.stride(0) >= gate.shape[1]
-                and not _library_only(gate, up, b)))):
+                _mfma_ok(up, [b]) and _rows_addressable(gate) and gate.stride(0) >= gate.shape[1]))):
         return skinny_matmul_group(up, [b], gate=gate)[0]
     return matmul(torch.nn.functional.silu(gate) * up, b)
 
@@ -337,8 +341,9 @@ def matmul(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     assert a.shape[1] == b.shape[0], f"inner dims must match: a is {tuple(a.shape)}, b is {tuple(b.shape)}"
     assert a.is_cuda and b.is_cuda, "the gfx950 path needs GPU tensors"
     assert a.dtype == b.dtype, f"dtype mismatch: a={a.dtype} b={b.dtype}"
-    if _auto_skinny(a, [b]):
-        return _skinny_run(a, [b])[0]
-    if _gemm_ok(a, [b]):
-        return _gemm_group(a, [b])[0]
+    if a.shape[0] <= AUTO_MAX_ROWS or not _library_only(a, b):
+        if _auto_skinny(a, [b]):
+            return _skinny_run(a, [b])[0]
+        if _gemm_ok(a, [b]):
+            return _gemm_group(a, [b])[0]
     return torch.matmul(a, b)

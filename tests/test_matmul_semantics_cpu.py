@@ -1,0 +1,92 @@
+"""matmul, matmul_shared_input and swiglu_matmul where torch's own operators
+have to see the call: transforms, tracers and subclasses, whose tensors have no
+address to read.
+
+Without a GPU: the module's source with its GPU tests turned into CPU tests, so
+that the routes are decided on CPU tensors, and every launch turned into a
+failure."""
+import sys
+import types
+import warnings
+
+import pytest
+import torch
+from torch.func import grad, jvp, vmap
+
+from lightserve_amd.kernels import tiled_matmul
+
+ROWS = [1, 2, 3, 9, 16, 33, 64, 512, 5000]
+ROUTED = [m for m in ROWS if m > tiled_matmul.AUTO_MAX_ROWS]
+
+
+@pytest.fixture
+def tm(monkeypatch):
+    path = tiled_matmul.__file__
+    with open(path) as f:
+        source = f.read().replace(".is_cuda", ".is_cpu")
+    module = types.ModuleType("lightserve_amd.kernels.tiled_matmul_on_cpu")
+    module.__package__, module.__file__ = "lightserve_amd.kernels", path
+    monkeypatch.setitem(sys.modules, module.__name__, module)
+    exec(compile(source, path, "exec"), module.__dict__)
+
+    def launch(*args, **kwargs):
+        raise AssertionError("routed to a kernel")
+    module._run_group = launch
+    return module
+
+
+def _calls(tm, x, w):
+    return [lambda a: tm.matmul(a, w), lambda a: tm.matmul_shared_input(a, [w, w])[1],
+            lambda a: tm.swiglu_matmul(a, x, w), lambda a: tm.swiglu_matmul(x, a, w)]
+
+
+def _operands(m, k=4096, n=256):
+    g = torch.Generator().manual_seed(m)
+    return (torch.randn(m, k, generator=g).to(torch.bfloat16), torch.randn(m, k, generator=g).to(torch.bfloat16),
+            (torch.randn(k, n, generator=g) / k ** 0.5).to(torch.bfloat16))
+
+
+def test_plain_calls_reach_the_kernels(tm):
+    """The stand-in decides as on a GPU: without a transform these are routed."""
+    for m in (1, 3, 32, 512):
+        x, y, w = _operands(m, n=4096 if m > 32 else 256)
+        for f in _calls(tm, x, w)[:2 if m > 32 else 4]:
+            with pytest.raises(AssertionError, match="routed to a kernel"):
+                f(y)
+
+
+@pytest.mark.parametrize("m", ROUTED)
+def test_transforms(tm, m):
+    x, y, w = _operands(m, 128, 128)
+    for f in _calls(tm, x, w):
+        want = f(y.clone().requires_grad_()).detach().float()
+        torch.testing.assert_close(vmap(f)(torch.stack([y, y])).float(), torch.stack([want, want]), rtol=2 ** -7, atol=1e-6)
+        assert torch.isfinite(grad(lambda a: f(a).float().sum())(y)).all()
+        assert torch.isfinite(jvp(f, (y,), (y,))[1]).all()
+
+
+@pytest.mark.parametrize("m", [16, 64, 600])
+def test_compile_traces_the_whole_call(tm, m):
+    x, y, w = _operands(m, 128, 128)
+    for f in _calls(tm, x, w):
+        torch._dynamo.reset()
+        assert torch.compile(f, backend="eager", fullgraph=True)(y).shape == (m, 128)
+
+
+@pytest.mark.parametrize("m", ROUTED)
+def test_tensors_without_storage(m):
+    """Fake GPU tensors through the module itself."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    with FakeTensorMode():
+        x = torch.empty(m, 4096, dtype=torch.bfloat16, device="cuda")
+        w = torch.empty(4096, 512, dtype=torch.bfloat16, device="cuda")
+    # an address read of a fake tensor only warns
+    always = torch.is_warn_always_enabled()
+    torch.set_warn_always(True)
+    warnings.simplefilter("error")
+    try:
+        assert tiled_matmul.matmul(x, w).shape == (m, 512)
+        assert [t.shape for t in tiled_matmul.matmul_shared_input(x, [w, w])] == [(m, 512)] * 2
+        assert tiled_matmul.swiglu_matmul(x, x, w).shape == (m, 512)
+    finally:
+        torch.set_warn_always(always)
