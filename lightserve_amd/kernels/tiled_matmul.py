@@ -216,15 +216,16 @@ def skinny_matmul_group(a: torch.Tensor, bs, outs=None, gate: torch.Tensor = Non
 def _library_only(*tensors) -> bool:
     """Whether a call on these tensors has to go through torch's own operators:
     a gradient is recorded (reverse or forward mode), a subclass, mode or
-    transform looks at the operators, or autocast may change their types. To be
-    asked before anything reads an address: what a transform or tracer passes
-    has none."""
+    transform looks at the operators, autocast may change their types, or one
+    is sparse. To be asked before anything reads an address or a stride: what a
+    transform or tracer passes has no address, a sparse tensor neither."""
     if torch.compiler.is_compiling():
         return True
     grad = torch.is_grad_enabled()
     for t in tensors:
         kind = type(t)
-        if (kind is not torch.Tensor and kind is not torch.nn.Parameter) or (grad and t.requires_grad):
+        if ((kind is not torch.Tensor and kind is not torch.nn.Parameter) or (grad and t.requires_grad)
+                or t.layout is not torch.strided):
             return True
     return (forward_ad._current_level >= 0 or _interpreter() is not None or _dispatch_modes() > 0
             or _function_modes() > 0 or _tracing() is not None or torch.is_autocast_enabled("cuda"))

@@ -1,6 +1,6 @@
 """matmul, matmul_shared_input and swiglu_matmul where torch's own operators
 have to see the call: transforms, tracers and subclasses, whose tensors have no
-address to read.
+address to read, and sparse tensors.
 
 Without a GPU: the module's source with its GPU tests turned into CPU tests, so
 that the routes are decided on CPU tensors, and every launch turned into a
@@ -90,3 +90,16 @@ def test_tensors_without_storage(m):
         assert tiled_matmul.swiglu_matmul(x, x, w).shape == (m, 512)
     finally:
         torch.set_warn_always(always)
+
+
+@pytest.mark.parametrize("layout", ["to_sparse", "to_sparse_csr", "to_sparse_csc"])
+@pytest.mark.parametrize("m", ROUTED)
+def test_sparse_weights(tm, m, layout, monkeypatch):
+    """Sparse operands are torch.matmul's (which has no bf16 sparse product on a CPU)."""
+    x, _, w = _operands(m, 128, 128)
+    w, got = getattr(w, layout)(), []
+    monkeypatch.setattr(torch, "matmul", lambda a, b: got.append((a.shape, b)))
+    tm.matmul(x, w)
+    tm.matmul_shared_input(x, [w])
+    tm.swiglu_matmul(x, x, w)
+    assert len(got) == 3 and all(shape == (m, 128) and b is w for shape, b in got)
