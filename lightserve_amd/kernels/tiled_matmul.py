@@ -51,6 +51,8 @@ import threading
 
 import torch
 from torch.autograd import forward_ad
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from .. import _lib
 
@@ -216,8 +218,9 @@ def skinny_matmul_group(a: torch.Tensor, bs, outs=None, gate: torch.Tensor = Non
 def _library_only(*tensors) -> bool:
     """Whether a call on these tensors has to go through torch's own operators:
     a gradient is recorded (reverse or forward mode), a subclass, mode or
-    transform looks at the operators, autocast may change their types, or one
-    is sparse. To be asked before anything reads an address or a stride: what a
+    transform looks at the operators, autocast to another type is on, or one
+    is sparse. (A default device is a mode too, but one that only places new
+    tensors.) To be asked before anything reads an address or a stride: what a
     transform or tracer passes has no address, a sparse tensor neither."""
     if torch.compiler.is_compiling():
         return True
@@ -228,7 +231,9 @@ def _library_only(*tensors) -> bool:
                 or t.layout is not torch.strided):
             return True
     return (forward_ad._current_level >= 0 or _interpreter() is not None or _dispatch_modes() > 0
-            or _function_modes() > 0 or _tracing() is not None or torch.is_autocast_enabled("cuda"))
+            or (_function_modes() > 0 and any(type(m) is not DeviceContext for m in _get_current_function_mode_stack()))
+            or _tracing() is not None
+            or (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != tensors[0].dtype))
 
 
 def _mfma_ok(a: torch.Tensor, bs) -> bool:

@@ -103,3 +103,34 @@ def test_sparse_weights(tm, m, layout, monkeypatch):
     tm.matmul_shared_input(x, [w])
     tm.swiglu_matmul(x, x, w)
     assert len(got) == 3 and all(shape == (m, 128) and b is w for shape, b in got)
+
+
+class _Seen(torch.overrides.TorchFunctionMode):
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        self.names.append(func.__name__)
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("m", ROUTED[:3])
+def test_modes_that_change_nothing(tm, m):
+    """A default device and autocast to the operands' own type leave the
+    kernels in place; autocast to another type and any other mode do not."""
+    x, y, w = _operands(m, n=128)
+    mode = _Seen()
+    mode.names = []
+    for f in _calls(tm, x, w):
+        with torch.device("cpu"), pytest.raises(AssertionError, match="routed to a kernel"):
+            f(y)
+        with mode:
+            f(y)
+        try:
+            torch.set_autocast_enabled("cuda", True)
+            torch.set_autocast_dtype("cuda", torch.float16)
+            f(y)
+            torch.set_autocast_dtype("cuda", torch.bfloat16)
+            with pytest.raises(AssertionError, match="routed to a kernel"):
+                f(y)
+        finally:
+            torch.set_autocast_dtype("cuda", torch.float16)
+            torch.set_autocast_enabled("cuda", False)
+    assert mode.names.count("matmul") == 5  # matmul_shared_input makes two
