@@ -20,8 +20,9 @@ LLaMA-3-8B decode projections at 8 and 32 rows (us, graph replays, weights
 that no cache holds), this kernel against hipBLASLt: q/k/v 13.5 and 16.4
 against 51.9 and 54.1, o 10.9 and 13.7 against 21.9 and 20.9, gate/up 42.3 and
 46.2 against 56.1 and 56.8, down 23.1 and 27.2 against 71.0 and 61.4, LM head
-165 and 177 against 190 and 198; so every such product goes to it, unless
-autograd, a tracer or autocast has to see the call (_library_only). The norm
+165 and 177 against 190 and 198; so every such product goes to it. Calls that
+autograd, a tracer or autocast has to see stay on torch's operators at every
+row count (_library_only). The norm
 is folded into the launch at up to 2 rows only. Above 32 rows the same kernel
 runs over blocks of 64 rows (lsfa_gemm_group) as long as the launch has at most
 one tile of 64 x 128 per CU (GEMM_*); there it beats hipBLASLt's larger tiles
@@ -286,7 +287,7 @@ def _gemm_group(a: torch.Tensor, bs):
 def matmul_shared_input(a: torch.Tensor, bs):
     """[matmul(a, b) for b in bs]: one grouped launch when the products
     qualify for the library's kernels together, else one matmul each."""
-    if a.ndim == 2 and (a.shape[0] <= AUTO_MAX_ROWS or not _library_only(a, *bs)):
+    if a.ndim == 2 and not _library_only(a, *bs):
         if _auto_skinny(a, bs):
             return _skinny_run(a, bs)
         if _gemm_ok(a, bs):
@@ -299,7 +300,7 @@ def swiglu_matmul(gate: torch.Tensor, up: torch.Tensor, b: torch.Tensor) -> torc
     kernels' load of their input when the product qualifies for them."""
     if (gate.ndim == 2 and gate.shape == up.shape and gate.dtype == up.dtype == b.dtype and gate.is_cuda
             and up.device == gate.device and b.device == gate.device and b.ndim == 2 and b.shape[0] == up.shape[1]
-            and (gate.shape[0] <= AUTO_MAX_ROWS or not _library_only(gate, up, b))
+            and not _library_only(gate, up, b)
             and gate.stride(1) == 1 and (_skinny_ok(up, b, AUTO_MAX_ROWS) or (
                 _mfma_ok(up, [b]) and _rows_addressable(gate) and gate.stride(0) >= gate.shape[1]))):
         return skinny_matmul_group(up, [b], gate=gate)[0]
@@ -322,10 +323,12 @@ def add_rmsnorm_matmul_shared_input(x, residual, weight, eps, bs, write_residual
     assert x.ndim == 2 and weight.ndim == 1 and weight.shape[0] == x.shape[1], "x [M, K] and weight [K] expected"
     M, K = x.shape
     fused = (len(bs) <= _lib.GEMV_MAX_GROUP and x.is_cuda and x.dtype in (torch.bfloat16, torch.float16)
+             and M <= AUTO_MAX_ROWS and not _library_only(x, weight, *bs, *(() if residual is None else (residual,)))
+             and weight.device == x.device and (residual is None or residual.device == x.device)
              and K % 8 == 0 and _rows_addressable(x) and weight.is_contiguous() and weight.data_ptr() % 16 == 0
              and weight.dtype == x.dtype and (residual is None or (residual.shape == x.shape and residual.dtype == x.dtype
                                                                    and _rows_addressable(residual)))
-             and all(b.ndim == 2 and b.is_cuda and b.dtype == x.dtype and b.shape[0] == K
+             and all(b.ndim == 2 and b.device == x.device and b.dtype == x.dtype and b.shape[0] == K
                      and _skinny_ok(x, b, AUTO_MAX_ROWS) for b in bs))
     if not fused:
         normed, h = (fused_add_rmsnorm(x, residual, weight, eps) if residual is not None
@@ -347,7 +350,7 @@ def matmul(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     assert a.shape[1] == b.shape[0], f"inner dims must match: a is {tuple(a.shape)}, b is {tuple(b.shape)}"
     assert a.is_cuda and b.is_cuda, "the gfx950 path needs GPU tensors"
     assert a.dtype == b.dtype, f"dtype mismatch: a={a.dtype} b={b.dtype}"
-    if a.shape[0] <= AUTO_MAX_ROWS or not _library_only(a, b):
+    if not _library_only(a, b):
         if _auto_skinny(a, [b]):
             return _skinny_run(a, [b])[0]
         if _gemm_ok(a, [b]):

@@ -16,7 +16,6 @@ from torch.func import grad, jvp, vmap
 from lightserve_amd.kernels import tiled_matmul
 
 ROWS = [1, 2, 3, 9, 16, 33, 64, 512, 5000]
-ROUTED = [m for m in ROWS if m > tiled_matmul.AUTO_MAX_ROWS]
 
 
 @pytest.fixture
@@ -48,14 +47,14 @@ def _operands(m, k=4096, n=256):
 
 def test_plain_calls_reach_the_kernels(tm):
     """The stand-in decides as on a GPU: without a transform these are routed."""
-    for m in (1, 3, 32, 512):
+    for m in (1, 2, 3, 32, 512):
         x, y, w = _operands(m, n=4096 if m > 32 else 256)
         for f in _calls(tm, x, w)[:2 if m > 32 else 4]:
             with pytest.raises(AssertionError, match="routed to a kernel"):
                 f(y)
 
 
-@pytest.mark.parametrize("m", ROUTED)
+@pytest.mark.parametrize("m", ROWS)
 def test_transforms(tm, m):
     x, y, w = _operands(m, 128, 128)
     for f in _calls(tm, x, w):
@@ -65,7 +64,7 @@ def test_transforms(tm, m):
         assert torch.isfinite(jvp(f, (y,), (y,))[1]).all()
 
 
-@pytest.mark.parametrize("m", [16, 64, 600])
+@pytest.mark.parametrize("m", [1, 16, 64, 600])
 def test_compile_traces_the_whole_call(tm, m):
     x, y, w = _operands(m, 128, 128)
     for f in _calls(tm, x, w):
@@ -73,7 +72,7 @@ def test_compile_traces_the_whole_call(tm, m):
         assert torch.compile(f, backend="eager", fullgraph=True)(y).shape == (m, 128)
 
 
-@pytest.mark.parametrize("m", ROUTED)
+@pytest.mark.parametrize("m", ROWS)
 def test_tensors_without_storage(m):
     """Fake GPU tensors through the module itself."""
     from torch._subclasses.fake_tensor import FakeTensorMode
@@ -93,7 +92,7 @@ def test_tensors_without_storage(m):
 
 
 @pytest.mark.parametrize("layout", ["to_sparse", "to_sparse_csr", "to_sparse_csc"])
-@pytest.mark.parametrize("m", ROUTED)
+@pytest.mark.parametrize("m", ROWS)
 def test_sparse_weights(tm, m, layout, monkeypatch):
     """Sparse operands are torch.matmul's (which has no bf16 sparse product on a CPU)."""
     x, _, w = _operands(m, 128, 128)
@@ -111,7 +110,7 @@ class _Seen(torch.overrides.TorchFunctionMode):
         return func(*args, **(kwargs or {}))
 
 
-@pytest.mark.parametrize("m", ROUTED[:3])
+@pytest.mark.parametrize("m", [1, 2, 3, 9, 16])
 def test_modes_that_change_nothing(tm, m):
     """A default device and autocast to the operands' own type leave the
     kernels in place; autocast to another type and any other mode do not."""
@@ -134,3 +133,37 @@ def test_modes_that_change_nothing(tm, m):
             torch.set_autocast_dtype("cuda", torch.float16)
             torch.set_autocast_enabled("cuda", False)
     assert mode.names.count("matmul") == 5  # matmul_shared_input makes two
+
+
+@pytest.mark.parametrize("m", ROWS)
+def test_gradients_are_recorded(tm, m):
+    """Every route is differentiable in each of its operands, at every row count."""
+    x, y, w = (t.requires_grad_() for t in _operands(m, 128, 128))
+    for f, leaves in zip(_calls(tm, x, w), ((y, w), (y, w), (y, x, w), (y, x, w))):
+        assert all(torch.isfinite(t).all() for t in torch.autograd.grad(f(y).float().sum(), leaves))
+
+
+@pytest.mark.parametrize("with_residual", [False, True])
+@pytest.mark.parametrize("m", [1, 2])
+def test_norm_route_asks_as_well(tm, m, with_residual, monkeypatch):
+    """The launch that folds the norm in: not where a gradient is recorded,
+    under autocast to another type, or with operands of two devices."""
+    from lightserve_amd.kernels import fused_rmsnorm_residual
+    x, y, w = _operands(m, 128, 128)
+    gain, residual = torch.ones(128, dtype=torch.bfloat16), y if with_residual else None
+    with pytest.raises(AssertionError, match="routed to a kernel"):
+        tm.add_rmsnorm_matmul_shared_input(x, residual, gain, 1e-6, [w])
+    monkeypatch.setattr(fused_rmsnorm_residual, "rmsnorm", lambda a, weight, eps: a)
+    monkeypatch.setattr(fused_rmsnorm_residual, "fused_add_rmsnorm", lambda a, r, weight, eps: (a, r))
+    (out,), _ = tm.add_rmsnorm_matmul_shared_input(x, residual, gain, 1e-6, [w.clone().requires_grad_()])
+    assert out.requires_grad
+    monkeypatch.setattr(tm, "matmul_shared_input", lambda a, bs: ["apart"])
+
+    def apart(residual=residual, gain=gain):
+        return tm.add_rmsnorm_matmul_shared_input(x, residual, gain, 1e-6, [w])[0] == ["apart"]
+    assert apart(gain=gain.to("meta")) and (not with_residual or apart(residual=y.to("meta")))
+    try:
+        torch.set_autocast_enabled("cuda", True)
+        assert torch.get_autocast_dtype("cuda") == torch.float16 and apart()
+    finally:
+        torch.set_autocast_enabled("cuda", False)

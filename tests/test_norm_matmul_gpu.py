@@ -386,7 +386,7 @@ def test_skinny_matmul_mfma_edges(M, K, N):
     assert torch.equal(skinny_matmul_group(x, [w], gate=gate)[0], skinny_matmul(act, w))
 
 
-@pytest.mark.parametrize("M", [3, 9, 32, 33])
+@pytest.mark.parametrize("M", [1, 2, 3, 9, 32, 33])
 def test_matmul_routes_keep_torch_semantics(M):
     """matmul, matmul_shared_input and swiglu_matmul at the row counts around
     the MFMA kernel's range: equal to the fp64 product, and differentiable as
