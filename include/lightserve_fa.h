@@ -535,6 +535,13 @@ int lsfa_prefill_paged_workspace_size(const lsfa_prefill_paged_args* args, uint6
 int lsfa_prefill_paged_split(const lsfa_prefill_paged_args* args, void* workspace, uint64_t workspace_bytes,
                              void* stream);
 
+/* The graph capture in progress on a stream: a number of its own for each
+ * capture, 0 where there is none. For callers that keep one workspace per
+ * stream for the skinny GEMM below: the counters that it finds at zero are only
+ * cleared in the graph if the fill was captured with it, and two graphs may
+ * run at the same time, so each capture needs a workspace and a fill of its own. */
+int lsfa_capture_id(void* stream, uint64_t* id);
+
 /* Host-only validation of skinny-GEMM arguments; never touches the GPU. */
 int lsfa_gemv_check(const lsfa_gemv_args* args);
 

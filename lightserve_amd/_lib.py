@@ -31,7 +31,7 @@ EXPORTED_SYMBOLS = ("lsfa_abi_version", "lsfa_last_error", "lsfa_fwd_check", "ls
                     "lsfa_rope_check", "lsfa_rope", "lsfa_rmsnorm_check", "lsfa_rmsnorm",
                     "lsfa_prefill_paged_check", "lsfa_prefill_paged",
                     "lsfa_prefill_paged_workspace_size", "lsfa_prefill_paged_split",
-                    "lsfa_gemv_check", "lsfa_gemv_workspace_size", "lsfa_gemv",
+                    "lsfa_capture_id", "lsfa_gemv_check", "lsfa_gemv_workspace_size", "lsfa_gemv",
                     "lsfa_gemv_group_check", "lsfa_gemv_group_workspace_size", "lsfa_gemv_group",
                     "lsfa_gemm_group_check", "lsfa_gemm_group_workspace_size", "lsfa_gemm_group",
                     "lsfa_greedy_check", "lsfa_greedy")
@@ -262,6 +262,8 @@ def load():
         for size in (lib.lsfa_gemv_group_workspace_size, lib.lsfa_gemm_group_workspace_size):
             size.restype = ctypes.c_int
             size.argtypes = [ctypes.POINTER(GemvGroupArgs), ctypes.POINTER(ctypes.c_uint64)]
+        lib.lsfa_capture_id.restype = ctypes.c_int
+        lib.lsfa_capture_id.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_uint64)]
         lib.lsfa_gemv_workspace_size.restype = ctypes.c_int
         lib.lsfa_gemv_workspace_size.argtypes = [ctypes.POINTER(GemvArgs), ctypes.POINTER(ctypes.c_uint64)]
         lib.lsfa_decode_workspace_size.restype = ctypes.c_int
@@ -337,6 +339,13 @@ def prefill_paged_workspace_size(args):
 def prefill_paged_split(args, workspace, nbytes, stream):
     _raise_on(load().lsfa_prefill_paged_split(ctypes.byref(args), ctypes.c_void_p(workspace), nbytes,
                                               ctypes.c_void_p(stream)), "lsfa_prefill_paged_split")
+
+
+def capture_id(stream):
+    """The graph capture in progress on the stream, as a number of its own; 0 for none."""
+    n = ctypes.c_uint64(0)
+    _raise_on(load().lsfa_capture_id(stream, ctypes.byref(n)), "lsfa_capture_id")
+    return n.value
 
 
 def gemv_check(args):

@@ -738,6 +738,16 @@ long long gemv_total_n(const lsfa_gemv_group_args* a) {
 
 extern "C" {
 
+int lsfa_capture_id(void* stream, uint64_t* id) {
+  if (id == nullptr) return fail(LSFA_ERR_INVALID, "id is NULL");
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long n = 0;
+  const hipError_t e = hipStreamGetCaptureInfo(reinterpret_cast<hipStream_t>(stream), &status, &n);
+  if (e != hipSuccess) return fail(LSFA_ERR_LAUNCH, "capture query failed: %s", hipGetErrorString(e));
+  *id = status == hipStreamCaptureStatusActive ? n + 1 : 0;
+  return ok();
+}
+
 int lsfa_gemv_group_check(const lsfa_gemv_group_args* a) {
   if (a == nullptr) return fail(LSFA_ERR_INVALID, "args is NULL");
   if (a->dtype != LSFA_DTYPE_FP16 && a->dtype != LSFA_DTYPE_BF16)

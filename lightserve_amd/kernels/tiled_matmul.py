@@ -40,12 +40,14 @@ LSFA_GEMV_COUNTER_BYTES) that must start at zero and that every call leaves
 at zero, so this module keeps one workspace per (device, stream), zeroes its
 counter bytes once when it is created, and reuses it for every call on that
 stream (stream order keeps the calls apart). Workspaces start at 16 MB, so
-they rarely grow. The cache is bounded: a workspace that grows is freed
-unless a graph capture used it (a captured HIP graph that recorded it keeps
-using it, so such workspaces stay until release_workspaces()), and at most
-MAX_CACHED_STREAMS streams keep one, the least recently used uncaptured entry
-going first. (A workspace first created inside a graph capture records its
-counter fill into the graph, which then clears the 256 KB on every replay.)
+they rarely grow. A graph capture gets a workspace of its own, from the
+graph's memory pool, whose fill it records: the graph clears its 256 KB of
+counters before its first product on every replay, whatever ran before it, and
+shares neither counters nor partials with eager calls or with another graph
+that may run at the same time. (Captures share a stream: torch captures on one
+default capture stream per device.) The cache is bounded: it holds one eager
+workspace and the last capture's per stream, and at most MAX_CACHED_STREAMS
+streams without a capture, the least recently used going first.
 """
 import collections
 import threading
@@ -78,12 +80,12 @@ MAX_CACHED_STREAMS = 8
 
 
 class _Entry:
-    __slots__ = ("buf", "captured", "kept")
+    __slots__ = ("buf", "captured", "graph_buf")
 
     def __init__(self):
-        self.buf = None       # the workspace in use
-        self.captured = False  # a graph capture used buf
-        self.kept = []         # smaller workspaces a captured graph may still use
+        self.buf = None        # the workspace of eager calls
+        self.captured = 0      # the last graph capture on the stream (lsfa_capture_id)
+        self.graph_buf = None  # its workspace
 
 
 # (device index, stream handle) -> _Entry, least recently used first
@@ -99,27 +101,29 @@ def _workspace(device, stream, nbytes):
 def _workspace_locked(device, stream, nbytes):
     key = (device.index, stream)
     entry = _workspaces.pop(key, None) or _Entry()
-    if entry.buf is None or entry.buf.numel() < nbytes:
-        if entry.buf is not None and entry.captured:
-            entry.kept.append(entry.buf)
-        entry.buf = torch.empty(max(nbytes, 16 << 20), dtype=torch.uint8, device=device)
-        entry.buf[:_lib.GEMV_COUNTER_BYTES].zero_()
-        entry.captured = False
-    if torch.cuda.is_current_stream_capturing():
-        entry.captured = True
+    capture = _lib.capture_id(stream) if torch.cuda.is_current_stream_capturing() else 0
+    if capture and entry.captured != capture:
+        entry.captured, entry.graph_buf = capture, None
+    buf = entry.graph_buf if capture else entry.buf
+    if buf is None or buf.numel() < nbytes:
+        buf = torch.empty(max(nbytes, 16 << 20), dtype=torch.uint8, device=device)
+        buf[:_lib.GEMV_COUNTER_BYTES].zero_()
+        if capture:
+            entry.graph_buf = buf
+        else:
+            entry.buf = buf
     _workspaces[key] = entry
     while len(_workspaces) > MAX_CACHED_STREAMS:
-        victim = next((k for k, e in _workspaces.items() if not e.captured and not e.kept), None)
+        victim = next((k for k, e in _workspaces.items() if not e.captured), None)
         if victim is None:
             break
         del _workspaces[victim]
-    return entry.buf
+    return buf
 
 
 def release_workspaces():
-    """Frees every cached skinny-GEMM workspace. Call it once no captured HIP
-    graph that ran a skinny product is alive (those graphs keep using the
-    workspaces they recorded)."""
+    """Frees every cached skinny-GEMM workspace. (Those that captured graphs
+    recorded live in the graphs' own memory pools.)"""
     with _workspaces_lock:
         _workspaces.clear()
 

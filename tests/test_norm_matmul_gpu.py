@@ -482,3 +482,51 @@ def test_gemm_route(monkeypatch):
     assert run(33, 4096, (2048,)) == 1 and run(200, 2048, (1024, 512)) == 1 and run(512, 4096, (4096,)) == 1
     assert run(48, 4096, (1024,)) == 0 and run(200, 2048, (1024,)) == 0 and run(513, 4096, (4096,)) == 0
     assert run(64, 4096, (4096,), grad=True) == 0 and run(32, 4096, (4096,)) == 0 and run(64, 4096, (2048, 1000)) == 1
+
+
+def test_graphs_have_their_own_workspaces():
+    """Two graphs captured one after the other on torch's capture stream, at two
+    row counts, through the decoder's capture(): the second replayed first, then
+    both in turn with eager calls between them, then both at the same time on
+    two streams, always with the eager results. Each capture is given its own
+    number, and none outside one."""
+    from lightserve_amd.model.graph_decode import capture
+    from lightserve_amd.kernels import tiled_matmul as tm
+    print("case graphs with their own workspaces", flush=True)
+    tm.release_workspaces()
+    assert _lib.capture_id(torch.cuda.current_stream().cuda_stream) == 0
+    g = torch.Generator(device="cuda").manual_seed(3)
+    w1 = (torch.randn(4096, 4096, device="cuda", generator=g) / 64).to(torch.bfloat16)
+    w2 = (torch.randn(4096, 2048, device="cuda", generator=g) / 64).to(torch.bfloat16)
+    xs = [torch.randn(m, 4096, device="cuda", generator=g).to(torch.bfloat16) for m in (8, 64, 1)]
+
+    def chain(x):  # three products that split K, each reading the one before
+        return matmul(matmul(matmul(x, w1), w1), w2)
+    eager = [chain(x) for x in xs]
+    graphs, ids, bufs = [], [], []
+    for x in xs:
+        graphs.append(capture(lambda x=x: chain(x)))
+        (entry,) = (e for e in tm._workspaces.values() if e.captured)
+        ids.append(entry.captured)
+        bufs.append(entry.graph_buf)
+    assert len(set(ids)) == 3 and len({b.data_ptr() for b in bufs}) == 3
+    torch.cuda.synchronize()
+
+    def check():
+        torch.cuda.synchronize()
+        for (_, out), want in zip(graphs, eager):
+            assert torch.equal(out, want)
+    for i in (1, 0, 2, 2, 0, 1):
+        graphs[i][1].zero_()
+        graphs[i][0].replay()
+        torch.cuda.synchronize()
+        assert torch.equal(graphs[i][1], eager[i])
+        assert torch.equal(chain(xs[0]), eager[0])
+    streams = [torch.cuda.Stream() for _ in graphs]
+    for _ in range(5):
+        for s, (graph, out) in zip(streams, graphs):
+            with torch.cuda.stream(s):
+                out.zero_()
+                for _ in range(3):
+                    graph.replay()
+        check()
