@@ -220,6 +220,28 @@ def skinny_matmul_group(a: torch.Tensor, bs, outs=None, gate: torch.Tensor = Non
     return outs
 
 
+def _sizes_fit(rows: int, k: int, cols) -> bool:
+    """Whether products of these sizes (rows and columns of a, columns of each
+    b) are routed to a kernel of the library, if nothing else is against it.
+    Arithmetic only, and asked first: a call that stays on torch anyway is short
+    enough (5 us at 64 rows of 1024 x 1024) for the other tests to show. (Sizes
+    that a tracer passes are symbols: no test of them becomes a guard.)"""
+    if torch.compiler.is_compiling():
+        return False
+    if rows <= AUTO_MAX_ROWS:
+        return True
+    total = 0
+    for n in cols:
+        if n % 128:
+            return False
+        total += n
+    if k % 8:
+        return False
+    if rows <= MFMA_AUTO_ROWS:
+        return total <= MFMA_AUTO_MAX_COLS
+    return (len(cols) > 1 or k >= GEMM_MIN_K) and GEMM_MIN_TILES <= total // 128 * ((rows + 63) // 64) <= GEMM_MAX_TILES
+
+
 def _library_only(*tensors) -> bool:
     """Whether a call on these tensors has to go through torch's own operators:
     a gradient is recorded (reverse or forward mode), a subclass, mode or
@@ -277,8 +299,7 @@ def _gemm_ok(a: torch.Tensor, bs) -> bool:
                 b.ndim == 2 and b.device == a.device and b.dtype == a.dtype and b.shape[0] == a.shape[1]
                 and b.shape[1] % 128 == 0 and b.shape[1] > 0 and _rows_addressable(b)
                 and b.shape[1] <= b.stride(0) <= MFMA_MAX_STRIDE for b in bs)
-            and GEMM_MIN_TILES <= sum(b.shape[1] for b in bs) // 128 * ((a.shape[0] + 63) // 64) <= GEMM_MAX_TILES
-            and (len(bs) > 1 or a.shape[1] >= GEMM_MIN_K))
+            and _sizes_fit(*a.shape, [b.shape[1] for b in bs]))
 
 
 def _gemm_group(a: torch.Tensor, bs):
@@ -291,7 +312,8 @@ def _gemm_group(a: torch.Tensor, bs):
 def matmul_shared_input(a: torch.Tensor, bs):
     """[matmul(a, b) for b in bs]: one grouped launch when the products
     qualify for the library's kernels together, else one matmul each."""
-    if a.ndim == 2 and not _library_only(a, *bs):
+    if (a.ndim == 2 and all(b.ndim == 2 for b in bs) and _sizes_fit(*a.shape, [b.shape[1] for b in bs])
+            and not _library_only(a, *bs)):
         if _auto_skinny(a, bs):
             return _skinny_run(a, bs)
         if _gemm_ok(a, bs):
@@ -302,8 +324,8 @@ def matmul_shared_input(a: torch.Tensor, bs):
 def swiglu_matmul(gate: torch.Tensor, up: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     """matmul(F.silu(gate) * up, b), the activation folded into the skinny
     kernels' load of their input when the product qualifies for them."""
-    if (gate.ndim == 2 and gate.shape == up.shape and gate.dtype == up.dtype == b.dtype and gate.is_cuda
-            and up.device == gate.device and b.device == gate.device and b.ndim == 2 and b.shape[0] == up.shape[1]
+    if (gate.ndim == 2 and gate.shape[0] <= MFMA_AUTO_ROWS and gate.shape == up.shape
+            and gate.dtype == up.dtype == b.dtype and gate.is_cuda and up.device == gate.device and b.device == gate.device and b.ndim == 2 and b.shape[0] == up.shape[1]
             and not _library_only(gate, up, b)
             and gate.stride(1) == 1 and (_skinny_ok(up, b, AUTO_MAX_ROWS) or (
                 _mfma_ok(up, [b]) and _rows_addressable(gate) and gate.stride(0) >= gate.shape[1]))):
@@ -354,7 +376,7 @@ def matmul(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     assert a.shape[1] == b.shape[0], f"inner dims must match: a is {tuple(a.shape)}, b is {tuple(b.shape)}"
     assert a.is_cuda and b.is_cuda, "the gfx950 path needs GPU tensors"
     assert a.dtype == b.dtype, f"dtype mismatch: a={a.dtype} b={b.dtype}"
-    if not _library_only(a, b):
+    if _sizes_fit(*a.shape, b.shape[1:]) and not _library_only(a, b):
         if _auto_skinny(a, [b]):
             return _skinny_run(a, [b])[0]
         if _gemm_ok(a, [b]):

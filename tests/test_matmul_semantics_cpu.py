@@ -167,3 +167,18 @@ def test_norm_route_asks_as_well(tm, m, with_residual, monkeypatch):
         assert torch.get_autocast_dtype("cuda") == torch.float16 and apart()
     finally:
         torch.set_autocast_enabled("cuda", False)
+
+
+@pytest.mark.parametrize("m,k,n", [(64, 128, 128), (600, 4096, 4096), (64, 4096, 200), (5000, 4096, 4096), (9, 128, 200),
+                                   (16, 12, 128)])
+def test_sizes_that_stay_on_torch_are_told_first(tm, m, k, n, monkeypatch):
+    """A product that no kernel takes by its size goes on without the other questions."""
+    def asked(*args):
+        raise AssertionError("asked")
+    for name in ("_library_only", "_auto_skinny", "_gemm_ok"):
+        monkeypatch.setattr(tm, name, asked)
+    monkeypatch.setattr(torch, "matmul", lambda a, b: "torch")
+    x, w = torch.empty(m, k, dtype=torch.bfloat16), torch.empty(k, n, dtype=torch.bfloat16)
+    assert tm.matmul(x, w) == "torch" and tm.matmul_shared_input(x, [w])[0] == "torch"
+    if m > 32:
+        assert tm.swiglu_matmul(x, x, w) == "torch"
