@@ -548,9 +548,11 @@ int lsfa_gemv_check(const lsfa_gemv_args* args);
 /* Workspace bytes lsfa_gemv needs (m, k and n matter); no GPU work. */
 int lsfa_gemv_workspace_size(const lsfa_gemv_args* args, uint64_t* bytes);
 
-/* y = x @ w for m <= 32 rows (see lsfa_gemv_args): one launch on the stream,
- * a K-split pass over w whose last-arriving workgroup per column block sums
- * the splits (in split order: deterministic) and rounds once into y. */
+/* y = x @ w for m <= 32 rows (see lsfa_gemv_args): a K-split pass over w
+ * whose last-arriving workgroup per column block sums the splits (in split
+ * order: deterministic) and rounds once into y. One launch on the stream; from
+ * 3 rows on, several where x rows lie so far apart that their byte offsets pass
+ * 31 bits. More than 8 rows also need w_stride <= 2^25. */
 int lsfa_gemv(const lsfa_gemv_args* args, void* stream);
 
 /* The grouped form (lsfa_gemv_group_args): validation, workspace size, launch. */
@@ -559,7 +561,7 @@ int lsfa_gemv_group_workspace_size(const lsfa_gemv_group_args* args, uint64_t* b
 int lsfa_gemv_group(const lsfa_gemv_group_args* args, void* stream);
 
 /* The same product above 32 rows (no gate, no norm; every width a multiple of
- * 128, k % 8 == 0, x rows 16-byte aligned) for launches of at most 256 tiles
+ * 128, k % 8 == 0, x rows 16-byte aligned, x_stride <= 2^23, w_stride <= 2^25) for launches of at most 256 tiles
  * of 64 rows x 128 columns, where a general GEMM's tiles leave CUs idle. */
 int lsfa_gemm_group_check(const lsfa_gemv_group_args* args);
 int lsfa_gemm_group_workspace_size(const lsfa_gemv_group_args* args, uint64_t* bytes);

@@ -680,12 +680,15 @@ bool gemv_uses_mfma(const lsfa_gemv_group_args* a) {
   return n / 128 <= LSFA_GEMV_COUNTER_BYTES / 64;
 }
 
-// Its split: as many K-ranges of at least 256 rows as keep the grid within
-// one workgroup per CU (column blocks x splits <= 256), ranges multiples of the
-// 32-row step. Measured at 8 rows over 1..16 splits: 48 blocks 28.0 us at 1,
+// Its split: as many K-ranges, one for each 256 rows of K begun at most, as
+// keep the grid within one workgroup per CU (column blocks x 64-row blocks x
+// splits <= 256), in equal ranges rounded up to the 32-row step (K = 264: 160 and
+// 104). Measured at 8 rows over 1..16 splits: 48 blocks 28.0 us at 1,
 // 13.5 at 5, 16.6 at 6; 32 blocks of K = 14336 88 at 1, 23.1 at 8, 30.4 at 10;
 // 224 blocks 42.3 at 1, 44.0 at 2, 47.6 at 8: a second workgroup on some CUs
-// only adds partials. The workspace has room for 512 workgroups' partials.
+// only adds partials. Up to 32 rows the size asked for stays what it was when
+// launches took up to 512 workgroups (a caller may hold it): more than these
+// splits use.
 GemvSplit gemv_split_mfma(long long M, long long K, long long N) {
   GemvSplit g;
   M = std::max(M, 0LL); K = std::max(K, 0LL); N = std::max(N, 0LL);
@@ -758,7 +761,7 @@ int lsfa_gemv_group_check(const lsfa_gemv_group_args* a) {
   if (a->m < 0 || a->k < 0) return fail(LSFA_ERR_INVALID, "negative size (m=%d k=%d)", a->m, a->k);
   if (a->m > 8 && !gemv_uses_mfma(a))
     return fail(LSFA_ERR_UNSUPPORTED, "gemv takes at most 8 rows, or 32 without a fused norm, widths that are multiples of "
-                "128 and 16-byte aligned x rows (m=%d)", a->m);
+                "128, w_stride at most 2^25 and 16-byte aligned x rows (m=%d)", a->m);
   for (int i = 0; i < a->count; ++i) {
     if (a->n[i] < 0) return fail(LSFA_ERR_INVALID, "negative size (n=%d)", a->n[i]);
     if (a->n[i] % 8 != 0) return fail(LSFA_ERR_UNSUPPORTED, "gemv needs n %% 8 == 0 (n=%d)", a->n[i]);

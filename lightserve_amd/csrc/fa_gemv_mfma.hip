@@ -289,7 +289,7 @@ __global__ __launch_bounds__(64 * NW, 2) void fa_gemv_mfma_kernel(const GemvPara
   float t0[IT], t1[IT];
 #pragma unroll
   for (int it = 0; it < IT; ++it) t0[it] = t1[it] = 0.f;
-  constexpr int SB = IT <= 2 ? 8 : (IT <= 4 ? 4 : 2);
+  constexpr int SB = IT <= 4 ? 4 : 2;
   for (int s0 = 0; s0 < p.splits; s0 += SB) {
     uint64_t v[SB][IT];
 #pragma unroll

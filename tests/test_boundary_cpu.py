@@ -535,6 +535,8 @@ def test_abi_gemv_validation(built_library):
     assert rc == -2 and "8 rows" in msg
     rc, msg = _lib.gemv_check(_gemv_args(m=9, n=4104, w_stride=4104))  # not a multiple of 128
     assert rc == -2 and "8 rows" in msg
+    rc, msg = _lib.gemv_check(_gemv_args(m=9, w_stride=(1 << 25) + 8))
+    assert rc == -2 and "w_stride" in msg
     # MFMA workspace: K-ranges of 256 rows -> 16 splits at K = 4096
     assert _lib.gemv_workspace_size(_gemv_args(m=16)) == 262144 + 16 * 16 * 4096 * 4
     rc, msg = _lib.gemv_check(_gemv_args(n=4092, w_stride=4096))
