@@ -13,7 +13,7 @@
 
 namespace lsfa {
 hipError_t fwd_mfma(FwdParams p, bool is_bf16, int dp, bool causal, bool varlen, hipStream_t s);
-int fwd_splits(int B, int Hq, int Nq, int dp, long long max_keys);
+int fwd_splits(int B, int Hq, int Nq, int dp, bool varlen, long long max_keys);
 uint64_t fwd_part_bytes(int B, int Hq, int Nq, int dp, int splits);
 hipError_t fwd_paged(FwdParams p, bool is_bf16, int dp, bool causal, hipStream_t s);
 hipError_t bwd_mfma(const BwdParams& p, bool is_bf16, int dp, bool causal, int phases, hipStream_t s);
@@ -224,7 +224,8 @@ static int check_split_workspace(const char* query, const void* workspace, uint6
 
 static int fwd_split_count(const lsfa_fwd_args* a) {
   if (a->dtype == LSFA_DTYPE_FP32) return 1;
-  return lsfa::fwd_splits(a->batch, a->heads_q, a->seqlen_q, padded_dim(a->head_dim), a->seqlen_k);
+  return lsfa::fwd_splits(a->batch, a->heads_q, a->seqlen_q, padded_dim(a->head_dim), a->cu_seqlens_q != nullptr,
+                          a->seqlen_k);
 }
 
 int lsfa_fwd_workspace_size(const lsfa_fwd_args* a, uint64_t* bytes) {
@@ -593,7 +594,7 @@ int lsfa_prefill_paged_check(const lsfa_prefill_paged_args* a) {
 static int prefill_split_count(const lsfa_prefill_paged_args* a) {
   if (a->batch <= 0 || a->max_seqlen_q <= 0 || a->heads_q <= 0 || a->max_blocks_per_seq <= 0 || a->block_size <= 0)
     return 1;
-  return lsfa::fwd_splits(a->batch, a->heads_q, a->max_seqlen_q, padded_dim(a->head_dim),
+  return lsfa::fwd_splits(a->batch, a->heads_q, a->max_seqlen_q, padded_dim(a->head_dim), true,
                           (long long)a->max_blocks_per_seq * a->block_size);
 }
 

@@ -1241,27 +1241,43 @@ static hipError_t launch_fwd_nw(FwdParams p, hipStream_t s) {
 
 // Key splits (4-wave workgroups, two of which share a CU) of a launch of
 // B x Hq x ceil(Nq / 128) items over at most max_keys keys each: the count of
-// least estimated time, 1 where splitting does not pay. A 64-key step takes
-// about 1.2 us with one workgroup on its CU and 1.95 us with two; a split
-// launch adds 5 us (the combine launch and the partials' latency) and 23 ns per
-// workgroup for writing and reading its 64 KB of partials (head dim 128).
-// Measured, unsplit against split: 96 items of 100 tiles 154 -> 60 us (5
-// splits; 73 at 2), 128 of 64 87 -> 42 (4), 128 of 32 37 -> 30 (2; 29 at 4),
-// 252 of 125 167 -> 132 (2), but 128 of 8 14.5 -> 17.9 (2), 168 of 13 18.2 ->
-// 23.4 (3): both left unsplit by this rule.
-int fwd_splits(int B, int Hq, int Nq, int dp, long long max_keys) {
-  const long long items = (long long)B * Hq * ((Nq + 127) / 128);
-  const double tiles = (double)((max_keys + 63) / 64);
-  int best = 1;
-  double least = tiles * 1.2;
-  for (int s = 2; s <= 16 && items > 0 && items * s <= 512 && s * kSplitMinTiles <= tiles; ++s) {
-    const double us = tiles / s * (items * s <= 256 ? 1.2 : 1.95) + 5.0 + 0.023 * (double)(items * s) * dp / 128;
+// least estimated time, 1 where splitting does not pay. A launch takes a 64-key
+// step's time for each tile of its longest workgroup (split_tiles rounds a
+// split's tiles up to an even number), and a split one the combine launch, the
+// partials' latency and the writing and reading of its workgroups' partials on
+// top. The times are those that choose best over measured launches of 3 to 256
+// items of 5 to 235 tiles at 1 to 16 splits, dense and paged, causal and not. A
+// split has to win by half a microsecond to one.
+// Dense, us unsplit against split as chosen: head dim 128, 16 items of 32 tiles 34.2
+// -> 14.4 (8 splits), 64 of 16 20.8 -> 19.3 (4), 128 of 16 21.4 (24.8 in two: left
+// whole); head dim 64, 32 of 64 60.2 -> 15.5 (8), 64 of 16 15.3 -> 12.0 (4), 128 of 16
+// 16.4 (17.9 in two, 19.4 in four: left whole), 160 of 20 18.7 (23.4 in three: left
+// whole); head dim 32, 64 of 32 20.3 -> 13.1 (8), 80 of 10 9.2 (10.9 in two: left
+// whole). Paged, head dim 128: 96 items of 100 tiles 154 -> 60 us (5 splits), 128 of
+// 64 87 -> 42 (4), 252 of 125 167 -> 132 (2), 168 of 13 18.2 (23.4 in three: left whole).
+struct StepUs {
+  double one, two, eight;  // one and two 4-wave workgroups on a CU; an 8-wave workgroup of 256 rows
+};
+static long long split_count(long long items, long long tiles, int dp, bool varlen, bool eight) {
+  const StepUs c = varlen ? StepUs{1.2, 1.95, 1.2}
+                          : (dp == 32 ? StepUs{0.48, 0.73, 0.48} : (dp == 64 ? StepUs{0.77, 1.05, 0.86} : StepUs{1.0, 1.4, 1.2}));
+  const double fixed = varlen ? 5.0 : 2.9, per_part = (varlen ? 0.023 : 0.025) * dp / 128, margin = varlen ? 0.0 : 1.1;
+  long long best = 1;
+  double least = tiles * (eight ? c.eight : (items <= 256 ? c.one : c.two)) - margin;
+  for (long long s = 2; s <= 16 && items * s <= 512 && s * kSplitMinTiles <= tiles; ++s) {
+    const double longest = varlen ? (double)tiles / s : (double)(((tiles + s - 1) / s + 1) & ~1LL);
+    const double us = longest * (items * s <= 256 ? c.one : c.two) + fixed + per_part * (double)(items * s);
     if (us < least) {
       least = us;
       best = s;
     }
   }
   return best;
+}
+int fwd_splits(int B, int Hq, int Nq, int dp, bool varlen, long long max_keys) {
+  const long long items = (long long)B * Hq * ((Nq + 127) / 128), tiles = (max_keys + 63) / 64;
+  if (items <= 0 || tiles <= 2 * kSplitMinTiles) return 1;
+  return (int)split_count(items, tiles, dp, varlen, !varlen && dp >= 64 && Nq >= 4096);
 }
 // Bytes of p.part for that launch.
 uint64_t fwd_part_bytes(int B, int Hq, int Nq, int dp, int splits) {

@@ -759,6 +759,21 @@ def test_abi_key_split_workspace(built_library):
                     assert _lib.fwd_workspace_size(dense(batch=b, heads_q=h, heads_kv=h, seqlen_q=n, seqlen_k=n)) == 0
 
 
+@pytest.mark.parametrize("head_dim,heads,n,split", [
+    (32, 16, 640, False), (32, 4, 640, False), (64, 16, 640, False), (64, 4, 640, False), (128, 4, 640, False),
+    (64, 16, 1024, False), (64, 16, 1280, False), (128, 16, 1024, False), (32, 32, 768, False),
+    (64, 8, 1024, True), (64, 8, 2048, True), (128, 8, 1024, True), (128, 4, 4096, True), (32, 2, 1024, True)])
+def test_dense_split_where_it_pays(built_library, head_dim, heads, n, split):
+    """The key-split rule on either side of its measured line, at each padded
+    head dim: the launches named False were slower split than whole."""
+    st = _lib._i64x4(1 << 20, 1 << 18, head_dim, 1)
+    for causal in (0, 1):
+        args = _lib.FwdArgs(q=4096, k=4096, v=4096, o=4096, lse=None, dtype=_lib.DTYPE_BF16, batch=1, heads_q=heads,
+                            heads_kv=heads, seqlen_q=n, seqlen_k=n, head_dim=head_dim, causal=causal, sm_scale=0.125,
+                            q_stride=st, k_stride=st, v_stride=st, o_stride=st, lse_stride=_lib._i64x3(0, 0, 0))
+        assert (_lib.fwd_workspace_size(args) > 0) == split
+
+
 def test_abi_gemm_group_validation(built_library):
     """lsfa_gemm_group: more than 32 rows, at most 256 tiles of 64 x 128; other
     checks as lsfa_gemv_group's; the workspace checked for its own row count."""
