@@ -20,7 +20,8 @@ LLaMA-3-8B decode projections at 8 and 32 rows (us, graph replays, weights
 that no cache holds), this kernel against hipBLASLt: q/k/v 13.5 and 16.4
 against 51.9 and 54.1, o 10.9 and 13.7 against 21.9 and 20.9, gate/up 42.3 and
 46.2 against 56.1 and 56.8, down 23.1 and 27.2 against 71.0 and 61.4, LM head
-165 and 177 against 190 and 198; so every such product goes to it. Calls that
+165 and 177 against 190 and 198; so such products go to it, small single ones
+above 8 rows apart (MFMA_MIN_*). Calls that
 autograd, a tracer or autocast has to see stay on torch's operators at every
 row count (_library_only). The norm
 is folded into the launch at up to 2 rows only. Above 32 rows the same kernel
@@ -70,11 +71,24 @@ AUTO_MAX_ROWS = 2    # rows that every product (and the fused norm / SwiGLU inpu
 MFMA_AUTO_ROWS = 32
 MFMA_AUTO_MAX_COLS = 128 * (_lib.GEMV_COUNTER_BYTES // 64)
 MFMA_MAX_STRIDE = 1 << 25  # of W's rows: 32 of them in a 31-bit byte offset
+# A matrix by itself has to be large enough for the pass over it to outweigh the
+# launch and the split's reduction (a group saves launches too, and runs from 256 x
+# 256 on). Measured against hipBLASLt in us: up to 16 rows K of 1536 or 2.4 million
+# elements (1024 x 1024 6.4 against 5.8, 512 x 1024 8.2 against 5.6, 2048 x 512 6.7
+# against 7.3; up to 256 columns all the same); above 16 rows, where hipBLASLt has its own kernels for them, 9.4
+# million (4096 x 1024 13.6 against 10.1, 4096 x 2048 1.2..1.3 times its time, 3072 x
+# 3072 0.7 times). Up to 8 rows all go to the kernel.
+MFMA_MIN_K, MFMA_MIN_ELEMS, MFMA_MIN_ELEMS_17 = 1536, 9 << 18, 9 << 20
 # Above MFMA_AUTO_ROWS rows, lsfa_gemm_group runs launches of this many tiles of
 # 64 x 128 whose K is at least GEMM_MIN_K or which group several matrices (a
 # short K alone: 2048 -> 2048 at 128 rows 15.7 us against hipBLASLt's 12.6; few
-# tiles: 4096 -> 1024 at 48 rows 19.0 against 14.6).
-GEMM_MIN_TILES, GEMM_MAX_TILES, GEMM_MIN_K = 16, 256, 4096
+# tiles: 4096 -> 1024 at 48 rows 19.0 against 14.6). Fewer than GEMM_FEW_TILES
+# need more: a matrix by itself a K of 8192 or 2048 columns (4096 -> 1024 at 128 rows
+# 19.2 against 16.3, 4096 -> 256 at 512 21.5 against 15.0; 8192 -> 1024 0.72 times
+# hipBLASLt's time), two matrices a K of 1024 (512 -> 512 + 512 at 192 rows 11.2
+# against 10.5). Over 64 rows and 8192 columns a matrix by itself is hipBLASLt's
+# (4096 -> 14336 at 128 rows 44.4 against 41.7).
+GEMM_MIN_TILES, GEMM_FEW_TILES, GEMM_MAX_TILES, GEMM_MIN_K = 16, 32, 256, 4096
 
 MAX_CACHED_STREAMS = 8
 
@@ -237,9 +251,19 @@ def _sizes_fit(rows: int, k: int, cols) -> bool:
         total += n
     if k % 8:
         return False
+    alone = len(cols) == 1
     if rows <= MFMA_AUTO_ROWS:
-        return total <= MFMA_AUTO_MAX_COLS
-    return (len(cols) > 1 or k >= GEMM_MIN_K) and GEMM_MIN_TILES <= total // 128 * ((rows + 63) // 64) <= GEMM_MAX_TILES
+        if alone and rows > 16:
+            return MFMA_MIN_ELEMS_17 <= k * total <= k * MFMA_AUTO_MAX_COLS
+        return total <= MFMA_AUTO_MAX_COLS and (not alone or rows <= 8 or total <= 256 or k >= MFMA_MIN_K
+                                                or k * total >= MFMA_MIN_ELEMS)
+    tiles = total // 128 * ((rows + 63) // 64)
+    if tiles < GEMM_MIN_TILES or tiles > GEMM_MAX_TILES:
+        return False
+    if alone:
+        return (k >= GEMM_MIN_K and (tiles >= GEMM_FEW_TILES or k >= 2 * GEMM_MIN_K or total >= 2048)
+                and (rows <= 64 or total <= 8192))
+    return tiles >= GEMM_FEW_TILES or k >= 1024 or len(cols) > 2
 
 
 def _library_only(*tensors) -> bool:

@@ -48,7 +48,7 @@ def _operands(m, k=4096, n=256):
 def test_plain_calls_reach_the_kernels(tm):
     """The stand-in decides as on a GPU: without a transform these are routed."""
     for m in (1, 2, 3, 32, 512):
-        x, y, w = _operands(m, n=4096 if m > 32 else 256)
+        x, y, w = _operands(m, n=4096 if m > 16 else 256)
         for f in _calls(tm, x, w)[:2 if m > 32 else 4]:
             with pytest.raises(AssertionError, match="routed to a kernel"):
                 f(y)
@@ -114,7 +114,7 @@ class _Seen(torch.overrides.TorchFunctionMode):
 def test_modes_that_change_nothing(tm, m):
     """A default device and autocast to the operands' own type leave the
     kernels in place; autocast to another type and any other mode do not."""
-    x, y, w = _operands(m, n=128)
+    x, y, w = _operands(m, n=256)
     mode = _Seen()
     mode.names = []
     for f in _calls(tm, x, w):
@@ -170,7 +170,9 @@ def test_norm_route_asks_as_well(tm, m, with_residual, monkeypatch):
 
 
 @pytest.mark.parametrize("m,k,n", [(64, 128, 128), (600, 4096, 4096), (64, 4096, 200), (5000, 4096, 4096), (9, 128, 200),
-                                   (16, 12, 128)])
+                                   (16, 12, 128),
+                                   (9, 1024, 1024), (16, 512, 2048), (17, 4096, 2048), (32, 8192, 512), (128, 4096, 1024),
+                                   (512, 4096, 256), (128, 4096, 14336)])
 def test_sizes_that_stay_on_torch_are_told_first(tm, m, k, n, monkeypatch):
     """A product that no kernel takes by its size goes on without the other questions."""
     def asked(*args):
@@ -182,3 +184,12 @@ def test_sizes_that_stay_on_torch_are_told_first(tm, m, k, n, monkeypatch):
     assert tm.matmul(x, w) == "torch" and tm.matmul_shared_input(x, [w])[0] == "torch"
     if m > 32:
         assert tm.swiglu_matmul(x, x, w) == "torch"
+
+
+@pytest.mark.parametrize("rows,k,cols", [(8, 512, (128,)), (9, 1536, (128,)), (16, 768, (3072,)), (9, 512, (256,)), (17, 3072, (3072,)),
+                                         (32, 4096, (4096,)), (32, 256, (256, 256, 256)), (64, 4096, (14336,)),
+                                         (128, 8192, (1024,)), (200, 4096, (1024,)), (512, 4096, (4096,)), (33, 4096, (2048,)),
+                                         (65, 1024, (512, 512)), (129, 512, (1024, 1024)), (192, 256, (256, 256, 256))])
+def test_sizes_that_have_a_kernel(rows, k, cols):
+    """The other side of the same lines."""
+    assert tiled_matmul._sizes_fit(rows, k, cols)
