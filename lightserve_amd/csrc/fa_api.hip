@@ -13,7 +13,7 @@
 
 namespace lsfa {
 hipError_t fwd_mfma(FwdParams p, bool is_bf16, int dp, bool causal, bool varlen, hipStream_t s);
-int fwd_splits(int B, int Hq, int Nq, int dp, bool varlen, long long max_keys);
+int fwd_splits(int B, int Hq, int Nq, int dp, bool varlen, long long max_keys, int* least_tiles);
 uint64_t fwd_part_bytes(int B, int Hq, int Nq, int dp, int splits);
 hipError_t fwd_paged(FwdParams p, bool is_bf16, int dp, bool causal, hipStream_t s);
 hipError_t bwd_mfma(const BwdParams& p, bool is_bf16, int dp, bool causal, int phases, hipStream_t s);
@@ -222,25 +222,28 @@ static int check_split_workspace(const char* query, const void* workspace, uint6
   return ok();
 }
 
-static int fwd_split_count(const lsfa_fwd_args* a) {
+static int fwd_split_count(const lsfa_fwd_args* a, int* least_tiles) {
+  *least_tiles = 0;
   if (a->dtype == LSFA_DTYPE_FP32) return 1;
   return lsfa::fwd_splits(a->batch, a->heads_q, a->seqlen_q, padded_dim(a->head_dim), a->cu_seqlens_q != nullptr,
-                          a->seqlen_k);
+                          a->seqlen_k, least_tiles);
 }
 
 int lsfa_fwd_workspace_size(const lsfa_fwd_args* a, uint64_t* bytes) {
   if (a == nullptr || bytes == nullptr) return fail(LSFA_ERR_INVALID, "args or bytes is NULL");
   int rc = check_common(a->dtype, a->batch, a->heads_q, a->heads_kv, a->seqlen_q, a->seqlen_k, a->head_dim, a->sm_scale);
   if (rc) return rc;
-  *bytes = lsfa::fwd_part_bytes(a->batch, a->heads_q, a->seqlen_q, padded_dim(a->head_dim), fwd_split_count(a));
+  int least = 0;
+  *bytes = lsfa::fwd_part_bytes(a->batch, a->heads_q, a->seqlen_q, padded_dim(a->head_dim), fwd_split_count(a, &least));
   return ok();
 }
 
-static int run_fwd(const lsfa_fwd_args* a, int splits, void* workspace, void* stream) {
+static int run_fwd(const lsfa_fwd_args* a, int splits, int split_min, void* workspace, void* stream) {
   if ((long long)a->batch * a->heads_q * a->seqlen_q == 0) return ok();
   lsfa::FwdParams p;
   memset(&p, 0, sizeof(p));
   p.splits = splits;
+  p.split_min = split_min;
   p.part = static_cast<float*>(workspace);
   p.q = a->q;
   p.k = a->k;
@@ -275,7 +278,7 @@ static int run_fwd(const lsfa_fwd_args* a, int splits, void* workspace, void* st
 
 int lsfa_fwd(const lsfa_fwd_args* a, void* stream) {
   const int rc = lsfa_fwd_check(a);
-  return rc ? rc : run_fwd(a, 1, nullptr, stream);
+  return rc ? rc : run_fwd(a, 1, 0, nullptr, stream);
 }
 
 int lsfa_fwd_split(const lsfa_fwd_args* a, void* workspace, uint64_t workspace_bytes, void* stream) {
@@ -284,7 +287,9 @@ int lsfa_fwd_split(const lsfa_fwd_args* a, void* workspace, uint64_t workspace_b
   uint64_t need = 0;
   if ((rc = lsfa_fwd_workspace_size(a, &need))) return rc;
   if ((rc = check_split_workspace("lsfa_fwd_workspace_size", workspace, workspace_bytes, need))) return rc;
-  return run_fwd(a, need > 0 ? fwd_split_count(a) : 1, workspace, stream);
+  int least = 0;
+  const int splits = need > 0 ? fwd_split_count(a, &least) : 1;
+  return run_fwd(a, splits, least, workspace, stream);
 }
 
 int lsfa_bwd_check(const lsfa_bwd_args* a) {
@@ -591,24 +596,28 @@ int lsfa_prefill_paged_check(const lsfa_prefill_paged_args* a) {
   return ok();
 }
 
-static int prefill_split_count(const lsfa_prefill_paged_args* a) {
+static int prefill_split_count(const lsfa_prefill_paged_args* a, int* least_tiles) {
+  *least_tiles = 0;
   if (a->batch <= 0 || a->max_seqlen_q <= 0 || a->heads_q <= 0 || a->max_blocks_per_seq <= 0 || a->block_size <= 0)
     return 1;
   return lsfa::fwd_splits(a->batch, a->heads_q, a->max_seqlen_q, padded_dim(a->head_dim), true,
-                          (long long)a->max_blocks_per_seq * a->block_size);
+                          (long long)a->max_blocks_per_seq * a->block_size, least_tiles);
 }
 
 int lsfa_prefill_paged_workspace_size(const lsfa_prefill_paged_args* a, uint64_t* bytes) {
   if (a == nullptr || bytes == nullptr) return fail(LSFA_ERR_INVALID, "args or bytes is NULL");
-  *bytes = lsfa::fwd_part_bytes(a->batch, a->heads_q, a->max_seqlen_q, padded_dim(a->head_dim), prefill_split_count(a));
+  int least = 0;
+  *bytes = lsfa::fwd_part_bytes(a->batch, a->heads_q, a->max_seqlen_q, padded_dim(a->head_dim),
+                                prefill_split_count(a, &least));
   return ok();
 }
 
-static int run_prefill_paged(const lsfa_prefill_paged_args* a, int splits, void* workspace, void* stream) {
+static int run_prefill_paged(const lsfa_prefill_paged_args* a, int splits, int split_min, void* workspace, void* stream) {
   if (a->batch == 0 || a->max_seqlen_q == 0) return ok();
   lsfa::FwdParams p;
   memset(&p, 0, sizeof(p));
   p.splits = splits;
+  p.split_min = split_min;
   p.part = static_cast<float*>(workspace);
   p.q = a->q; p.k = a->k_cache; p.v = a->v_cache; p.o = a->o; p.lse = a->lse;
   p.sqn = a->q_stride[0]; p.sqh = a->q_stride[1];
@@ -635,7 +644,7 @@ static int run_prefill_paged(const lsfa_prefill_paged_args* a, int splits, void*
 
 int lsfa_prefill_paged(const lsfa_prefill_paged_args* a, void* stream) {
   const int rc = lsfa_prefill_paged_check(a);
-  return rc ? rc : run_prefill_paged(a, 1, nullptr, stream);
+  return rc ? rc : run_prefill_paged(a, 1, 0, nullptr, stream);
 }
 
 int lsfa_prefill_paged_split(const lsfa_prefill_paged_args* a, void* workspace, uint64_t workspace_bytes, void* stream) {
@@ -644,7 +653,9 @@ int lsfa_prefill_paged_split(const lsfa_prefill_paged_args* a, void* workspace, 
   uint64_t need = 0;
   if ((rc = lsfa_prefill_paged_workspace_size(a, &need))) return rc;
   if ((rc = check_split_workspace("lsfa_prefill_paged_workspace_size", workspace, workspace_bytes, need))) return rc;
-  return run_prefill_paged(a, need > 0 ? prefill_split_count(a) : 1, workspace, stream);
+  int least = 0;
+  const int splits = need > 0 ? prefill_split_count(a, &least) : 1;
+  return run_prefill_paged(a, splits, least, workspace, stream);
 }
 
 }  // extern "C"

@@ -165,6 +165,7 @@ struct FwdParams {
   // Key splits (more than one: each item's keys are shared out over that many
   // workgroups, whose partial results meet in part).
   int splits;
+  int split_min;  // items of fewer key tiles keep one workgroup
   float* part;
 };
 

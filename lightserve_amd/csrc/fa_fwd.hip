@@ -96,11 +96,13 @@ __device__ __forceinline__ bool item_at(const FwdParams& p, int lane, int& b, in
 }
 
 // Key tiles [lo, hi) of split `split` of an item of ntiles tiles over at most
-// `most` splits, and how many splits the item has: at least kSplitMinTiles
-// tiles each, an even number (the tiles' LDS buffers go by parity).
+// `most` splits, and how many splits the item has: one if it has fewer than
+// `least` tiles, else at most one for kSplitMinTiles tiles; each but the last
+// takes the same number of tiles, an even one (the tiles' LDS buffers go by
+// parity).
 constexpr int kSplitMinTiles = 4;
-__device__ __forceinline__ int split_tiles(int ntiles, int most, int split, int& lo, int& hi) {
-  const int want = max(1, min(most, ntiles / kSplitMinTiles));
+__device__ __forceinline__ int split_tiles(int ntiles, int most, int least, int split, int& lo, int& hi) {
+  const int want = ntiles < least ? 1 : max(1, min(most, ntiles / kSplitMinTiles));
   const int per = ((ntiles + want - 1) / want + 1) & ~1;
   lo = split * per;
   hi = min(ntiles, lo + per);
@@ -205,7 +207,7 @@ __global__ __launch_bounds__((NW * 64), (8 / NW)) void fa_fwd_kernel(const FwdPa
   int first = 0, splits = 1;
   if constexpr (SPLIT) {
     int hi;
-    splits = split_tiles(ntiles, gridDim.y, blockIdx.y, first, hi);
+    splits = split_tiles(ntiles, gridDim.y, p.split_min, blockIdx.y, first, hi);
     if ((int)blockIdx.y >= splits) return;  // uniform, before any barrier
     ntiles = hi;
     if (blockIdx.y == 0 && tid == 0)
@@ -1254,19 +1256,23 @@ static hipError_t launch_fwd_nw(FwdParams p, hipStream_t s) {
 // 16.4 (17.9 in two, 19.4 in four: left whole), 160 of 20 18.7 (23.4 in three: left
 // whole); head dim 32, 64 of 32 20.3 -> 13.1 (8), 80 of 10 9.2 (10.9 in two: left
 // whole). Paged, head dim 128: 96 items of 100 tiles 154 -> 60 us (5 splits), 128 of
-// 64 87 -> 42 (4), 252 of 125 167 -> 132 (2), 168 of 13 18.2 (23.4 in three: left whole).
+// 64 87 -> 42 (4), 252 of 125 167 -> 132 (2), 256 of 40 (8-wave unsplit) 64.5 -> 58.8 (2),
+// 256 of 16 30.8 (34.9 in two: left whole); head dim 64, 256 of 48 56 -> 42 (2).
 struct StepUs {
-  double one, two, eight;  // one and two 4-wave workgroups on a CU; an 8-wave workgroup of 256 rows
+  double one, one_full, two, eight;  // 4-wave workgroups, one on a few CUs, on every CU, two on a CU; an 8-wave one of 256 rows
 };
 static long long split_count(long long items, long long tiles, int dp, bool varlen, bool eight) {
-  const StepUs c = varlen ? StepUs{1.2, 1.95, 1.2}
-                          : (dp == 32 ? StepUs{0.48, 0.73, 0.48} : (dp == 64 ? StepUs{0.77, 1.05, 0.86} : StepUs{1.0, 1.4, 1.2}));
-  const double fixed = varlen ? 5.0 : 2.9, per_part = (varlen ? 0.023 : 0.025) * dp / 128, margin = varlen ? 0.0 : 1.1;
+  const StepUs c = varlen ? (dp == 32 ? StepUs{0.65, 0.72, 1.0, 0.65} : (dp == 64 ? StepUs{0.88, 0.97, 1.39, 1.26} : StepUs{1.1, 1.2, 1.9, 1.84}))
+                          : (dp == 32 ? StepUs{0.48, 0.48, 0.73, 0.48} : (dp == 64 ? StepUs{0.77, 0.77, 1.05, 0.86} : StepUs{1.0, 1.0, 1.4, 1.2}));
+  const double fixed = varlen ? 2.1 : 2.9, per_part = 0.025 * dp / 128, margin = varlen ? 0.5 : 1.1;
+  auto step = [&](long long workgroups) {
+    return workgroups > 256 ? c.two : c.one + (c.one_full - c.one) * (double)workgroups / 256;
+  };
   long long best = 1;
-  double least = tiles * (eight ? c.eight : (items <= 256 ? c.one : c.two)) - margin;
+  double least = tiles * (eight ? c.eight : step(items)) - margin;
   for (long long s = 2; s <= 16 && items * s <= 512 && s * kSplitMinTiles <= tiles; ++s) {
-    const double longest = varlen ? (double)tiles / s : (double)(((tiles + s - 1) / s + 1) & ~1LL);
-    const double us = longest * (items * s <= 256 ? c.one : c.two) + fixed + per_part * (double)(items * s);
+    const long long longest = ((tiles + s - 1) / s + 1) & ~1LL;
+    const double us = longest * step(items * s) + fixed + per_part * (double)(items * s);
     if (us < least) {
       least = us;
       best = s;
@@ -1274,10 +1280,25 @@ static long long split_count(long long items, long long tiles, int dp, bool varl
   }
   return best;
 }
-int fwd_splits(int B, int Hq, int Nq, int dp, bool varlen, long long max_keys) {
+// The splits of a launch, and in *least_tiles the fewest tiles for which its
+// items are split. A paged launch's max_keys is what the block tables have room
+// for; a varlen one's is the longest sequence's: shorter items, for which the
+// same rule would not split the launch, keep one workgroup.
+int fwd_splits(int B, int Hq, int Nq, int dp, bool varlen, long long max_keys, int* least_tiles) {
   const long long items = (long long)B * Hq * ((Nq + 127) / 128), tiles = (max_keys + 63) / 64;
+  *least_tiles = 0;
   if (items <= 0 || tiles <= 2 * kSplitMinTiles) return 1;
-  return (int)split_count(items, tiles, dp, varlen, !varlen && dp >= 64 && Nq >= 4096);
+  const bool eight = dp >= 64 && (varlen ? B <= 64 && Nq >= 512 : Nq >= 4096);
+  const int splits = (int)split_count(items, tiles, dp, varlen, eight);
+  if (splits > 1 && varlen) {
+    long long lo = 2 * kSplitMinTiles, hi = tiles;  // not split at lo, split at hi
+    while (hi - lo > 1) {
+      const long long mid = (lo + hi) / 2;
+      (split_count(items, mid, dp, varlen, eight) > 1 ? hi : lo) = mid;
+    }
+    *least_tiles = (int)hi;
+  }
+  return splits;
 }
 // Bytes of p.part for that launch.
 uint64_t fwd_part_bytes(int B, int Hq, int Nq, int dp, int splits) {

@@ -141,3 +141,29 @@ def test_split_keeps_nan_inf_and_capture(monkeypatch):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(o, eager)
+
+
+@pytest.mark.parametrize("B,chunk,prefix,D", [(2, 512, 0, 128), (2, 512, 256, 128), (1, 512, 0, 64), (4, 128, 256, 128),
+                                              (4, 16, 0, 128), (1, 1024, 0, 128), (2, 300, 100, 64)])
+def test_wide_table_leaves_short_prompts_whole(B, chunk, prefix, D, monkeypatch):
+    """A block table sized for a context limit, over sequences too short to be
+    split: the same bits as under a table that just holds them."""
+    print(f"case wide table {B} x {prefix}+{chunk} D={D}", flush=True)
+    H, Hkv, bs, n = 32, 8, 16, prefix + chunk
+    g = torch.Generator(device="cuda").manual_seed(n)
+    blocks = -(-n // bs)
+    kc, vc = (torch.randn(B * blocks, bs, Hkv, D, device="cuda", generator=g).to(torch.bfloat16) for _ in range(2))
+    tight = torch.randperm(B * blocks, device="cuda", generator=g).to(torch.int32).view(B, blocks)
+    wide = torch.full((B, 1024), -1, dtype=torch.int32, device="cuda")
+    wide[:, :blocks] = tight
+    q = torch.randn(B * chunk, H, D, device="cuda", generator=g).to(torch.bfloat16)
+    cu = torch.arange(0, (B + 1) * chunk, chunk, dtype=torch.int32, device="cuda")
+    sl = torch.full((B,), n, dtype=torch.int32, device="cuda")
+    seen = []
+    real = _lib.prefill_paged_split
+    monkeypatch.setattr(_lib, "prefill_paged_split", lambda *a: (seen.append(1), real(*a)))
+    got = paged_prefill(q, kc, vc, wide, cu, sl, max_seqlen_q=chunk, return_lse=True)
+    assert seen, "the launch under the wide table has splits to give"
+    _unsplit(monkeypatch)
+    want = paged_prefill(q, kc, vc, tight, cu, sl, max_seqlen_q=chunk, return_lse=True)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
