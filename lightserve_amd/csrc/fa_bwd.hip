@@ -27,6 +27,7 @@
 // Every dP accumulation starts from -delta (the MFMA's C input), so that
 // dS = P (dP - delta) costs one multiply per score.
 #include "fa_common.hpp"
+#include <algorithm>
 
 namespace lsfa {
 
@@ -63,7 +64,7 @@ __global__ __launch_bounds__(256, 2) void fa_bwd_dq_kernel(const BwdParams p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (SGPR)
   const int l32 = lane & 31, hh = lane >> 5;
   int b, h, qt;
-  if (VARLEN && p.B <= 64) {
+  if (VARLEN && p.ranked_tokens >= 0 && p.cu_q[p.B] - p.cu_q[0] <= p.ranked_tokens) {
     // Sequences differ in length: (sequence, query tile) items longest first,
     // workgroup L taking rank L / H and head slot L % H (ranked_head).
     const int rank = blockIdx.x / p.H;
@@ -411,7 +412,7 @@ __global__ __launch_bounds__(256, 1) void fa_bwd_dkdv_kernel(const BwdParams p) 
   static_assert(!((GQA || VARLEN) && DS), "the stored-dS path has no GQA or varlen");
   const int G = GQA ? p.G : 1, Hkv = p.H / G;
   int bh, kt, b, hk;
-  if (VARLEN && p.B <= 64) {
+  if (VARLEN && p.ranked_tokens >= 0 && p.cu_k[p.B] - p.cu_k[0] <= p.ranked_tokens) {
     // Longest first, as in fa_bwd_dq_kernel: key tile kt of a sequence takes
     // the query tiles from max(0, 128 kt - off) / 64 on, so more than x of
     // them iff 128 kt < 64 (tiles - x) + off.
@@ -1147,6 +1148,29 @@ static hipError_t launch_bwd_ds(BwdParams p, int phases, hipStream_t s) {
   return e;
 }
 
+// BwdParams::ranked_tokens of a varlen launch of B sequences of up to num_tiles
+// tiles (`longest` tokens) on `heads` heads (heads_kv K/V heads).
+// Longest first keeps the XCDs and the tail level where lengths differ, but it
+// streams the rows of all sequences at once, so that an L2 holds none of them for
+// long once many K/V heads take part, and each workgroup pays 1 to 2 us for its
+// rank. Measured on 688 packed batches of 2..64 sequences (head dims 64 and 128,
+// 16/16, 32/8 and 16/2 heads, shortest 16 tokens, half, 0.85 or all of the longest),
+// map_tile's order (batch, then head) against longest first, us:
+//   one or two tiles, or no more items than CUs: 82 -> 108 (64 x 250, 16/16), 18 -> 20;
+//   few sequences: 87 -> 72 (3 x 1000, 16/16), 826 -> 387 (8 of 16..2000, 32/8), 1552 -> 1061
+//   (8 of 16..4000, 16/16), but 157 -> 165 (8 x 1000, 16/16);
+//   many: 1769 -> 1501 (33 of 16..2000, 32/8), 2187 -> 2026 (33 x 2000, 16/2), but 1159 -> 1265
+//   (33 x 1000, 32/8), 2099 -> 2624 (33 x 2000, 16/16), 1.2 times (64 of 1000..2000, 16/16).
+// So the share of the tokens that may be there falls with the K/V heads in all
+// sequences: 92% at 128 of them, 84% at 264, 67% at 528.
+static int ranked_tokens_for(int B, int heads, int heads_kv, int num_tiles, int longest) {
+  const long long grid = (long long)B * num_tiles * heads, streams = (long long)B * heads_kv;
+  if (B > 64 || num_tiles < 3 || grid <= 256) return -1;
+  if (grid <= 1024 && num_tiles >= 8 && streams < 64) return 0x7fffffff;
+  const long long percent = std::min(97LL, 100 - streams / 16) - (num_tiles < 5 ? 15 : 0);
+  return (int)std::min(0x7fffffffLL, (long long)B * longest * std::max(40LL, percent) / 100);
+}
+
 // phases: bit 0 dQ, bit 1 dK/dV. With p.ds set, the stored-dS path above;
 // otherwise the recompute path: fa_bwd_dq_kernel (whose prologue writes the
 // ld blocks), then fa_bwd_dkdv_kernel.
@@ -1166,6 +1190,7 @@ static hipError_t launch_bwd(BwdParams p, int phases, hipStream_t s) {
   p.num_tiles = (p.Nq + 127) / 128;
   p.heads_per_group = heads_per_group_for((long long)p.Nk * DP * 2 * 2);  // K and V rows of a head
   const bool varlen = p.cu_q != nullptr;  // grids over the longest sequence; shorter ones exit early
+  p.ranked_tokens = varlen ? ranked_tokens_for(p.B, p.H, p.H / p.G, p.num_tiles, p.Nq) : -1;
   if ((phases & 1) && p.num_tiles > 0) {
     if (varlen)
       hipLaunchKernelGGL((fa_bwd_dq_kernel<T, DP, CAUSAL, true>), dim3(p.num_tiles * BH), dim3(256), 0, s, p);
@@ -1176,6 +1201,7 @@ static hipError_t launch_bwd(BwdParams p, int phases, hipStream_t s) {
   p.num_tiles = (p.Nk + 127) / 128;
   // one workgroup per (b, KV head, key tile); it streams the Q and dO rows of the group's G heads
   p.heads_per_group = heads_per_group_for((long long)p.Nq * DP * 2 * 2 * p.G);
+  p.ranked_tokens = varlen ? ranked_tokens_for(p.B, p.H / p.G, p.H / p.G, p.num_tiles, p.Nk) : -1;
   if ((phases & 2) && p.num_tiles > 0) {
     const dim3 grid(p.num_tiles * (BH / p.G));
     if (varlen && p.G > 1)

@@ -211,6 +211,7 @@ struct BwdParams {
   const int32_t* cu_k;
   int num_tiles;     // tiles per (b, h) along the kernel's stationary axis
   int heads_per_group;  // map_tile grouping
+  int ranked_tokens;    // varlen: at most this many tokens in all sequences go longest first (-1: never)
   float scale;       // sm_scale
   float scale_log2;  // sm_scale * log2(e)
 };

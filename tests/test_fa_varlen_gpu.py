@@ -282,23 +282,11 @@ def test_varlen_backward_validation(gpu):
     assert o.shape == qf.shape
 
 
-@pytest.mark.parametrize("heads", [(8, 8), (6, 2), (16, 8)])
-@pytest.mark.parametrize("B", [1, 2, 5, 64, 65])
-@pytest.mark.parametrize("causal", [True, False])
-def test_varlen_order_does_not_change_results(B, heads, causal):
-    """Batches of up to 64 sequences run their tiles longest first, longer ones
-    in launch order: forward and gradients of a batch (empty sequences, empty
-    key or query sides, more keys than queries and fewer) equal the same
-    sequences run one at a time, bit for bit."""
-    import random
+def _same_as_one_by_one(lq, lk, heads, causal):
+    """Forward and gradients of a packed batch equal the same sequences run one
+    at a time, bit for bit."""
     from lightserve_amd.kernels.flash_attention_varlen import flash_attention_varlen_backward
-    print(f"case varlen order B={B} heads={heads} causal={causal}", flush=True)
-    rng = random.Random(B)
-    lq = [rng.choice([0, 1, 63, 64, 129, 200, 300]) for _ in range(B)]
-    lk = [rng.choice([0, 1, 64, 65, 128, 257, n, n]) for n in lq]
-    if B == 1:
-        lq, lk = [300], [257]
-    g = torch.Generator(device="cuda").manual_seed(B)
+    g = torch.Generator(device="cuda").manual_seed(len(lq))
     Hq, Hkv = heads
     q, do = (torch.randn(sum(lq), Hq, 64, device="cuda", generator=g).to(torch.bfloat16) for _ in range(2))
     k, v = (torch.randn(sum(lk), Hkv, 64, device="cuda", generator=g).to(torch.bfloat16) for _ in range(2))
@@ -319,3 +307,38 @@ def test_varlen_order_does_not_change_results(B, heads, causal):
     for i, t in enumerate(got):
         want = torch.cat([p[i] for p in parts])
         assert torch.equal(t, want), i
+
+
+@pytest.mark.parametrize("heads", [(8, 8), (6, 2), (16, 8)])
+@pytest.mark.parametrize("B", [1, 2, 5, 64, 65])
+@pytest.mark.parametrize("causal", [True, False])
+def test_varlen_order_does_not_change_results(B, heads, causal):
+    """Batches of up to 64 sequences run their tiles longest first, longer ones
+    in launch order: forward and gradients of a batch (empty sequences, empty
+    key or query sides, more keys than queries and fewer) equal the same
+    sequences run one at a time, bit for bit."""
+    import random
+    print(f"case varlen order B={B} heads={heads} causal={causal}", flush=True)
+    rng = random.Random(B)
+    lq = [rng.choice([0, 1, 63, 64, 129, 200, 300]) for _ in range(B)]
+    lk = [rng.choice([0, 1, 64, 65, 128, 257, n, n]) for n in lq]
+    if B == 1:
+        lq, lk = [300], [257]
+    _same_as_one_by_one(lq, lk, heads, causal)
+
+
+@pytest.mark.parametrize("lens,heads", [
+    ([1000] * 3, (16, 16)),                       # few sequences: longest first also at equal length
+    ([1500, 16, 700], (16, 8)), ([16, 2000], (16, 2)),
+    ([900, 20, 450, 870, 0, 130, 620, 900], (16, 16)),
+    ([400] * 33, (8, 8)), ([390, 400] * 16, (6, 2)),  # near equal length: in launch order
+    ([1000, 30, 500, 77] * 8, (16, 16)), ([400, 16, 90, 200] * 16, (6, 2)),
+    ([250, 100] * 32, (8, 8))])                   # two tiles
+@pytest.mark.parametrize("causal", [True, False])
+def test_varlen_backward_orders(lens, heads, causal, monkeypatch):
+    """Batches on either side of the rule that chooses the backward's order
+    (the forward whole: alone, a long sequence's keys would be split)."""
+    import importlib
+    monkeypatch.setattr(importlib.import_module("lightserve_amd.kernels.flash_attention"), "SPLIT_MAX_TILES", 0)
+    print(f"case varlen backward order {lens[:4]} of {len(lens)} heads={heads} causal={causal}", flush=True)
+    _same_as_one_by_one(lens, lens, heads, causal)
