@@ -132,12 +132,20 @@ BwdWorkspace bwd_workspace(int dtype, int flags, int batch, int heads, int nq, i
   return w;
 }
 
-// Decode split: enough workgroups (batch x kv heads x splits) to fill the
-// GPU, splits of a multiple of 64 tokens whose block-table slice fits the
-// kernel's LDS table. Partial outputs go to the workspace when split.
+// How a decode launch is split (decode_split_size in fa_decode.hip has the rule
+// that these are the parameters of). Partial outputs go to the workspace when
+// split.
 struct DecodeSplit {
-  int num_splits = 1, split_tokens = 64;
-  uint64_t o_off = 0, lse_off = 0, bytes = 0;
+  int num_splits = 1, split_tokens = 64, grid_units = 0, unit_shift = 6;
+  bool compact = false;
+  double lo = 64, hi = 64, scale = 0, fill = 0, share = 0;
+  int turn_mask = 0, turn_min = 0;
+  uint64_t o_off = 0, lse_off = 0, n_off = 0, bytes = 0;
+  // Tokens per split (before rounding up) for W = KV heads x tokens.
+  double size(double work) const {
+    const double fit = std::min(hi, std::max(lo, std::min(scale * std::sqrt(work), work * fill)));
+    return std::min<double>(split_tokens, std::max(fit, work * share));
+  }
 };
 
 int log2_exact(int x) {
@@ -146,37 +154,94 @@ int log2_exact(int x) {
   return (1 << s) == x ? s : -1;
 }
 
+// Measured at 1 to 55 sequences of 300 to 14502 tokens, all as long or from a tenth
+// of the longest, 32, 8, 4 and 2 KV heads of groups 1, 2, 4, 7 and 8 at head dims 64
+// and 128, over splits of 64 to 8192 tokens.
+// Lane-group kernel: up to 256 workgroups, splits as small as give each CU one (us,
+// at 128, 256 and 512 tokens: 1 x 1000 x 8 KV heads of group 4 and head dim 128 12.4,
+// 14.8, 19.8; 4 of 1450..14502 x 2 of group 8 37, 32, 30.5, at 384 27); beyond, about
+// the square root of the work, as the combine kernel reads a sequence's splits one
+// after another (16 of 1450..14502 x 8 124, 100, 94, at 4096 121), to 1024 tokens (512
+// for group 8, which holds the CU's registers: 55 of 400..4000 x 2 63, 49, 43, at 1024
+// 68); beyond 4096 workgroups sizes grow with the work. That is 1 to 3% from
+// the best size on average, 17% at worst. Sizes go by what a workgroup loads at once
+// (128 tokens at head dim 64, where those of 192 take as long as those of 256; 64 at
+// 128, from group 4 on). A launch of short limits has no split: that is worth the
+// combine kernel's 2 us from 128 tokens on (group 8, head dim 128: 1 x 300 18.1 -> 13.4)
+// to 512 (group 1, 64: 1 x 500 8.2 -> 9.2), later where many (sequence, KV head) pairs
+// share the GPU (16 of 100..1000 x 32 21.7 whole, 25.7).
+// MFMA kernel: two workgroups on a CU at most (one at head dim 128), which are
+// filled with fewer of them: 4 of 1450..14502 x 4 KV heads of group 7 at 128 34.8 at 384
+// tokens, 26.1 at 768. Above 128 pairs only long sequences are split (55 of
+// 100..1000 x 4 21.7 whole, 31 at 512; at head dim 64 16.4 and 18, but of 400..4000 48
+// and 37).
 DecodeSplit decode_split(const lsfa_decode_args* a) {
   DecodeSplit d;
-  const int maxs = std::max(a->max_seq_len, 0);
-  const long long units = std::max(1LL, (long long)a->batch * a->heads_kv);
-  // Lane-group kernel: up to ~16 workgroups per CU, splits of at least 256
-  // tokens (128 where 256 would leave CUs idle; none up to 512 tokens where the
-  // sequences alone fill half the GPU: 16 x 500 x 8 KV heads 11.1 us unsplit, 14.0
-  // split in two). Each sequence gets splits by its own length (kernel). MFMA
-  // kernel (one workgroup per CU): up to one workgroup per CU, splits of at least
-  // 512 tokens: 16 sequences of 1000..3000 with 4 KV heads of group 7, 64
-  // workgroups unsplit, 39.0 -> 23.5 us (1024 and 256 the same).
-  const int g = a->heads_kv > 0 ? a->heads_q / a->heads_kv : 1;
-  const bool mfma = lsfa::decode_uses_mfma(g, std::max(0, log2_exact(std::max(1, a->block_size))));
-  const long long target = mfma ? 256 : 4096;
-  const long long min_split = mfma ? 512 : (units * ((maxs + 255) / 256) < 256 ? 128 : (units >= 128 && maxs <= 512 ? 512 : 256));
-  long long ns = 1;
-  if (units < target && maxs > min_split)
-    ns = std::min<long long>((target + units - 1) / units, (maxs + min_split - 1) / min_split);
-  long long st = (maxs + ns - 1) / ns;
-  st = std::max(64LL, (st + 63) / 64 * 64);
+  const long long maxs = std::max(a->max_seq_len, 0), batch = std::max(a->batch, 0), hkv = std::max(a->heads_kv, 1);
+  const long long units = std::max(1LL, batch * hkv);
   const int shift = std::max(0, log2_exact(std::max(1, a->block_size)));
-  const long long max_st = ((long long)(lsfa::kDecodeMaxTableSlots - 1) << shift) / 64 * 64;
-  st = std::min(st, std::max(64LL, max_st));
-  ns = std::max(1LL, (maxs + st - 1) / st);
-  d.num_splits = (int)ns;
-  d.split_tokens = (int)st;
-  if (ns > 1) {
-    const uint64_t rows = (uint64_t)a->batch * a->heads_q * ns;
+  const int g = a->heads_kv > 0 ? a->heads_q / a->heads_kv : 1;
+  const bool wide = a->head_dim > 64, mfma = lsfa::decode_uses_mfma(g, shift), many = units >= 64;
+  d.unit_shift = wide && g >= 4 && !mfma ? 6 : 7;
+  const int unit = 1 << d.unit_shift;
+  int whole;  // limit up to which nothing is split
+  // a split's block-table slice fits the kernel's LDS table
+  d.split_tokens = (int)std::min<long long>(((long long)(lsfa::kDecodeMaxTableSlots - 1) << shift) / unit * unit, 1 << 24);
+  d.compact = batch <= lsfa::kDecodeScanMax;
+  d.lo = unit;
+  d.hi = 1024;
+  if (mfma && units > 128) {
+    whole = wide ? 4096 : 1024;
+    d.lo = d.hi = whole;
+  } else if (mfma) {
+    whole = many ? (wide ? 1024 : 512) : 384;
+    d.scale = 1.8;
+    d.fill = 1.0 / 192;
+  } else if (units >= 4096) {
+    whole = d.split_tokens;
+    d.lo = d.hi = d.split_tokens;
+  } else if (!d.compact) {
+    const long long n = std::max(1LL, std::min((4096 + units - 1) / units, (maxs + 511) / 512));
+    whole = 512;
+    d.lo = d.hi = (double)std::max(512LL, (maxs + n - 1) / n);
+  } else {
+    if (wide) whole = g <= 2 ? (many ? 512 : 384) : (g == 4 ? (many ? 512 : 256) : (many ? 256 : 128));
+    else whole = g <= 4 || many ? 512 : 256;
+    if (units >= 512 || (units >= 256 && g == 1)) whole = 1024;
+    if (g == 8) d.hi = 512;
+    d.scale = 1.4;
+    d.fill = 1.0 / 256;
+    d.share = 1.0 / 4096;
+  }
+  whole = std::min(whole, d.split_tokens);
+  if (maxs > whole) {
+    // The most splits that a sequence, and all together, can have: sizes grow slower
+    // than the work, so both are largest where every sequence has maxs tokens.
+    // (0.999: the device computes in 32 bits; it counts at most 2^20 tokens a sequence.)
+    const double most = (double)std::min(maxs, 1LL << 20) * (double)hkv;
+    d.num_splits = (int)std::min(2147483647.0, std::ceil((double)maxs / (0.999 * d.size(most))));
+    if (d.compact) {
+      const double all = std::ceil((double)(batch * maxs) / (0.999 * d.size(most * (double)std::max(1LL, batch)))) + (double)batch;
+      d.grid_units = (int)std::min(std::min(all, (double)batch * d.num_splits), 2147483647.0);
+    }
+  }
+  if (d.num_splits == 1) d.compact = false;
+  // Which head goes to which XCD (decode_item): K/V bytes from which turning them pays.
+  // 16 KV heads of head dim 64, 100 x 4000 tokens (1.6 GB) 0.87 times, 32 x 1000 (131 MB)
+  // 1.06; 8 of them, 100 x 4000 0.90, 16 of 1450..14502 (234 MB) 1.035; 24 0.83 to
+  // 0.96 at any size.
+  if (hkv % 8 == 0 && (hkv > 8 || !wide)) {
+    const double bytes = hkv > 16 ? 0 : (hkv > 8 ? 200e6 : 300e6), token = (double)hkv * a->head_dim * 4;
+    d.turn_min = (int)std::min(bytes / (16 * token), 1e9);
+    d.turn_mask = d.compact || (double)(batch * maxs) * token >= bytes ? 7 : 0;
+    if (!d.compact) d.turn_min = 0;
+  }
+  if (d.num_splits > 1) {
+    const uint64_t rows = (uint64_t)a->batch * a->heads_q * d.num_splits;
     d.o_off = 0;
     d.lse_off = align256(rows * padded_decode_dim(a->head_dim) * 4);
-    d.bytes = d.lse_off + align256(rows * 4);
+    d.n_off = d.lse_off + align256(rows * 4);
+    d.bytes = d.n_off + align256((uint64_t)a->batch * 4);
   }
   return d;
 }
@@ -535,6 +600,7 @@ int lsfa_decode(const lsfa_decode_args* a, void* stream) {
     char* ws = static_cast<char*>(a->workspace);
     p.o_part = reinterpret_cast<float*>(ws + d.o_off);
     p.lse_part = reinterpret_cast<float*>(ws + d.lse_off);
+    p.splits_of = reinterpret_cast<int*>(ws + d.n_off);
   }
   p.sqb = a->q_stride[0]; p.sqh = a->q_stride[1];
   p.skb = a->k_stride[0]; p.sks = a->k_stride[1]; p.skh = a->k_stride[2];
@@ -549,6 +615,16 @@ int lsfa_decode(const lsfa_decode_args* a, void* stream) {
   p.max_seq_len = a->max_seq_len;
   p.num_splits = d.num_splits;
   p.split_tokens = d.split_tokens;
+  p.compact = d.compact;
+  p.grid_units = d.grid_units;
+  p.split_lo = (float)d.lo;
+  p.split_hi = (float)d.hi;
+  p.split_scale = (float)d.scale;
+  p.split_share = (float)d.share;
+  p.split_fill = (float)d.fill;
+  p.unit_shift = d.unit_shift;
+  p.turn_mask = d.turn_mask;
+  p.turn_min = d.turn_min;
   p.scale_log2 = a->sm_scale * 1.4426950408889634f;
   hipError_t e = lsfa::decode_gqa(p, a->dtype == LSFA_DTYPE_BF16, padded_decode_dim(a->head_dim),
                                   reinterpret_cast<hipStream_t>(stream));

@@ -217,6 +217,7 @@ struct BwdParams {
 };
 
 // Paged-KV decode (one query token per sequence); strides in elements.
+constexpr int kDecodeScanMax = 256;        // sequences of a launch whose workgroups find their split by a prefix sum
 constexpr int kDecodeMaxTableSlots = 512;  // block-table entries one split may span
 
 // Skinny GEMM y[M, N] = x[M, K] @ W[K, N] (M <= 8; element strides; W rows
@@ -275,7 +276,13 @@ struct DecodeParams {
   int max_blocks;         // block-table entries per sequence
   int num_blocks;         // blocks in the cache; other ids read as zero
   int max_seq_len;        // sequences are clamped to min(this, max_blocks * block_size)
-  int num_splits, split_tokens;  // split_tokens is a multiple of 16
+  int num_splits, split_tokens;  // most splits of a sequence, most tokens of a split (a multiple of 64)
+  // Split sizes (decode_split_size in fa_decode.hip).
+  int compact, grid_units;       // whether the grid holds grid_units splits in a row, or num_splits for each sequence
+  int unit_shift;                // log2 of the tokens that split sizes are multiples of
+  float split_lo, split_hi, split_scale, split_fill, split_share;
+  int turn_mask, turn_min;       // KV heads are turned (xor) from split to split, from turn_min x 16 tokens on
+  int* splits_of;                // [B] splits of each sequence (written by the split kernel)
   float scale_log2;       // sm_scale * log2(e)
 };
 

@@ -79,47 +79,141 @@ __device__ __forceinline__ float dot8(const X8& a, const X8& b) {
   return dot2(__builtin_shufflevector(a, a, 6, 7), __builtin_shufflevector(b, b, 6, 7), d);
 }
 
-// Tokens per split of a sequence of seq tokens. The host sizes the grid and the
-// workspace for the longest sequence it was told of (num_splits splits of at
-// most split_tokens); each sequence shares those splits out by its own length,
-// in splits of at least 512 tokens, or 256 or 128 where longer ones would leave
-// CUs without a workgroup. 64 sequences of 100..1000 tokens under a limit of
-// 16384 took splits of 2048, one workgroup for each longest sequence: 165 -> 42 us
-// (with the order below); 4 of 2000..6000 44.5 -> 27.9, 1 x 1000 x 32 heads 18.9 ->
-// 10.8.
-__device__ __forceinline__ int decode_split_tokens(const DecodeParams& p, int seq) {
-  if (p.num_splits == 1) return p.split_tokens;
-  const int64_t units = (int64_t)p.B * p.Hkv;
-  const int least = units * ((seq + 511) >> 9) >= 256 ? 512 : (units * ((seq + 255) >> 8) >= 256 ? 256 : 128);
-  const int even = __builtin_amdgcn_readfirstlane((seq + p.num_splits - 1) / p.num_splits);
-  return min((max(even, least) + 63) & ~63, p.split_tokens);
+// Inclusive sum over the wave's lanes, on DPP (row shifts, then row broadcasts).
+__device__ __forceinline__ int wave_prefix_sum(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15, rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31, rows 2 and 3
+  return v;
+}
+__device__ __forceinline__ int decode_seq(const DecodeParams& p, int b) {
+  return min(max(p.seq_lens[b], 0), min(p.max_seq_len, p.max_blocks << p.block_shift));
 }
 
-// Workgroups are numbered [split][sequence][KV head]: the heads of a token range
-// run side by side, so that the 256-byte rows they read of a token (adjacent in
-// the cache) are requested together (with the splits innermost, 32 sequences of
-// 1024..8192 tokens read 4.3 instead of 4.7 TB/s, 64 of 3000..4000 with 32 KV heads
-// 6.0 instead of 6.5), and the splits that no sequence has come last. Splits past
-// the grid's 65535 go on along x.
-__device__ __forceinline__ void decode_item(const DecodeParams& p, int& hk, int& b, int& split) {
+// How sequences are split. The host (decode_split) gives a split's size as a
+// function of the work there is, W = KV heads x tokens of all sequences, which only
+// the device knows: split_scale sqrt(W) and W * split_fill, whichever is less, within
+// split_lo and split_hi, but no less than W * split_share. So few or short sequences
+// spread over the GPU in small splits (each adds to what the combine kernel reads
+// one after another), many or long ones keep large ones, and all splits are about
+// equally long whatever the lengths. A sequence shares its tokens out evenly.
+// Launches of more than kDecodeScanMax sequences (not compact) have a fixed size.
+// Sizes are in units of 1 << unit_shift tokens here; tokens16 is the tokens of all
+// sequences in 16s.
+__device__ __forceinline__ int decode_split_size(const DecodeParams& p, int tokens16) {
+  float size = p.split_lo;
+  if (p.compact) {
+    const float work = 16.f * p.Hkv * (float)tokens16;
+    const float fit = fminf(p.split_hi, fmaxf(p.split_lo, fminf(p.split_scale * __builtin_amdgcn_sqrtf(work), work * p.split_fill)));
+    size = fmaxf(fit, work * p.split_share);
+    // one sequence, all splits alike: no second workgroup on some CUs only
+    if (p.B == 1 && work > 256.f * size && work <= 512.f * size) size = work * (1.f / 256);
+  }
+  return ((int)ceilf(fminf(size, (float)p.split_tokens)) + (1 << p.unit_shift) - 1) >> p.unit_shift;
+}
+// ceil(a / b) for quotients below 2^21.
+__device__ __forceinline__ int div_up(int a, int b) {
+  int q = (int)((float)a * __builtin_amdgcn_rcpf((float)b));
+  q += q * b < a;
+  q += q * b < a;
+  q -= (q - 1) * b >= a;
+  return q;
+}
+// Units per split of a sequence, at most split_tokens' worth, and how many splits that makes.
+__device__ __forceinline__ int decode_split_units(const DecodeParams& p, int seq, int size, int& have) {
+  const int u = (int)(((unsigned)seq + (1u << p.unit_shift) - 1) >> p.unit_shift);
+  const int n = max(1, min(div_up(u, size), p.num_splits));
+  const int st = max(1, div_up(u, n));
+  have = max(1, div_up(u, st));
+  return st;
+}
+
+// The KV head, sequence and split of a workgroup, and the tokens per split of
+// the sequence; b = -1 past the last. Workgroups are numbered [sequence][split][KV
+// head] over the splits that there are (a prefix sum over the sequences, lane l
+// holding sequences l per .. l per + per - 1): numbered over the grid of all
+// possible ones instead, those that a long sequence alone has came at a stride of
+// the batch and gathered on a few CUs (16 sequences of 1450..14502 tokens, 8 KV
+// heads of head dim 64: 78.7 us, this way 59.5). The heads of a token range run side
+// by side, so that the rows that they read of a token (adjacent in the cache) are
+// requested together; 8 heads and multiples of 8 are turned by one XCD from range to
+// range, so that each XCD reads all of a row's channels (55 sequences of 1450..14502, 32
+// heads of head dim 64, splits of 1024: 725 -> 619 us), where that pays (decode_split).
+__device__ __forceinline__ void decode_item(const DecodeParams& p, int lane, int& hk, int& b, int& split, int& seq, int& tokens) {
   hk = blockIdx.x;
-  b = blockIdx.y;
+  int unit = blockIdx.y;  // (on from the grid's 65535 along x)
   split = blockIdx.z;
   if (hk >= p.Hkv) {
     // (integer division runs on the VALU: back to a scalar, or every address
     // that follows is computed per lane, which cost the loop a quarter)
     const int round = __builtin_amdgcn_readfirstlane(hk / p.Hkv);
-    split += round * gridDim.z;
+    if (p.compact) unit += round * gridDim.y;
+    else split += round * gridDim.z;
     hk -= round * p.Hkv;
   }
+  int st, have, sum = 0;
+  if (!p.compact) {
+    b = unit;
+    seq = decode_seq(p, b);
+    if (p.num_splits == 1) {
+      tokens = max(seq, 64);
+      have = 1;
+    } else {
+      st = decode_split_units(p, seq, decode_split_size(p, 0), have);
+      tokens = __builtin_amdgcn_readfirstlane(st) << p.unit_shift;
+    }
+    if (split >= have) b = -1;
+  } else if (p.B <= 64) {
+    const int mine = lane < p.B ? decode_seq(p, lane) : 0;
+    sum = __builtin_amdgcn_readlane(wave_prefix_sum((min(mine, 1 << 20) + 15) >> 4), 63);
+    st = decode_split_units(p, mine, decode_split_size(p, sum), have);
+    const int upto = wave_prefix_sum(lane < p.B ? have : 0);
+    const unsigned long long hit = __ballot(unit < upto);
+    b = hit == 0 ? -1 : (int)__builtin_ctzll(hit);
+    const int src = max(b, 0);
+    split = unit - __builtin_amdgcn_readlane(upto - have, src);
+    seq = __builtin_amdgcn_readlane(mine, src);
+    tokens = __builtin_amdgcn_readlane(st, src) << p.unit_shift;
+    have = __builtin_amdgcn_readlane(have, src);
+  } else {
+    int n = 0;
+    const int per = (p.B + 63) >> 6;
+    for (int j = lane * per; j < min(p.B, (lane + 1) * per); ++j) sum += (min(decode_seq(p, j), 1 << 20) + 15) >> 4;
+    sum = __builtin_amdgcn_readlane(wave_prefix_sum(sum), 63);
+    const int size = __builtin_amdgcn_readfirstlane(decode_split_size(p, sum));
+    for (int j = lane * per; j < min(p.B, (lane + 1) * per); ++j) {
+      decode_split_units(p, decode_seq(p, j), size, have);
+      n += have;
+    }
+    const int upto = wave_prefix_sum(n);
+    const unsigned long long hit = __ballot(unit < upto);
+    b = -1;
+    if (hit == 0) return;
+    const int src = __builtin_amdgcn_readfirstlane((int)__builtin_ctzll(hit));
+    split = unit - __builtin_amdgcn_readlane(upto - n, src);
+    for (int j = src * per; j < min(p.B, (src + 1) * per) && b < 0; ++j) {
+      seq = decode_seq(p, j);
+      st = decode_split_units(p, seq, size, have);
+      tokens = __builtin_amdgcn_readfirstlane(st) << p.unit_shift;
+      have = __builtin_amdgcn_readfirstlane(have);
+      if (split < have) b = j;
+      else split -= have;
+    }
+  }
+  if (b >= 0 && p.num_splits > 1 && hk == 0 && split == 0 && threadIdx.x == 0) p.splits_of[b] = have;
+  if (sum >= p.turn_min) hk ^= unit & p.turn_mask;
 }
 static dim3 decode_grid(const DecodeParams& p) {
-  const int rounds = (p.num_splits + 65534) / 65535;
-  return dim3(p.Hkv * rounds, p.B, (p.num_splits + rounds - 1) / rounds);
+  const int n = p.compact ? p.grid_units : p.num_splits, rounds = (n + 65534) / 65535, per = (n + rounds - 1) / rounds;
+  return p.compact ? dim3(p.Hkv * rounds, per) : dim3(p.Hkv * rounds, p.B, per);
 }
 
+// (Waves per SIMD that the registers allow; group 2 was one register over four.)
 template <typename T, int DP, int G>
-__global__ __launch_bounds__(256) void fa_decode_split_kernel(const DecodeParams p) {
+__global__ __launch_bounds__(256, (G <= 2 ? 4 : (G == 4 ? 3 : 2))) void fa_decode_split_kernel(const DecodeParams p) {
   using X8 = typename VecT<T>::x8;
   constexpr int LPT = DP / 8;    // lanes per token row (16 B each)
   constexpr int TPW = 64 / LPT;  // tokens per wave per load instruction
@@ -127,16 +221,13 @@ __global__ __launch_bounds__(256) void fa_decode_split_kernel(const DecodeParams
   constexpr int TPI = NW * TPW;  // tokens per workgroup per load instruction
   constexpr int CH = 4;          // tokens per lane group between offset updates
 
-  int hk, b, split;
-  decode_item(p, hk, b, split);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int hk, b, split, seq, st;
+  decode_item(p, lane, hk, b, split, seq, st);
+  if (b < 0) return;  // uniform, before any barrier
   const int c = lane % LPT, tq = lane / LPT;
-  const int seq = min(max(p.seq_lens[b], 0), min(p.max_seq_len, p.max_blocks << p.block_shift));
-  const int st = decode_split_tokens(p, seq);
-  const int t0 = split * st;
-  if (split > 0 && t0 >= seq) return;  // uniform, before any barrier
-  const int t1 = min(seq, t0 + st);
+  const int t0 = split * st, t1 = min(seq, t0 + st);
 
   __shared__ int s_blk[kDecodeMaxTableSlots];
   __shared__ float st_m[NW][G], st_l[NW][G];
@@ -367,17 +458,14 @@ __global__ __launch_bounds__(256) void fa_decode_mfma_kernel(const DecodeParams 
   __shared__ float st_m[NW][32], st_l[NW][32], st_le[NW][32];
   LDS_AS char* smem = (LDS_AS char*)smem_raw;
 
-  int hk, b, split;
-  decode_item(p, hk, b, split);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int hk, b, split, seq, st;
+  decode_item(p, lane, hk, b, split, seq, st);
+  if (b < 0) return;  // uniform, before any barrier
   const int l32 = lane & 31, hh = lane >> 5;
   const int G = p.Hq / p.Hkv;
-  const int seq = min(max(p.seq_lens[b], 0), min(p.max_seq_len, p.max_blocks << p.block_shift));
-  const int st = decode_split_tokens(p, seq);
-  const int t0 = split * st;
-  if (split > 0 && t0 >= seq) return;  // uniform, before any barrier
-  const int t1 = min(seq, t0 + st);
+  const int t0 = split * st, t1 = min(seq, t0 + st);
   const int ntile = t1 > t0 ? (t1 - t0 + BT - 1) / BT : 0;
   const int D = p.D;
   const float sl2 = p.scale_log2;
@@ -586,10 +674,8 @@ __global__ __launch_bounds__(DP) void fa_decode_combine_kernel(const DecodeParam
   __shared__ float s_red[DP / 64];
   const int h = blockIdx.x, b = blockIdx.y, d = threadIdx.x;
   const int64_t row0 = ((int64_t)b * p.Hq + h) * p.num_splits;
-  const int seq = min(max(p.seq_lens[b], 0), min(p.max_seq_len, p.max_blocks << p.block_shift));
-  const int st = decode_split_tokens(p, seq);
-  if (seq <= st) return;  // one split, already in o
-  const int ns = (seq + st - 1) / st;
+  const int ns = min(p.splits_of[b], p.num_splits);
+  if (ns <= 1) return;  // already in o
   float M = -INFINITY, W = 0.f, O = 0.f;
   for (int c0 = 0; c0 < ns; c0 += kCombineBatch) {
     const int cn = min(kCombineBatch, ns - c0);
