@@ -74,10 +74,10 @@ MFMA_MAX_STRIDE = 1 << 25  # of W's rows: 32 of them in a 31-bit byte offset
 # A matrix by itself has to be large enough for the pass over it to outweigh the
 # launch and the split's reduction (a group saves launches too, and runs from 256 x
 # 256 on). Measured against hipBLASLt in us: up to 16 rows K of 1536 or 2.4 million
-# elements (1024 x 1024 6.4 against 5.8, 512 x 1024 8.2 against 5.6, 2048 x 512 6.7
-# against 7.3; up to 256 columns all the same); above 16 rows, where hipBLASLt has its own kernels for them, 9.4
-# million (4096 x 1024 13.6 against 10.1, 4096 x 2048 1.2..1.3 times its time, 3072 x
-# 3072 0.7 times). Up to 8 rows all go to the kernel.
+# elements (at 9 rows 768 x 768 6.5 against 5.3, 512 x 1024 6.2 against 4.2, 2048 x 512
+# 7.2 against 7.8; up to 256 columns all the same); above 16 rows, where hipBLASLt is
+# faster on them, 9.4 million (at 17 rows 5120 x 1024 14.6 against 11.2, 4096 x 2048 13.8
+# against 11.2, 3072 x 3072 12.1 against 17.8). Up to 8 rows all go to the kernel.
 MFMA_MIN_K, MFMA_MIN_ELEMS, MFMA_MIN_ELEMS_17 = 1536, 9 << 18, 9 << 20
 # Above MFMA_AUTO_ROWS rows, lsfa_gemm_group runs launches of this many tiles of
 # 64 x 128 whose K is at least GEMM_MIN_K or which group several matrices (a
