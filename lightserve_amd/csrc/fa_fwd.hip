@@ -1247,8 +1247,8 @@ static hipError_t launch_fwd_nw(FwdParams p, hipStream_t s) {
 // step's time for each tile of its longest workgroup (split_tiles rounds a
 // split's tiles up to an even number), and a split one the combine launch, the
 // partials' latency and the writing and reading of its workgroups' partials on
-// top. The times are those that choose best over measured launches of 3 to 256
-// items of 5 to 235 tiles at 1 to 16 splits, dense and paged, causal and not. A
+// top. The times are those that choose best over measured launches of 3 to 384
+// items of 5 to 251 tiles at 1 to 16 splits, dense and paged, causal and not. A
 // split has to win by half a microsecond to one.
 // Dense, us unsplit against split as chosen: head dim 128, 16 items of 32 tiles 34.2
 // -> 14.4 (8 splits), 64 of 16 20.8 -> 19.3 (4), 128 of 16 21.4 (24.8 in two: left

@@ -183,3 +183,20 @@ def test_decode_limit_does_not_change_results(gpu, heads, limit):
         s = (q[b].double() * k).sum(2).T / 8.0
         assert (got[b].double() - (s.softmax(1).T[:, :, None] * v).sum(0)).abs().max() < 2e-2, n
         assert (lse[b].double() - s.logsumexp(1)).abs().max() < 1e-3, n
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(4, 2, 64), (24, 24, 64), (14, 2, 128)])
+@pytest.mark.parametrize("batch", [1, 63, 64, 65, 129, 256, 257])
+def test_decode_split_numbering(gpu, batch, hq, hkv, d):
+    """Split launches on either side of the ways to number the splits: one
+    sequence per lane up to 64, several up to 256, fixed sizes above; 24 KV heads
+    turned from split to split; the MFMA kernel on both sides of 128 (sequence,
+    KV head) pairs. Long and short, empty and equal sequences in any order."""
+    g = torch.Generator().manual_seed(batch * 31 + hq)
+    lens = torch.randint(0, 200, (batch,), generator=g)
+    lens[::7] = 0
+    for at, n in ((0, 5003), (batch // 2, 2049), (batch - 1, 1537)):
+        lens[at] = n
+    print(f"case decode split numbering B={batch} hq={hq} hkv={hkv} d={d}", flush=True)
+    _check(*_make_case(lens.tolist(), hq, hkv, d, 16, torch.bfloat16, gpu, seed=batch), f"B={batch} hq={hq} hkv={hkv} d={d}",
+           max_seq_len=16384)
